@@ -35,6 +35,7 @@ FILE_FLAGS = {
     "ssd2_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "ssd3_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "mamba3_fused.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "ssd_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     # the decode products: accumulators in VGPRs keep a wave within 128
     # registers (four waves per SIMD)
     "lin.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "ssd2.h"
+#include "ssd_f32.h"
 
 namespace mamba {
 
@@ -322,6 +323,26 @@ int ssd2_generic_launch(const Ssd2Params& p, void* ws, hipStream_t stream, hipEv
     return MAMBA_OK;
 }
 
+// The same call for the f32-MFMA kernels (ssd_f32.hip): one rank, with
+// sc = gm = dt and the log-decay dt A.  False where they do not apply.
+static bool ssd2_f32_params(const Ssd2Params& p, SsdF32Params* out) {
+    SsdF32Params f{};
+    f.nb = p.nb; f.L = p.L; f.M = 1; f.H = p.H; f.P = p.P; f.G = p.G; f.N = p.N;
+    f.io_dtype = p.io_dtype;
+    f.v = p.x; f.v_sb = p.x_sb; f.v_sl = p.x_sl; f.v_sh = p.x_sh;
+    f.da = p.dt; f.da_sb = p.dt_sb; f.da_sl = p.dt_sl; f.da_sh = p.dt_sh;
+    f.A = p.A;
+    f.gm = p.dt; f.gm_sb = p.dt_sb; f.gm_sl = p.dt_sl; f.gm_sh = p.dt_sh;
+    f.sc = p.dt; f.sc_sb = p.dt_sb; f.sc_sl = p.dt_sl; f.sc_sh = p.dt_sh;
+    f.Bm = p.Bm; f.B_sb = p.B_sb; f.B_sl = p.B_sl; f.B_sg = p.B_sg;
+    f.Cm = p.Cm; f.C_sb = p.C_sb; f.C_sl = p.C_sl; f.C_sg = p.C_sg;
+    f.D = p.D; f.h0 = p.h0; f.init_hpr = p.init_hpr;
+    f.y = p.y; f.y_sb = p.y_sb; f.y_sl = p.y_sl; f.y_sh = p.y_sh;
+    f.hT = p.hT;
+    *out = f;
+    return ssd_f32_plan(out);
+}
+
 // Host-side validation of the public arguments (the reference asserts the same
 // conditions: mamba2.rs:562-566, serial_recalculated.rs:41-44, gqa.rs:37-41).
 int ssd2_make_params(const mamba_ssd2_args* a, Ssd2Params* out) {
@@ -358,7 +379,10 @@ extern "C" size_t mamba_ssd2_workspace_size(const mamba_ssd2_args* a) {
     if (ssd2_make_params(a, &p) != MAMBA_OK) return 0;
     size_t ws = ssd2_generic_workspace(p);
     const size_t fast = ssd2_mfma_workspace(p);
-    return ws > fast ? ws : fast;
+    if (ws < fast) ws = fast;
+    SsdF32Params f;
+    if (ssd2_f32_params(p, &f) && ws < ssd_f32_workspace(f)) ws = ssd_f32_workspace(f);
+    return ws;
 }
 
 extern "C" int mamba_ssd2_fast_path(const mamba_ssd2_args* a) {
@@ -391,6 +415,11 @@ static int ssd2_dispatch(const mamba_ssd2_args* a, void* ws, size_t ws_bytes, hi
         }
         return ssd2_mfma_launch(p, ws, stream, ev0, ev1);
     }
+    // f32 MFMA wherever shape and layout allow; the SIMT kernels take the rest,
+    // and a workspace sized for them alone
+    SsdF32Params f;
+    if (ssd2_f32_params(p, &f) && (ssd_f32_workspace(f) == 0 || (ws != nullptr && ws_bytes >= ssd_f32_workspace(f))))
+        return ssd_f32_launch(f, ws, stream, ev0, ev1);
     if (ws == nullptr || ws_bytes < ssd2_generic_workspace(p)) {
         set_error("mamba_ssd2_fwd: workspace missing or too small");
         return MAMBA_ERR_WORKSPACE;

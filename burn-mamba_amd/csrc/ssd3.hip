@@ -20,7 +20,10 @@
 // (ssd3_mfma.hip), which chunks on 128 fused positions whatever chunk_len
 // says: the chunked form is exact for any chunk length, so only rounding
 // differs.
+#include <algorithm>
+
 #include "common.h"
+#include "ssd_f32.h"
 
 namespace mamba {
 
@@ -359,6 +362,33 @@ static size_t ssd3_ws_bytes(const Ssd3Params& p) {
     return align_up((size_t)p.nb * p.nch * p.H * p.P * p.N * 4, 256) + align_up((size_t)p.nb * p.H * p.nch * 4, 256);
 }
 
+// The same call for the f32-MFMA kernels (ssd_f32.hip); false where they do
+// not apply.
+static bool ssd3_f32_params(const Ssd3Params& p, SsdF32Params* out) {
+    SsdF32Params f{};
+    f.nb = p.nb; f.L = p.L; f.M = p.M; f.H = p.H; f.P = p.P; f.G = p.G; f.N = p.N;
+    f.io_dtype = p.io_dtype;
+    f.v = p.v; f.v_sb = p.v_sb; f.v_sl = p.v_sl; f.v_sm = p.v_sm; f.v_sh = p.v_sh;
+    f.da = p.da; f.da_sb = p.da_sb; f.da_sl = p.da_sl; f.da_sh = p.da_sh;
+    f.gm = p.gm; f.gm_sb = p.gm_sb; f.gm_sl = p.gm_sl; f.gm_sh = p.gm_sh;
+    f.sc = p.sc; f.sc_sb = p.sc_sb; f.sc_sl = p.sc_sl; f.sc_sh = p.sc_sh;
+    f.Bm = p.Bm; f.B_sb = p.B_sb; f.B_sl = p.B_sl; f.B_sm = p.B_sm; f.B_sg = p.B_sg;
+    f.Cm = p.Cm; f.C_sb = p.C_sb; f.C_sl = p.C_sl; f.C_sm = p.C_sm; f.C_sg = p.C_sg;
+    f.h0 = p.h0;
+    f.y = p.y; f.y_sb = p.y_sb; f.y_sl = p.y_sl; f.y_sm = p.y_sm; f.y_sh = p.y_sh;
+    f.hT = p.hT;
+    *out = f;
+    return ssd_f32_plan(out);
+}
+
+// Scratch of the call: the generic kernels' and, where they apply, the f32-MFMA
+// kernels' (the bf16 MFMA path needs none).
+static size_t ssd3_ws_need(const Ssd3Params& p) {
+    SsdF32Params f;
+    const size_t need = ssd3_ws_bytes(p);
+    return ssd3_f32_params(p, &f) ? std::max(need, ssd_f32_workspace(f)) : need;
+}
+
 bool ssd3_mfma_supported(const mamba_ssd3_args* a);
 int ssd3_mfma_launch(const mamba_ssd3_args* a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
 
@@ -368,6 +398,12 @@ static int ssd3_dispatch(const mamba_ssd3_args* a, void* ws, size_t ws_bytes, hi
     int st = ssd3_make_params(a, &p, unit);
     if (st != MAMBA_OK) return st;
     if (allow_fast && ssd3_mfma_supported(a)) return ssd3_mfma_launch(a, stream, ev0, ev1);
+    // f32 MFMA wherever shape and layout allow; the SIMT kernels take the rest,
+    // and a workspace sized for them alone
+    SsdF32Params f;
+    if (allow_fast && ssd3_f32_params(p, &f) &&
+        (ssd_f32_workspace(f) == 0 || (ws != nullptr && ws_bytes >= ssd_f32_workspace(f))))
+        return ssd_f32_launch(f, ws, stream, ev0, ev1);
     const size_t need = ssd3_ws_bytes(p);
     if (ws == nullptr || ws_bytes < need) {
         set_error("mamba_ssd3_fwd: workspace of " + std::to_string(need) + " bytes required");
@@ -422,7 +458,7 @@ using namespace mamba;
 extern "C" size_t mamba_ssd3_workspace_size(const mamba_ssd3_args* a) {
     Ssd3Params p;
     if (ssd3_make_params(a, &p) != MAMBA_OK) return 0;
-    return ssd3_ws_bytes(p);  // the MFMA path needs none; this covers both paths
+    return ssd3_ws_need(p);
 }
 
 extern "C" int mamba_ssd3_fast_path(const mamba_ssd3_args* a) {
@@ -453,7 +489,7 @@ extern "C" size_t mamba_ssd3_double_workspace_size(const mamba_ssd3_double_args*
     const mamba_ssd3_args a = ssd3_from_double(d);
     Ssd3Params p;
     if (ssd3_make_params(&a, &p, true) != MAMBA_OK) return 0;
-    return ssd3_ws_bytes(p);
+    return ssd3_ws_need(p);
 }
 
 extern "C" int mamba_ssd3_double_fast_path(const mamba_ssd3_double_args* d) {
