@@ -1,11 +1,8 @@
-// f32 MFMA helpers shared by the SSD backward kernels (ssd2_bwd.hip,
-// ssd3_bwd.hip): v_mfma_f32_32x32x2_f32 (f32 operands and accumulation).  For
+// f32 MFMA helpers shared by the f32 SSD kernels (ssd_f32.hip,
+// ssd_f32_bwd.hip): v_mfma_f32_32x32x2_f32 (f32 operands and accumulation).  For
 // that instruction lane l supplies A[l % 32][k0 + l / 32] and
 // B[k0 + l / 32][l % 32], and accumulator r of lane l holds
-// D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].  LDS rows are padded to an odd
-// number of words, so that both the K-major reads (32 rows, one column) and
-// the row-major reads (32 consecutive words) of a half-wave fall in 32
-// distinct banks.
+// D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,9 +10,6 @@
 namespace mamba {
 
 typedef float bwd_f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr int kFP = 64, kFN = 128;                 // headdim, dstate of the MFMA paths
-constexpr int kSX = 65, kSB = 129, kSQ = 33;       // padded row lengths (words)
 
 __device__ __forceinline__ bwd_f32x16 bwd_mfma(float a, float b, bwd_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -52,15 +46,6 @@ __device__ __forceinline__ float bwd_half_sum16(const float (&v)[16], int i32) {
     const float z = (b1 ? y[1] : y[0]) + bwd_xor2(b1 ? y[0] : y[1]);
     return z + bwd_xor1(z);
 }
-// Sum over the 32 lanes of a wave half (every lane of the half gets it).
-__device__ __forceinline__ float bwd_half_sum(float v) {
-    v += __shfl_xor(v, 16, 64);
-    v += bwd_xor8(v);
-    v += bwd_xor4(v);
-    v += bwd_xor2(v);
-    return v + bwd_xor1(v);
-}
-
 __device__ __forceinline__ void bwd_put4(float* dst, float4 v) {
     dst[0] = v.x;
     dst[1] = v.y;

@@ -36,29 +36,10 @@
 // take k = 8 s + 4 (lane / 32) + 0..3 on both sides.
 #include <algorithm>
 
-#include "bwd_core.h"
 #include "ssd_f32.h"
+#include "ssd_f32_rows.h"
 
 namespace mamba {
-
-constexpr int kFR = 64;  // fused rows per chunk
-
-// four values of a row, as f32
-template <typename T>
-struct FRaw;
-template <>
-struct FRaw<float> {
-    float4 v;
-    __device__ __forceinline__ float4 get() const { return v; }
-};
-template <>
-struct FRaw<bf16_t> {
-    uint2 v;
-    __device__ __forceinline__ float4 get() const {
-        return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
-                           __uint_as_float(v.y & 0xffff0000u));
-    }
-};
 
 // log-decay and weights of one fused row (lane) of a chunk, in flight
 struct FTabRaw {
@@ -92,33 +73,6 @@ __device__ __forceinline__ FJob f_job(const SsdF32Params& p, int nseg, int PB) {
     return j;
 }
 
-// The rows of chunk c that thread tid stages: W values per row, NT threads.
-// Rows past the sequence end read as zero.
-template <typename T, int W, int NT>
-__device__ __forceinline__ void f_fetch(FRaw<T> (&raw)[kFR * W / 4 / NT], const T* base, int64_t sl, int64_t sm,
-                                        const SsdF32Params& p, int c, int tid) {
-    constexpr int RW = W / 4;
-#pragma unroll
-    for (int q = 0; q < kFR * W / 4 / NT; ++q) {
-        const int e = tid + NT * q, row = e / RW, col = (e % RW) * 4;
-        const int t = c * (kFR >> p.mshift) + (row >> p.mshift);
-        const int64_t at = (int64_t)min(t, p.L - 1) * sl + (int64_t)(row & (p.M - 1)) * sm + col;
-        raw[q].v = *reinterpret_cast<const decltype(raw[q].v)*>(base + at);
-    }
-}
-template <typename T, int W, int NT, int PITCH>
-__device__ __forceinline__ void f_commit(const FRaw<T> (&raw)[kFR * W / 4 / NT], float* dst, const SsdF32Params& p,
-                                         int c, int tid) {
-    constexpr int RW = W / 4;
-#pragma unroll
-    for (int q = 0; q < kFR * W / 4 / NT; ++q) {
-        const int e = tid + NT * q, row = e / RW, col = (e % RW) * 4;
-        const int t = c * (kFR >> p.mshift) + (row >> p.mshift);
-        const float4 z = {0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<float4*>(dst + row * PITCH + col) = t < p.L ? raw[q].get() : z;
-    }
-}
-
 // one wave: lane = fused row
 __device__ __forceinline__ FTabRaw f_tab_fetch(const SsdF32Params& p, const FJob& j, int c, int lane) {
     const int t = min(c * (kFR >> p.mshift) + (lane >> p.mshift), p.L - 1);
@@ -145,33 +99,6 @@ __device__ __forceinline__ void f_tab_commit(const SsdF32Params& p, const FTabRa
     }
 }
 
-// One wave's state tiles h[n][p] (rows n, columns p): tile t = slot + 4 q at
-// rows 32 (t / (PB / 32)), columns 32 (t % (PB / 32)).
-//   h <- dec h + sum_j B[j][n] (w_j v[j][p])
-template <int PB, int N, int QT>
-__device__ __forceinline__ void f_update(bwd_f32x16 (&acc)[QT], const float* sB, const float* sV, const FTables& T,
-                                         int slot, int i32, int hf) {
-    constexpr int PT = PB / 32, TILES = PT * (N / 32), BP = N + 4, VP = PB + 8;
-    const float dec = T.dec;
-#pragma unroll
-    for (int q = 0; q < QT; ++q) {
-        const int t = slot + 4 * q;
-        if (t >= TILES) break;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[q][r] *= dec;
-        const float* Ap = sB + 4 * hf * BP + 32 * (t / PT) + i32;
-        const float* Bp = sV + 4 * hf * VP + 32 * (t % PT) + i32;
-#pragma unroll
-        for (int s = 0; s < kFR / 8; ++s) {
-            const float4 w = *reinterpret_cast<const float4*>(&T.w[8 * s + 4 * hf]);
-            const float wj[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-                acc[q] = bwd_mfma(Ap[(8 * s + jj) * BP], wj[jj] * Bp[(8 * s + jj) * VP], acc[q]);
-        }
-    }
-}
-
 template <int PB, int N>
 struct FStateLds {
     float B[kFR * (N + 4)];
@@ -180,7 +107,7 @@ struct FStateLds {
 };
 
 template <typename T, int PB, int N>
-__global__ __launch_bounds__(256) void ssd_f32_state(SsdF32Params p) {
+__global__ __launch_bounds__(256, 3) void ssd_f32_state(SsdF32Params p) {
     extern __shared__ __align__(16) char f_smem[];
     FStateLds<PB, N>& S = *reinterpret_cast<FStateLds<PB, N>*>(f_smem);
     constexpr int PT = PB / 32, TILES = PT * (N / 32), QT = (TILES + 3) / 4, NT = 256;
@@ -197,13 +124,13 @@ __global__ __launch_bounds__(256) void ssd_f32_state(SsdF32Params p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
     auto fetch = [&](int c) {
-        f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p, c, tid);
-        f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p, c, tid);
+        f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
+        f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
         if (wv == 0) rt = f_tab_fetch(p, j, c, lane);
     };
     auto commit = [&](int c) {
-        f_commit<T, N, NT, N + 4>(rb, S.B, p, c, tid);
-        f_commit<T, PB, NT, PB + 8>(rv, S.V, p, c, tid);
+        f_commit<T, N, NT, N + 4>(rb, S.B, p.L, p.mshift, c, tid);
+        f_commit<T, PB, NT, PB + 8>(rv, S.V, p.L, p.mshift, c, tid);
         if (wv == 0) f_tab_commit(p, rt, S.T, A, c, lane);
     };
     fetch(j.c0);
@@ -213,7 +140,7 @@ __global__ __launch_bounds__(256) void ssd_f32_state(SsdF32Params p) {
     for (int c = j.c0; c < j.c1; ++c) {
         if (c + 1 < j.c1) fetch(c + 1);
         total += S.T.end;
-        f_update<PB, N, QT>(acc, S.B, S.V, S.T, wv, i32, hf);
+        f_update<PB, N, QT, PB + 8>(acc, S.B, S.V, S.T.w, S.T.dec, wv, i32, hf);
         __syncthreads();
         if (c + 1 < j.c1) commit(c + 1);
         __syncthreads();
@@ -257,15 +184,15 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
     FRaw<T> rb[kFR * N / 4 / NT], rc[kFR * N / 4 / NT], rv[kFR * PB / 4 / NT];
     FTabRaw rt = {0.f, 0.f, 0.f};
     auto fetch = [&](int c) {
-        f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p, c, tid);
-        f_fetch<T, N, NT>(rc, Cb, p.C_sl, p.C_sm, p, c, tid);
-        f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p, c, tid);
+        f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
+        f_fetch<T, N, NT>(rc, Cb, p.C_sl, p.C_sm, p.L, p.mshift, c, tid);
+        f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
         if (wv == 0) rt = f_tab_fetch(p, j, c, lane);
     };
     auto commit = [&](int c) {
-        f_commit<T, N, NT, NP>(rb, S.B, p, c, tid);
-        f_commit<T, N, NT, NP>(rc, S.C, p, c, tid);
-        f_commit<T, PB, NT, VP>(rv, S.V, p, c, tid);
+        f_commit<T, N, NT, NP>(rb, S.B, p.L, p.mshift, c, tid);
+        f_commit<T, N, NT, NP>(rc, S.C, p.L, p.mshift, c, tid);
+        f_commit<T, PB, NT, VP>(rv, S.V, p.L, p.mshift, c, tid);
         if (wv == 0) f_tab_commit(p, rt, S.T, A, c, lane);
     };
     const bool st = wv >= 4;  // wave-uniform
@@ -394,7 +321,7 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
                 }
             }
         }
-        if (st) f_update<PB, N, QT>(acc, S.B, S.V, S.T, w4, i32, hf);
+        if (st) f_update<PB, N, QT, PB + 8>(acc, S.B, S.V, S.T.w, S.T.dec, w4, i32, hf);
         __syncthreads();
         if (c + 1 < j.c1) {
             commit(c + 1);
