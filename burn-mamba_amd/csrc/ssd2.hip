@@ -378,7 +378,7 @@ extern "C" size_t mamba_ssd2_workspace_size(const mamba_ssd2_args* a) {
     Ssd2Params p;
     if (ssd2_make_params(a, &p) != MAMBA_OK) return 0;
     size_t ws = ssd2_generic_workspace(p);
-    const size_t fast = ssd2_mfma_workspace(p);
+    const size_t fast = ssd2_mfma_supported(p) ? ssd2_mfma_workspace_best(p) : ssd2_mfma_workspace(p);
     if (ws < fast) ws = fast;
     SsdF32Params f;
     if (ssd2_f32_params(p, &f) && ws < ssd_f32_workspace(f)) ws = ssd_f32_workspace(f);
@@ -413,7 +413,7 @@ static int ssd2_dispatch(const mamba_ssd2_args* a, void* ws, size_t ws_bytes, hi
             set_error("mamba_ssd2_fwd: workspace missing or too small");
             return MAMBA_ERR_WORKSPACE;
         }
-        return ssd2_mfma_launch(p, ws, stream, ev0, ev1);
+        return ssd2_mfma_launch(p, ws, ws_bytes, stream, ev0, ev1);
     }
     // f32 MFMA wherever shape and layout allow; the SIMT kernels take the rest,
     // and a workspace sized for them alone

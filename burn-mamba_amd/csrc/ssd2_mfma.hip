@@ -4,11 +4,13 @@
 // state, K4 state passing, K5 chunk scan) and the trait default body
 // src/mamba2/ssd/serial_recalculated/serial_recalculated.rs:98-155.
 //
-// Two launches per call:
+// Two launches per call, three where the sequence is split into segments:
 //   1. ssd2_prep_pack (per batch, chunk, group): the group-shared causal
 //      C_c.B_c^T tiles (K2, computed once per group instead of once per head,
 //      f32 accumulation rounded to bf16), C_c and B_c in bf16, written as one
 //      packed run of 1 KB MFMA operand fragments per (batch, chunk, group).
+//   (ssd2_seg_state: the segments' states from zero, where (batch, head) alone
+//      leaves the chip idle.)
 //   2. ssd2_scan_wu: one wave per (batch, head, 32-wide headdim half) walks
 //      the chunks in order, with the running state in its MFMA accumulators
 //      for the whole sequence (K4 needs no HBM round trip).  The HPW waves of
@@ -28,6 +30,7 @@
 // Any permutation of k that A and B share leaves the product unchanged; the
 // row/col mappings and the D layout are what the indexing below relies on.
 
+#include <algorithm>
 #include <cstdlib>
 
 #include "ssd2.h"
@@ -75,6 +78,15 @@ __device__ __forceinline__ f32x16_t zero16() {
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
     return z;
 }
+
+// Segments of a launch: chunks [s cps, (s + 1) cps) each, with the states of all
+// but the last from zero ([b h, headdim half][S][tile][16][64], accumulator
+// order) and their log2 decays ([b h][S]).
+struct Ssd2Seg {
+    int S, cps;
+    float* state;
+    float* decay;
+};
 
 // Fragments per (batch, chunk, group), in the order the scan kernel stages them:
 //   CB  it*(it+1) + ks         (C.B^T)[i = 32 it + lane%32][j = 16 ks + 8 (lane/32) + e],
@@ -230,8 +242,12 @@ __global__ __launch_bounds__(256) void ssd2_prep_pack(Ssd2Params p, bf16_t* frag
 // which chunk c + 1's fragments are complete and chunk c's buffer is free.
 // The launch bound caps a wave at 256 registers (two waves per SIMD), which
 // keeps the accumulators in VGPRs next to the VALU work that scales them.
-template <int N, int Q, int HPW>
-__global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu(Ssd2Params p, const bf16_t* frag) {
+//
+// SEG: blockIdx.y is a segment of sg.cps chunks, whose entry state is the
+// initial state carried through the earlier segments' (ssd2_seg_state).
+template <int N, int Q, int HPW, bool SEG>
+__global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu(Ssd2Params p, const bf16_t* frag,
+                                                                                Ssd2Seg sg) {
     using FL = FragLayout<N, Q>;
     constexpr int T = FL::T, NK = FL::NK, KS = FL::KS, NTN = FL::NTN, NF = FL::NF;
     constexpr int XP = Q + 8;                 // s_xg row pitch (bf16)
@@ -269,6 +285,8 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
     const int p0 = ph * 32;
     const float A2 = p.A[h] * kLog2e;
     const float Dh = p.D ? p.D[h] : 0.f;
+    const int c_lo = SEG ? (int)blockIdx.y * sg.cps : 0;
+    const int c_hi = SEG ? min(p.nch, c_lo + sg.cps) : p.nch;
 
     // ---- the state h^T: tile nt, register v holds (n = 32 nt + 8 (v/4) + 4 half + v%4, p = p0 + r)
     f32x16_t hacc[NTN];
@@ -291,6 +309,19 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
                 hacc[nt][4 * q] = v.x; hacc[nt][4 * q + 1] = v.y;
                 hacc[nt][4 * q + 2] = v.z; hacc[nt][4 * q + 3] = v.w;
             }
+        if constexpr (SEG) {
+            const int64_t bh = (int64_t)b * p.H + h;
+            const float* st = sg.state + (bh * 2 + ph) * sg.S * (NTN * 1024) + lane0;
+#pragma unroll 2
+            for (int u = 0; u < (int)blockIdx.y; ++u) {
+                const float dec = __builtin_amdgcn_exp2f(sg.decay[bh * sg.S + u]);
+#pragma unroll
+                for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        hacc[nt][v] = __builtin_fmaf(hacc[nt][v], dec, st[(int64_t)u * (NTN * 1024) + nt * 1024 + v * 64]);
+            }
+        }
     }
 
     const bf16_t* xhead = (const bf16_t*)p.x + (int64_t)b * p.x_sb + (int64_t)h * p.x_sh + p0;
@@ -353,8 +384,8 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
             }
     };
 
-    stage(0, s_fragA, lane0);
-    fetch(0, lane0);
+    stage(c_lo, s_fragA, lane0);
+    fetch(c_lo, lane0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     uint32_t pf = 0u, pf_sink = 0u;
@@ -372,10 +403,10 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
         const int r = lane & 31, half = lane >> 5;
         // ---- chunk c + 1's fragments into the other buffer (free since the
         // last barrier)
-        if (c + 1 < p.nch) stage(c + 1, nxt, lane);
+        if (c + 1 < c_hi) stage(c + 1, nxt, lane);
         // ---- the previous chunk's outputs: issued here, they have this whole
         // chunk to complete before the barrier's wait
-        if (c > 0) store_tiles(c - 1, lane);
+        if (c > c_lo) store_tiles(c - 1, lane);
         // ---- K1: dt and its cumsum (log2 units), one position per lane
         const float cs2 = wave_incl_scan(dtq * A2);
         if (lane < Q) {
@@ -426,11 +457,11 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
         }
         // ---- chunk c + 1's x rows and dt into registers (they land during
         // this chunk's MFMA work)
-        if (c + 1 < p.nch) fetch(c + 1, lane);
+        if (c + 1 < c_hi) fetch(c + 1, lane);
         // L2 warm-up of chunk c + 2's fragments: the workgroups of a group
         // share them and sit on one XCD; one dword per 128-byte line, spread
         // over the workgroups of the group
-        if (MAMBA_SSD2_L2_WARM && c + 2 < p.nch) {
+        if (MAMBA_SSD2_L2_WARM && c + 2 < c_hi) {
             const int nslice = (hpg / HPW) * 2, slice = (hq % (hpg / HPW)) * 2 + ph;
             const int line = threadIdx.x * nslice + slice;  // 128-byte lines of the NF KB block
             if (line < NF * 8)
@@ -633,15 +664,15 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
     };
-    for (int c = 0; c < p.nch; c += 2) {
+    for (int c = c_lo; c < c_hi; c += 2) {
         chunk(c, s_fragA, s_fragB);
-        if (c + 1 < p.nch) chunk(c + 1, s_fragB, s_fragA);
+        if (c + 1 < c_hi) chunk(c + 1, s_fragB, s_fragA);
     }
-    store_tiles(p.nch - 1, lane0);
+    store_tiles(c_hi - 1, lane0);
     // keeps the L2 warm-up loads alive (the condition never holds: L >= 1)
     if (p.L < 0 && pf_sink == 0x9e3779b9u) p.hT[0] = 0.f;
     // final state (f32): h[p = p0 + r][n] = phi h-hat^T[n][p]
-    {
+    if (!SEG || (int)blockIdx.y == sg.S - 1) {
         const int r = lane0 & 31, half = lane0 >> 5;
         const float ph = __builtin_amdgcn_exp2f(lphi);
 #pragma unroll
@@ -656,6 +687,101 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
                 *(float4*)(hTr + 32 * nt + 8 * q + 4 * half) =
                     make_float4(hacc[nt][4 * q], hacc[nt][4 * q + 1], hacc[nt][4 * q + 2], hacc[nt][4 * q + 3]);
     }
+}
+
+// ------------------------------------------------- segment states (K3 + K4) --
+// The state of each segment but the last from zero, one wave per (batch, head,
+// 32-wide headdim half, segment): the scan's state recurrence alone, with the
+// chunk's whole decay applied to the accumulators (xg_j = x_j dt_j exp(cs_end -
+// cs_j) <= x_j dt_j).  Waves share nothing, so there is no barrier; the B
+// fragments come straight from L2 as MFMA operands, a chunk ahead.
+template <int N, int Q>
+__global__ __launch_bounds__(256, 2) void ssd2_seg_state(Ssd2Params p, const bf16_t* frag, Ssd2Seg sg) {
+    using FL = FragLayout<N, Q>;
+    constexpr int KS = FL::KS, NTN = FL::NTN, NF = FL::NF, NB = NTN * KS, XP = Q + 8, XPT = Q / 32;
+    __shared__ __align__(16) bf16_t s_xg[4][32][XP];
+    const int wave = wave_id(), lane = threadIdx.x & 63, r = lane & 31, half = lane >> 5;
+    int64_t id = (int64_t)blockIdx.x * 4 + wave;
+    if (id >= (int64_t)p.nb * p.H * 2 * (sg.S - 1)) return;  // whole waves; no barrier follows
+    const int ph = (int)(id & 1);
+    id >>= 1;
+    const int h = (int)(id % p.H);
+    id /= p.H;
+    const int s = (int)(id % (sg.S - 1)), b = (int)(id / (sg.S - 1));
+    const int g = h / (p.H / p.G), p0 = 32 * ph;
+    const float A2 = p.A[h] * kLog2e;
+    const bf16_t* xhead = (const bf16_t*)p.x + (int64_t)b * p.x_sb + (int64_t)h * p.x_sh + p0;
+    const float* dthead = p.dt + (int64_t)b * p.dt_sb + (int64_t)h * p.dt_sh;
+    const uint32_t xrow = (uint32_t)p.x_sl * 2u;
+    const bf16_t* gfrag = frag + ((int64_t)b * p.nch * p.G + g) * NF * 512 + FL::B0 * 512 + lane * 8;
+    const int64_t grp_stride = (int64_t)p.G * NF * 512;
+    const int c0 = s * sg.cps, c1 = c0 + sg.cps;  // only the last segment is shorter
+    uint4 xq[XPT][2], bq[NB];
+    float dtq;
+    auto fetch = [&](int cc) {
+        const int jp = lane >> 2, pv = lane & 3;
+        const uint32_t rows = (uint32_t)max(0, min(Q, p.L - cc * Q));
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xhead + (int64_t)cc * Q * p.x_sl, rows * xrow);
+        const uint32_t off0 = (uint32_t)(2 * jp) * xrow + pv * 16;
+#pragma unroll
+        for (int m = 0; m < XPT; ++m) {
+            xq[m][0] = buf_ld16(rx, off0, (uint32_t)(32 * m) * xrow);
+            xq[m][1] = buf_ld16(rx, off0, (uint32_t)(32 * m + 1) * xrow);
+        }
+        const __amdgpu_buffer_rsrc_t rd =
+            buf_rsrc(dthead + (int64_t)cc * Q * p.dt_sl, rows * (uint32_t)p.dt_sl * 4u);
+        dtq = lane < Q ? buf_ld4(rd, lane * (uint32_t)p.dt_sl * 4u) : 0.f;
+#pragma unroll
+        for (int f = 0; f < NB; ++f) bq[f] = *(const uint4*)(gfrag + (int64_t)cc * grp_stride + f * 512);
+    };
+    f32x16_t hacc[NTN];
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt) hacc[nt] = zero16();
+    float total = 0.f;
+    fetch(c0);
+    for (int c = c0; c < c1; ++c) {
+        const float cs2 = wave_incl_scan(dtq * A2);
+        const float end = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs2), 63));
+        const float gj = dtq * __builtin_amdgcn_exp2f(end - cs2);
+        total += end;
+        const int jp = lane >> 2, pv = lane & 3;
+#pragma unroll
+        for (int m = 0; m < XPT; ++m) {
+            const int j0 = 2 * (jp + 16 * m);
+            const float g0 = __shfl(gj, j0, 64), g1 = __shfl(gj, j0 + 1, 64);
+            const uint32_t a0[4] = {xq[m][0].x, xq[m][0].y, xq[m][0].z, xq[m][0].w};
+            const uint32_t a1[4] = {xq[m][1].x, xq[m][1].y, xq[m][1].z, xq[m][1].w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                *(uint32_t*)&s_xg[wave][pv * 8 + 2 * k][j0] =
+                    pack_bf16x2(__uint_as_float(a0[k] << 16) * g0, __uint_as_float(a1[k] << 16) * g1);
+                *(uint32_t*)&s_xg[wave][pv * 8 + 2 * k + 1][j0] =
+                    pack_bf16x2(__uint_as_float(a0[k] & 0xffff0000u) * g0, __uint_as_float(a1[k] & 0xffff0000u) * g1);
+            }
+        }
+        uint4 bc[NB];
+#pragma unroll
+        for (int f = 0; f < NB; ++f) bc[f] = bq[f];
+        if (c + 1 < c1) fetch(c + 1);
+        const float dec = __builtin_amdgcn_exp2f(end);
+#pragma unroll
+        for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) hacc[nt][v] *= dec;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const bf16x8_t bx = *(const bf16x8_t*)&s_xg[wave][r][ks * 16 + 8 * half];
+#pragma unroll
+            for (int nt = 0; nt < NTN; ++nt) hacc[nt] = mfma32x32x16(as_bf16x8(bc[nt * KS + ks]), bx, hacc[nt]);
+        }
+    }
+    const int64_t bh = (int64_t)b * p.H + h;
+    float* out = sg.state + ((bh * 2 + ph) * sg.S + s) * (NTN * 1024) + lane;
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) out[nt * 1024 + v * 64] = hacc[nt][v];
+    if (ph == 0 && lane == 0) sg.decay[bh * sg.S + s] = total;
 }
 
 // ------------------------------------------------------------ host side --
@@ -694,70 +820,108 @@ static size_t frag_count(const Ssd2Params& p) {
     return (size_t)(T * (T + 1) + T * NK + NTN * KS);
 }
 
-size_t ssd2_mfma_workspace(const Ssd2Params& p0) {
-    const Ssd2Params p = fast_params(p0);
+static size_t frag_bytes(const Ssd2Params& p) {
     return align_up((size_t)p.nb * p.nch * p.G * frag_count(p) * 1024, 256);
 }
+static size_t seg_bytes(const Ssd2Params& p, int S) {
+    const size_t bh = (size_t)p.nb * p.H * S;
+    return S > 1 ? align_up(bh * 64 * p.N * sizeof(float), 256) + align_up(bh * sizeof(float), 256) : 0;
+}
 
-// Heads per workgroup (waves per workgroup): one of 5, 4, 2, 1 dividing the
-// heads of a group.  The scan kernel's LDS (two chunks of group fragments)
-// allows one workgroup per CU, so a launch of nwg workgroups takes
-// ceil(nwg / 256) rounds on MI355X's 256 CUs, each as long as the busiest
-// SIMD's ceil(HPW / 4) waves.  Ties go to the larger set, which stages each
-// fragment for more heads.  MAMBA_SSD2_HPW (read on every call) forces a
-// valid choice.
-static int choose_hpw(const Ssd2Params& p) {
+// Heads per workgroup (waves per workgroup: one of 5, 4, 2, 1 dividing the heads
+// of a group) and segments per sequence.  The scan's LDS (two chunks of group
+// fragments) allows one workgroup per CU, so a launch of nwg workgroups takes
+// ceil(nwg / 256) rounds on MI355X's 256 CUs, each as long as a segment's
+// chunks; five waves share four SIMDs, which costs a chunk about a fifth.  In
+// units of a chunk (about 4.5 us): a segment adds its entry state (0.5 and 0.1
+// per earlier segment) and the state pass a third of a chunk per chunk for
+// every 2048 waves, and a launch (1).  Measured at 80 heads x 64 x 128: batch 1,
+// 3001 positions 191 -> 73 us, batch 2 x 2048 (the forward of a training
+// step) 160 -> 87 us; batch 8 x 4096 fills the chip and stays whole.  Ties
+// go to the larger head set, which stages each fragment for more heads, and to
+// fewer segments.  MAMBA_SSD2_HPW (read on every call) forces a valid head set.
+struct Ssd2Plan {
+    int hpw, S, cps;
+};
+static Ssd2Plan choose_plan(const Ssd2Params& p, size_t ws_bytes) {
     const int hpg = p.H / p.G;
-    const char* e = getenv("MAMBA_SSD2_HPW");
-    if (e) {
+    int forced = 0;
+    if (const char* e = getenv("MAMBA_SSD2_HPW")) {
         const int v = atoi(e);
-        if ((v == 1 || v == 2 || v == 4 || v == 5) && hpg % v == 0) return v;
+        if ((v == 1 || v == 2 || v == 4 || v == 5) && hpg % v == 0) forced = v;
     }
     constexpr int kCUs = 256;
-    int best = 1;
-    int64_t best_cost = INT64_MAX;
+    Ssd2Plan best{1, 1, p.nch};
+    double best_cost = 0.;
     for (int hpw : {5, 4, 2, 1}) {
-        if (hpg % hpw != 0) continue;
+        if (forced ? hpw != forced : hpg % hpw != 0) continue;
         const int64_t nwg = (int64_t)p.nb * (p.H / hpw) * 2;
-        const int64_t cost = (nwg + kCUs - 1) / kCUs * ((hpw + 3) / 4);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = hpw;
+        for (int n = 1; n <= std::min(p.nch, 32); ++n) {
+            const int cps = (p.nch + n - 1) / n, S = (p.nch + cps - 1) / cps;
+            if (S != n || (S > 1 && frag_bytes(p) + seg_bytes(p, S) > ws_bytes)) continue;
+            const int64_t rounds = (nwg * S + kCUs - 1) / kCUs;
+            const int64_t pass = ((int64_t)p.nb * p.H * 2 * (S - 1) + 2047) / 2048;
+            const double chunk = hpw == 5 ? 1.2 : 1.;
+            const double cost =
+                rounds * chunk * (cps + (S > 1 ? 0.5 + 0.1 * S : 0.)) + (S > 1 ? pass * 0.33 * cps + 1. : 0.);
+            if (best_cost == 0. || cost < best_cost) {
+                best_cost = cost;
+                best = {hpw, S, cps};
+            }
         }
     }
     return best;
 }
 
+size_t ssd2_mfma_workspace(const Ssd2Params& p0) { return frag_bytes(fast_params(p0)); }
+size_t ssd2_mfma_workspace_best(const Ssd2Params& p0) {
+    const Ssd2Params p = fast_params(p0);
+    return frag_bytes(p) + seg_bytes(p, choose_plan(p, SIZE_MAX).S);
+}
+
 template <int N, int Q, int HPW>
-static void launch_scan(const Ssd2Params& p, const bf16_t* frag, hipStream_t stream) {
+static void launch_scan(const Ssd2Params& p, const bf16_t* frag, const Ssd2Seg& sg, hipStream_t stream) {
     const int nwg = p.nb * (p.H / HPW) * 2;
-    hipLaunchKernelGGL((ssd2_scan_wu<N, Q, HPW>), dim3(nwg), dim3(64 * HPW), 0, stream, p, frag);
+    if (sg.S > 1)
+        hipLaunchKernelGGL((ssd2_scan_wu<N, Q, HPW, true>), dim3(nwg, sg.S), dim3(64 * HPW), 0, stream, p, frag, sg);
+    else
+        hipLaunchKernelGGL((ssd2_scan_wu<N, Q, HPW, false>), dim3(nwg), dim3(64 * HPW), 0, stream, p, frag, sg);
 }
 
 template <int N, int Q>
-static int launch_q(const Ssd2Params& p, void* ws, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+static int launch_q(const Ssd2Params& p, void* ws, size_t ws_bytes, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
     bf16_t* frag = (bf16_t*)ws;
+    const Ssd2Plan plan = choose_plan(p, ws_bytes);
+    Ssd2Seg sg{plan.S, plan.cps, nullptr, nullptr};
     hipLaunchKernelGGL((ssd2_prep_pack<N, Q>), dim3(p.nch * p.G, p.nb), dim3(256), 0, stream, p, frag);
     MAMBA_CHECK_LAUNCH();
+    if (plan.S > 1) {
+        sg.state = (float*)((char*)ws + frag_bytes(p));
+        sg.decay = sg.state + align_up((size_t)p.nb * p.H * plan.S * 64 * N * sizeof(float), 256) / sizeof(float);
+        const int64_t waves = (int64_t)p.nb * p.H * 2 * (plan.S - 1);
+        hipLaunchKernelGGL((ssd2_seg_state<N, Q>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, p, frag, sg);
+        MAMBA_CHECK_LAUNCH();
+    }
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
-    switch (choose_hpw(p)) {
-        case 5: launch_scan<N, Q, 5>(p, frag, stream); break;
-        case 4: launch_scan<N, Q, 4>(p, frag, stream); break;
-        case 2: launch_scan<N, Q, 2>(p, frag, stream); break;
-        default: launch_scan<N, Q, 1>(p, frag, stream); break;
+    switch (plan.hpw) {
+        case 5: launch_scan<N, Q, 5>(p, frag, sg, stream); break;
+        case 4: launch_scan<N, Q, 4>(p, frag, sg, stream); break;
+        case 2: launch_scan<N, Q, 2>(p, frag, sg, stream); break;
+        default: launch_scan<N, Q, 1>(p, frag, sg, stream); break;
     }
     MAMBA_CHECK_LAUNCH();
     if (ev1) MAMBA_CHECK_HIP(hipEventRecord(ev1, stream));
     return MAMBA_OK;
 }
 
-int ssd2_mfma_launch(const Ssd2Params& p0, void* ws, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+int ssd2_mfma_launch(const Ssd2Params& p0, void* ws, size_t ws_bytes, hipStream_t stream, hipEvent_t ev0,
+                     hipEvent_t ev1) {
     const Ssd2Params p = fast_params(p0);
     if (p.N == 64)
-        return p.Q == 32 ? launch_q<64, 32>(p, ws, stream, ev0, ev1) : launch_q<64, 64>(p, ws, stream, ev0, ev1);
-    return p.Q == 32 ? launch_q<128, 32>(p, ws, stream, ev0, ev1) : launch_q<128, 64>(p, ws, stream, ev0, ev1);
+        return p.Q == 32 ? launch_q<64, 32>(p, ws, ws_bytes, stream, ev0, ev1)
+                         : launch_q<64, 64>(p, ws, ws_bytes, stream, ev0, ev1);
+    return p.Q == 32 ? launch_q<128, 32>(p, ws, ws_bytes, stream, ev0, ev1)
+                     : launch_q<128, 64>(p, ws, ws_bytes, stream, ev0, ev1);
 }
-
-int ssd2_mfma_hpw(const Ssd2Params& p) { return choose_hpw(fast_params(p)); }
 
 }  // namespace mamba
