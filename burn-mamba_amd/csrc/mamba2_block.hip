@@ -7,8 +7,8 @@
 //    window, + bias, SiLU (silu.rs:24-27); dt = softplus(dt_raw + dt_bias)
 //    clamped to dt_limit (:695, softplus.rs:17-48).  The conv window of the
 //    cache becomes the last `kernel` columns of the padded input
-//    (mamba2.rs:652-655); it is updated in place by a second kernel that runs
-//    after the first has read the old window.  With nheads = 0 there is no dt
+//    (mamba2.rs:652-655); it is updated in place by the workgroups of the first
+//    positions, the only ones that read the old window.  With nheads = 0 there is no dt
 //    and this is the Mamba-1 prefill conv (Mamba1::forward layer 2,
 //    src/mamba1/mamba1.rs:300-340: the same padded causal conv, SiLU and
 //    window update over the x half of the in_proj rows).
@@ -65,14 +65,19 @@ struct M2ConvParams {
     const float* dt_bias; float dt_lo, dt_hi;
     void* out; int64_t out_sb, out_sl;
     float* dt;
+    int tile, off;  // positions per workgroup (multiples of kM2ConvRows), fewer by off in the first
+    bool w_vec;     // the weights and the window are 16-byte aligned
 };
 
-constexpr int kM2ConvTile = 64;  // positions per workgroup
 constexpr int kM2ConvRows = 8;   // input rows in flight per thread
 constexpr int kM2MaxK = 8;
+static_assert(kM2ConvRows >= kM2MaxK - 1, "only a sequence's first tile reads the old window");
 
-// One thread per VW consecutive channels over a tile of kM2ConvTile positions:
-// the last K - 1 inputs stay in registers, so every input is read once.
+// One thread per VW consecutive channels over a tile of p.tile positions: the
+// last K - 1 inputs stay in registers, so a tile reads every input once and
+// K - 1 rows of the tile before it.  Bound by HBM (input read, output written)
+// where there are workgroups enough; the tile is 64 positions there and down to
+// 8 where 64 would leave CUs idle (conv_tile below).
 // Channels c of position l: sum_k w[c][k] xpad[l + k] with xpad = [the
 // window's last K - 1 columns | the new inputs].  The channel blocks of a
 // tile also share out the tile's dt.
@@ -80,14 +85,23 @@ template <typename TI, typename TO, int VW, int K>
 __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
     const int tile = blockIdx.x, b = blockIdx.z;
     const int c0 = (blockIdx.y * 256 + threadIdx.x) * VW;
-    const int l0 = tile * kM2ConvTile, l1 = min(p.L, l0 + kM2ConvTile);
+    // the first tile, which also writes the new window, is shorter by p.off
+    const int l0 = max(0, tile * p.tile - p.off), l1 = min(p.L, (tile + 1) * p.tile - p.off);
     const TI* proj = static_cast<const TI*>(p.proj) + (int64_t)b * p.proj_sb;
     if (c0 < p.V) {
         float w[VW][K], bias[VW];
 #pragma unroll
         for (int e = 0; e < VW; ++e) {
+            const float* we = p.w + (int64_t)(c0 + e) * K;
+            if (K == 4 && p.w_vec) {
+                const float4 v = *(const float4*)we;
+                const float wk[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int k = 0; k < K; ++k) w[e][k] = p.w[(int64_t)(c0 + e) * K + k];
+                for (int k = 0; k < K; ++k) w[e][k] = wk[k & 3];
+            } else {
+#pragma unroll
+                for (int k = 0; k < K; ++k) w[e][k] = we[k];
+            }
             bias[e] = p.bias ? p.bias[c0 + e] : 0.f;
         }
         // window: win[j] holds xpad[l0 + j] for j < K - 1 (positions l0 - K + 1 + j)
@@ -166,6 +180,33 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
             load(l, x);
             emit(l, x);
         }
+        // the new window: the last K columns of [old window's last K - 1 | inputs],
+        // by the only threads that have read the old one
+        if (tile == 0) {
+            float* st = p.state + ((int64_t)b * p.V + c0) * K;
+            float nw[VW][K];
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const int l = p.L - K + j;  // input position; before 0: old column K + l
+                float x[VW];
+                if (l >= 0)
+                    load(l, x);
+                else
+#pragma unroll
+                    for (int e = 0; e < VW; ++e) x[e] = st[e * K + K + l];
+#pragma unroll
+                for (int e = 0; e < VW; ++e) nw[e][j] = x[e];
+            }
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                if (K == 4 && p.w_vec) {
+                    *(float4*)(st + 4 * e) = make_float4(nw[e][0], nw[e][1 % K], nw[e][2 % K], nw[e][3 % K]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < K; ++j) st[e * K + j] = nw[e][j];
+                }
+            }
+        }
     }
     // the tile's dt, its (position, head) pairs split over the channel blocks;
     // each thread issues all its loads before its stores
@@ -192,26 +233,6 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
             }
         }
     }
-}
-
-// The new window: the last K columns of [old window's last K - 1 | inputs],
-// one thread per (batch, channel), in place (all K old values are read first).
-template <typename TI>
-__global__ __launch_bounds__(256) void mamba2_conv_state_kernel(M2ConvParams p) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t)p.nb * p.V) return;
-    const int b = (int)(i / p.V), c = (int)(i % p.V);
-    const TI* proj = static_cast<const TI*>(p.proj) + (int64_t)b * p.proj_sb;
-    float* st = p.state + i * p.K;
-    float old[kM2MaxK], nw[kM2MaxK];
-    for (int k = 0; k < p.K; ++k) old[k] = st[k];
-    // padded column j of the new window: padded index (L - 1) + j; padded
-    // index q < K - 1 is old column q + 1, else input position q - (K - 1)
-    for (int j = 0; j < p.K; ++j) {
-        const int q = p.L - 1 + j;
-        nw[j] = q < p.K - 1 ? old[q + 1] : m2_ld1(proj + (int64_t)(q - (p.K - 1)) * p.proj_sl + p.xbc_off + c);
-    }
-    for (int k = 0; k < p.K; ++k) st[k] = nw[k];
 }
 
 struct M2NormParams {
@@ -345,6 +366,18 @@ __global__ __launch_bounds__(256) void mamba2_gated_norm_res_kernel(M2NormParams
     }
 }
 
+// Positions per workgroup: 64, halved while the launch would have fewer than 192
+// workgroups; shorter tiles than that re-read the weights (20 bytes per channel)
+// and window rows too often.  Measured against 64 positions always and a launch
+// of its own for the window, 5376 channels, bf16: 1 x 200 tokens 26.6 -> 11.1 us,
+// 2 x 1021 31.4 -> 18.2, 4 x 2000 57.5 -> 50.7, 8 x 4096 173 -> 171 us (with 384
+// or 768 workgroups asked for, 2 x 1021 takes 25.6 or 28.1 us).
+static int conv_tile(const M2ConvParams& p, int cblocks) {
+    int t = 64;
+    while (t > kM2ConvRows && (int64_t)((p.L + t - 1) / t) * cblocks * p.nb < 192) t /= 2;
+    return t;
+}
+
 static bool aligned16(const void* q) { return ((uintptr_t)q & 15u) == 0; }
 
 }  // namespace mamba
@@ -378,8 +411,13 @@ extern "C" int mamba2_conv_fwd(const mamba2_conv_args* a, mamba_stream_t stream)
                      (p.nb == 1 || p.proj_sb % 8 == 0) && p.out_sl % 8 == 0 && (p.nb == 1 || p.out_sb % 8 == 0) &&
                      aligned16(p.proj) && aligned16(p.out);
     const int vw = vec ? 8 : 1;
-    const int tiles = (p.L + kM2ConvTile - 1) / kM2ConvTile;
     const int cblocks = (p.V / vw + 255) / 256;
+    p.tile = conv_tile(p, cblocks);
+    p.w_vec = aligned16(p.w) && aligned16(p.state);
+    // all workgroups run at once up to long sequences: the window's loads and
+    // stores would make the first tile's the last to end
+    p.off = p.tile >= 2 * kM2ConvRows ? p.tile / 2 : 0;
+    const int tiles = (p.L + p.off + p.tile - 1) / p.tile;
     MAMBA_CHECK_ARG(tiles < (1 << 30) && p.nb <= 65535, "too many tiles or batch rows");
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid(tiles, cblocks, p.nb), block(256);
@@ -413,12 +451,6 @@ extern "C" int mamba2_conv_fwd(const mamba2_conv_args* a, mamba_stream_t stream)
 #undef M2CONV_V
 #undef M2CONV_K
 #undef M2CONV
-    MAMBA_CHECK_LAUNCH();
-    const int64_t n = (int64_t)p.nb * p.V;
-    if (in_bf)
-        hipLaunchKernelGGL(mamba2_conv_state_kernel<bf16_t>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p);
-    else
-        hipLaunchKernelGGL(mamba2_conv_state_kernel<float>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p);
     MAMBA_CHECK_LAUNCH();
     return MAMBA_OK;
 }

@@ -1,0 +1,32 @@
+"""The prefill conv at every tile length its launch takes (8 to 64 positions per
+workgroup), ragged ends and sequences shorter than the window, with the window
+updated in place by the first tile's workgroups, vs the oracle (f32: rtol 1e-4;
+the window holds input values: exact)."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# (b, l, channels): tiles of 64, 32, 16 and 8 positions; scalar channels; l < kernel
+CASES = [(8, 4101, 8), (4, 4101, 8), (2, 4101, 8), (1, 500, 16), (2, 300, 7), (3, 2, 24), (1, 1, 8)]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_conv1d_fwd(case):
+    import torch
+    import mamba_hip
+    import oracle
+    b, L, c = case
+    K = 4
+    rng = np.random.default_rng(sum(case))
+    x, st = rng.standard_normal((b, L, c), dtype=np.float32), rng.standard_normal((b, c, K), dtype=np.float32)
+    w, bias = rng.standard_normal((c, K), dtype=np.float32), rng.standard_normal(c, dtype=np.float32)
+    s = torch.from_numpy(st).cuda()
+    g = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    out = mamba_hip.conv1d_fwd(g(x), s, g(w), g(bias))
+    torch.cuda.synchronize()
+    want, _, wst = oracle.mamba2_conv_fwd(x, w, bias, st, np.zeros(0), 0, 0, c, 0)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=1e-4, atol=2e-5)
+    np.testing.assert_array_equal(s.cpu().numpy(), wst.astype(np.float32))
