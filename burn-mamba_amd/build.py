@@ -36,6 +36,7 @@ FILE_FLAGS = {
     "ssd3_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "mamba3_fused.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "ssd_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "mm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "ssd_f32_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     # the decode products: accumulators in VGPRs keep a wave within 128
     # registers (four waves per SIMD)

@@ -270,6 +270,15 @@ class LinearArgs(ctypes.Structure):
     ]
 
 
+class MmF32Args(ctypes.Structure):
+    _fields_ = [
+        ("batch", c_i32), ("m", c_i32), ("n", c_i32), ("k", c_i32),
+        ("a", c_vp), ("a_sb", c_i64), ("a_sm", c_i64), ("a_sk", c_i64),
+        ("b", c_vp), ("b_sb", c_i64), ("b_sk", c_i64), ("b_sn", c_i64),
+        ("c", c_vp), ("c_sb", c_i64), ("c_sm", c_i64),
+    ]
+
+
 class Mamba2LayerArgs(ctypes.Structure):
     _fields_ = [
         ("batch", c_i32), ("d_model", c_i32), ("nheads", c_i32), ("headdim", c_i32), ("ngroups", c_i32),
@@ -334,6 +343,7 @@ _SIGNATURES = {
     "mamba_linear_pack": ([c_vp, c_i32, c_i32, c_i64, c_i32, c_vp, c_vp], ctypes.c_int),
     "mamba_linear_workspace_size": ([ctypes.POINTER(LinearArgs)], ctypes.c_size_t),
     "mamba_linear_fwd": ([ctypes.POINTER(LinearArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
+    "mamba_mm_f32": ([ctypes.POINTER(MmF32Args), c_vp], ctypes.c_int),
     "mamba2_layer_workspace_size": ([ctypes.POINTER(Mamba2LayerArgs)], ctypes.c_size_t),
     "mamba2_layer_step": ([ctypes.POINTER(Mamba2LayerArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
     "mamba2_layer_step_timed": ([ctypes.POINTER(Mamba2LayerArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp],

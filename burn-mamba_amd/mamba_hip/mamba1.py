@@ -255,6 +255,34 @@ class Mamba1Config:
         )
 
 
+def mm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """mamba_mm_f32: a [z, m, k] @ b [z, k, n] -> [z, m, n] (f32; a unit stride in
+    one of the last two axes of each; expanded batch axes are read in place)."""
+    z, m, k = a.shape
+    n = b.shape[2]
+    if out is None:
+        out = torch.empty((z, m, n), device=a.device, dtype=torch.float32)
+    g = _lib.MmF32Args()
+    g.batch, g.m, g.n, g.k = z, m, n, k
+    g.a, (g.a_sb, g.a_sm, g.a_sk) = a.data_ptr(), a.stride()
+    g.b, (g.b_sb, g.b_sk, g.b_sn) = b.data_ptr(), b.stride()
+    g.c, g.c_sb, g.c_sm = out.data_ptr(), out.stride(0), out.stride(1)
+    check(_lib.lib().mamba_mm_f32(ctypes.byref(g), _stream(a.device)), "mamba_mm_f32")
+    return out
+
+
+def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
+    """Where mamba_mm_f32 takes a block's x_proj and out_proj.  For at most 256
+    tokens per sequence and 512 channels the library picks 256-wide tiles (2 x 256
+    tokens, 512 channels: out_proj 118 us, x_proj 25 us against 7.9 and 7.5; 1 x
+    100: 62 and 28 against 7.3 and 7.5; 1 x 7: 12 and 6.8 against 7.5 and 6.4);
+    past either bound it is the faster one (1 x 301: 6.8 against 9.0; 768 channels
+    and more: 8.6 against 11.8).  Calls that autograd follows, and operands
+    without a unit stride, stay with the library."""
+    return L <= 256 and di <= 512 and all(1 in t.stride()[-2:] and t.dtype == torch.float32 for t in ts) and \
+        not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+
+
 def _wt(w: torch.Tensor, attr: str, col0: int) -> torch.Tensor:
     """The contiguous transpose of w[:, col0:], made once, kept on the weight
     and remade when the weight is updated in place (the derived-copy cache of
@@ -316,16 +344,20 @@ class Mamba1:
         # to the scan), then the selective scan with D u and the silu(res) gate
         # (x_proj and dt_proj time-major too: B and C then stream as whole rows)
         ut = u.transpose(1, 2).contiguous()
-        x_dbl = torch.matmul(_wt(self.x_proj_w, "_mamba_t", 0), ut)          # [b, r + 2n, l]
+        own = _mm_f32_pays(di, L, self.x_proj_w, self.out_proj_w, u)
+        if own:  # reads u where the conv wrote it
+            x_dbl = mm_f32(self.x_proj_w.t().expand(b, -1, -1), u.transpose(1, 2))
+        else:
+            x_dbl = torch.matmul(_wt(self.x_proj_w, "_mamba_t", 0), ut)      # [b, r + 2n, l]
         dt = torch.matmul(_wt(self.dt_proj_w, "_mamba_t", 0), x_dbl[:, :r])  # [b, d_inner, l]
         yt = torch.empty((b, di, L), device=x.device, dtype=torch.float32)
-        final = torch.empty_like(cache.ssm_bir)
+        # the scan reads a channel's initial state before it writes its final one
         mamba1_scan(ut, dt, self.A, x_dbl[:, r:r + n], x_dbl[:, r + n:],
                     D=self.d, z=zt, delta_bias=self.dt_proj_b, delta_softplus=True,
-                    initial_state=cache.ssm_bir, y=yt, final_state=final, events=events)
-        cache.ssm_bir.copy_(final)
+                    initial_state=cache.ssm_bir, y=yt, final_state=cache.ssm_bir, events=events)
+        if own:
+            return mm_f32(yt.transpose(1, 2), self.out_proj_w.expand(b, -1, -1)), cache
         return torch.matmul(yt.transpose(1, 2), self.out_proj_w), cache
-
 
     def step(self, x: torch.Tensor, cache: Optional[Mamba1Cache] = None):
         """Mamba1::step (mamba1.rs:533-612): returns (y [b, d_model], cache); the cache

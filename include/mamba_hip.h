@@ -645,6 +645,19 @@ size_t mamba_linear_workspace_size(const mamba_linear_args* args);
 int mamba_linear_fwd(const mamba_linear_args* args, void* workspace, size_t workspace_bytes,
                      mamba_stream_t stream);
 
+/* Batched f32 products C[b] = A[b] B[b] for prefill blocks of few tokens, in  */
+/* any layout with one unit stride per operand (C's rows are contiguous): the  */
+/* Linears of Mamba1::forward (src/mamba1/mamba1.rs:278-399) formed time-major  */
+/* where the scan wants them.  f32 operands and accumulation.                  */
+typedef struct mamba_mm_f32_args {
+    int32_t batch, m, n, k;
+    const float* a; int64_t a_sb, a_sm, a_sk;
+    const float* b; int64_t b_sb, b_sk, b_sn;
+    float* c; int64_t c_sb, c_sm;
+} mamba_mm_f32_args;
+
+int mamba_mm_f32(const mamba_mm_f32_args* args, mamba_stream_t stream);
+
 /* ------------------------------------------------------------------------- */
 /* Fused pre-norm Mamba-2 layer decode step (Layer::step_one around           */
 /* Mamba2::step, src/modules/layer.rs:224-232 + src/mamba2/mamba2.rs:820-1004): */

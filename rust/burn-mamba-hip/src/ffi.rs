@@ -633,6 +633,34 @@ impl Default for MambaLinearArgs {
 
 #[repr(C)]
 #[derive(Clone, Copy, Debug)]
+pub struct MambaMmF32Args {
+    pub batch: i32,
+    pub m: i32,
+    pub n: i32,
+    pub k: i32,
+    pub a: *const f32,
+    pub a_sb: i64,
+    pub a_sm: i64,
+    pub a_sk: i64,
+    pub b: *const f32,
+    pub b_sb: i64,
+    pub b_sk: i64,
+    pub b_sn: i64,
+    pub c: *mut f32,
+    pub c_sb: i64,
+    pub c_sm: i64,
+}
+
+impl Default for MambaMmF32Args {
+    /// Every size 0, every pointer null, every stride 0.
+    fn default() -> Self {
+        // SAFETY: all fields are integers, floats or raw pointers, for which zero is valid.
+        unsafe { core::mem::zeroed() }
+    }
+}
+
+#[repr(C)]
+#[derive(Clone, Copy, Debug)]
 pub struct Mamba2LayerArgs {
     pub batch: i32,
     pub d_model: i32,
@@ -806,6 +834,7 @@ extern "C" {
     pub fn mamba_linear_pack(weight: *const c_void, d_in: i32, d_out: i32, ld: i64, dtype: i32, packed: *mut c_void, stream: MambaStream) -> c_int;
     pub fn mamba_linear_workspace_size(args: *const MambaLinearArgs) -> usize;
     pub fn mamba_linear_fwd(args: *const MambaLinearArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
+    pub fn mamba_mm_f32(args: *const MambaMmF32Args, stream: MambaStream) -> c_int;
     pub fn mamba2_layer_workspace_size(args: *const Mamba2LayerArgs) -> usize;
     pub fn mamba2_layer_step(args: *const Mamba2LayerArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
     pub fn mamba2_layer_step_timed(args: *const Mamba2LayerArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
