@@ -47,11 +47,12 @@ __device__ __forceinline__ float m3_wrap(float a) {
     return a - rintf(a * (1.f / two_pi)) * two_pi;
 }
 
-// N4 = N/4 lanes per state row (a power of two, <= 64); MM = MIMO rank.
-template <int N4, int MM>
-__global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
+// N4 = N/4 lanes per state row (a power of two, <= 64); MM = MIMO rank; NT
+// threads (m3_launch_nt): the same sums in the same order for any.
+template <int N4, int MM, int NT>
+__global__ __launch_bounds__(NT) void mamba3_step_kernel(M3StepParams p) {
     constexpr int N = 4 * N4;
-    constexpr int RPP = 256 / N4;                  // state rows per pass
+    constexpr int RPP = NT / N4;                   // state rows per pass
     constexpr int MAXPASS = kM3MaxPN / (RPP * N);  // register budget of the prefetch
     const int b = blockIdx.x / p.H, h = blockIdx.x % p.H;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -79,11 +80,11 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     // for MIMO 1 (rotate_bc_step): a row's N/2 pairs over a group of GS lanes
     // (PPL pairs per lane), RPI rows per pass of the workgroup, JR passes
     constexpr int NP = N / 2, GS = NP < 64 ? NP : 64, PPL = NP / GS;
-    constexpr int NROW = 2 * MM, RPI = 256 / GS, JR = (NROW + RPI - 1) / RPI;
+    constexpr int NROW = 2 * MM, RPI = NT / GS, JR = (NROW + RPI - 1) / RPI;
     const int gl = t % GS, rsub = t / GS;
     // ---- this row's inputs first, into registers: the prep below waits for
     // them only, while the state tile (issued next) is still in flight
-    constexpr int RK = (MM * N + 255) / 256;
+    constexpr int RK = (MM * N + NT - 1) / NT;
     const float raw_dt = m3_proj(p, row, o_dt + h), raw_a = m3_proj(p, row, o_a + h),
                 raw_l = m3_proj(p, row, o_l + h), dtb = p.dt_bias[h];
     float raw_rot = 0.f, ang0 = 0.f;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     float rk[RK];
 #pragma unroll
     for (int j = 0; j < RK; ++j) {
-        const int i = t + 256 * j, m = i / N, n = i % N;
+        const int i = t + NT * j, m = i / N, n = i % N;
         rk[j] = i < MM * N ? p.kst[(((int64_t)b * MM + m) * p.H + h) * N + n] : 0.f;
     }
     float xv = 0.f, xo = 0.f, mxv[MM];
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     // the row's lane group), weight and bias, in registers
 #pragma unroll
     for (int j = 0; j < RK; ++j) {
-        const int i = t + 256 * j, m = i / N, n = i % N;
+        const int i = t + NT * j, m = i / N, n = i % N;
         if (i < MM * N) s_K[m][n] = rk[j];
     }
 #pragma unroll
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     }
     __syncthreads();
     // ---- new cache entries: K <- rotated B, v_state <- x (old ones are in LDS)
-    for (int i = t; i < MM * N; i += 256) {
+    for (int i = t; i < MM * N; i += NT) {
         const int m = i / N, n = i % N;
         p.kst[(((int64_t)b * MM + m) * p.H + h) * N + n] = s_B[m][n];
     }
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     }
     __syncthreads();
     // the rows' readout: SL partials per (row, rank), in order
-    for (int i = t; i < P * MM; i += 256) {
+    for (int i = t; i < P * MM; i += NT) {
         const int pr = i / MM, m = i % MM;
         float sum = 0.f;
 #pragma unroll
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     __syncthreads();
     // ---- gate (or per-head gated norm over P), MIMO merge
     if (p.onw) {
-        for (int m = wave; m < MM; m += 4) {
+        for (int m = wave; m < MM; m += NT / 64) {
             float ss = 0.f;
             for (int i = lane; i < P; i += 64) ss += s_out[m][i] * s_out[m][i];
             ss = wave_sum(ss);
@@ -310,14 +311,29 @@ __global__ __launch_bounds__(256) void mamba3_step_kernel(M3StepParams p) {
     }
 }
 
+// 512 threads per workgroup where the launch has at most one workgroup per CU
+// (two at rank 4): the CU has nothing else to hide the step's serial chain of
+// loads, norms and readout behind.  us per step at state 64 x 128, 256 against
+// 512 threads, by workgroups: rank 4, 32: 8.05 / 6.92, 256: 9.2 / 8.2, 512: 11.7 /
+// 11.0, 768: 14.5 / 16.6; rank 1, 32: 5.5 / 5.1, 256: 7.4 / 7.1, 384: 8.4 / 8.9;
+// rank 8, 32: 10.5 / 8.8, 256: 12.7 / 10.6, 384: 15.0 / 17.6.  (1024 threads: a
+// further 0.2 us below 256 workgroups up to rank 4, far slower above.)
+template <int N4, int MM>
+static void m3_launch_nt(const M3StepParams& p, hipStream_t s) {
+    const int grid = p.nb * p.H;
+    if (grid <= (MM == 4 ? 512 : 256))
+        hipLaunchKernelGGL((mamba3_step_kernel<N4, MM, 512>), dim3(grid), dim3(512), 0, s, p);
+    else
+        hipLaunchKernelGGL((mamba3_step_kernel<N4, MM, 256>), dim3(grid), dim3(256), 0, s, p);
+}
+
 template <int N4>
 static void m3_launch_m(const M3StepParams& p, hipStream_t s) {
-    const dim3 grid(p.nb * p.H), block(256);
     switch (p.M) {
-        case 1: hipLaunchKernelGGL((mamba3_step_kernel<N4, 1>), grid, block, 0, s, p); break;
-        case 2: hipLaunchKernelGGL((mamba3_step_kernel<N4, 2>), grid, block, 0, s, p); break;
-        case 4: hipLaunchKernelGGL((mamba3_step_kernel<N4, 4>), grid, block, 0, s, p); break;
-        default: hipLaunchKernelGGL((mamba3_step_kernel<N4, 8>), grid, block, 0, s, p); break;
+        case 1: m3_launch_nt<N4, 1>(p, s); break;
+        case 2: m3_launch_nt<N4, 2>(p, s); break;
+        case 4: m3_launch_nt<N4, 4>(p, s); break;
+        default: m3_launch_nt<N4, 8>(p, s); break;
     }
 }
 
