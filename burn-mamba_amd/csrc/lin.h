@@ -52,7 +52,12 @@ struct LinParams {
     // LIN_PARTIAL: part[z][m][n] = acc over k-split z (f32, planes of M x N);
     // the consumer sums the S planes in a fixed order
     float* part;
+    // one row (mamba_linear_row): the operand is RmsNorm(norm_x) * norm_w of this
+    // f32 row in place of A or X (K <= kLinRowMaxK); accumulate: out (f32) += ...
+    const float* norm_x; const float* norm_w;
+    bool accumulate;
 };
+constexpr int kLinRowMaxK = 4096;  // a normed row in LDS (8 KB) and 16 values of it per thread
 
 // k-splits for a product: enough workgroups (~1300 of 4 waves, ~10 weight
 // blocks per wave) to stream the weight at full HBM rate, fewer for large M

@@ -225,9 +225,17 @@ __global__ __launch_bounds__(64 * NW) void lin_stream(LinParams p) {
 // are zero), and the products accumulate in f32 on the VALU by packed bf16
 // dots (v_dot2c_f32_bf16: two products per instruction).  The two wave halves
 // (k 0..7 and 8..15 of each block) are summed at the end.
-template <int NW, int EPI, bool RM, int U, int MM>
+//
+// NORM (mamba_linear_row): the row is the f32 residual stream and the operand
+// its RmsNorm, formed by every workgroup for itself in LDS while its first
+// weight blocks are in flight; a norm launch in front of the product costs
+// more than the few KB read again.
+template <int NW, int EPI, bool RM, int U, int MM, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
+    static_assert(!NORM || (MM == 1 && RM), "one row");
     __shared__ float s_red[NW][MM][32];
+    __shared__ __align__(16) bf16_t s_x[NORM ? kLinRowMaxK : 8];
+    __shared__ float s_ss[NORM ? NW : 1];
     const int cs = lin_parts(p);
     const int j = blockIdx.x / cs, z = blockIdx.y;
     const int cw = 32 / cs, c0 = (blockIdx.x % cs) * cw;
@@ -252,8 +260,9 @@ __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
         for (int u = 0; u < U; ++u) {
             const bool ok = s + u < s1;
             st.w[u] = buf_ld16(rw, ok ? (uint32_t)(s + u) * 1024u + lo : kLinOut);
+            if constexpr (!NORM)
 #pragma unroll
-            for (int m = 0; m < MM; ++m) st.a[u][m] = buf_ld16(ra, ok && m < p.M ? aoff(m, s + u) : kLinOut);
+                for (int m = 0; m < MM; ++m) st.a[u][m] = buf_ld16(ra, ok && m < p.M ? aoff(m, s + u) : kLinOut);
         }
     };
     // four partial sums per row (k pairs e = 0..3 of each block), so that the
@@ -279,7 +288,63 @@ __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
         }
     };
     const int nstage = (s1 - s0 + U - 1) / U;
-    if (nstage > 0) {
+    // accumulate: the output's old value, in flight with the weights
+    float old = 0.f;
+    if (EPI == LIN_STORE && MM == 1 && p.accumulate) {
+        const int c = threadIdx.x;
+        if (c >= c0 && c < c0 + cw && 32 * j + c < p.N) old = static_cast<const float*>(p.out)[32 * j + c];
+    }
+    if constexpr (NORM) {
+        constexpr int NT = 64 * NW, V = kLinRowMaxK / 4 / NT;
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(p.norm_x, (uint32_t)p.K * 4u), rn = buf_rsrc(p.norm_w, (uint32_t)p.K * 4u);
+        float4 xv[V], nv[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) {  // past the row: zero
+            xv[i] = __builtin_bit_cast(float4, buf_ld16(rx, (threadIdx.x + NT * i) * 16u));
+            nv[i] = __builtin_bit_cast(float4, buf_ld16(rn, (threadIdx.x + NT * i) * 16u));
+        }
+        Stage sa, sb;
+        load(sa, s0);
+        load(sb, s0 + U);
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < V; ++i) ss += xv[i].x * xv[i].x + xv[i].y * xv[i].y + xv[i].z * xv[i].z + xv[i].w * xv[i].w;
+        ss = wave_sum_dpp(ss);
+        if (lane == 0) s_ss[wave] = ss;
+        __syncthreads();
+        ss = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) ss += s_ss[w];
+        const float rms = sqrtf(ss / (float)p.K + kDivEpsF32);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int c = 4 * (threadIdx.x + NT * i);
+            if (c < p.K)
+                *reinterpret_cast<uint2*>(s_x + c) =
+                    make_uint2((uint32_t)f32_to_bf16((xv[i].x / rms) * nv[i].x) |
+                                   ((uint32_t)f32_to_bf16((xv[i].y / rms) * nv[i].y) << 16),
+                               (uint32_t)f32_to_bf16((xv[i].z / rms) * nv[i].z) |
+                                   ((uint32_t)f32_to_bf16((xv[i].w / rms) * nv[i].w) << 16));
+        }
+        __syncthreads();
+        // k-steps past the wave's end meet zero weights: any k of the row will do
+        auto operand = [&](Stage& st, int s) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                st.a[u][0] = *reinterpret_cast<const uint4*>(s_x + 16 * min(s + u, KS - 1) + 8 * h);
+        };
+        for (int st = 0; st < nstage; st += 2) {
+            const int s = s0 + U * st;
+            operand(sa, s);
+            compute(sa);
+            if (st + 2 < nstage) load(sa, s + 2 * U);
+            if (st + 1 < nstage) {
+                operand(sb, s + U);
+                compute(sb);
+                if (st + 3 < nstage) load(sb, s + 3 * U);
+            }
+        }
+    } else if (nstage > 0) {
         Stage sa, sb;
         load(sa, s0);
         for (int st = 0; st < nstage; st += 2) {
@@ -311,7 +376,9 @@ __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
             for (int w = 0; w < NW; ++w) sum += s_red[w][m][c];
             if (EPI == LIN_STORE) {
                 if (p.bias) sum += p.bias[n];
-                if (p.out_bf16)
+                if (MM == 1 && p.accumulate)
+                    static_cast<float*>(p.out)[n] = old + sum;
+                else if (p.out_bf16)
                     static_cast<bf16_t*>(p.out)[(int64_t)m * p.out_ld + n] = f32_to_bf16(sum);
                 else
                     static_cast<float*>(p.out)[(int64_t)m * p.out_ld + n] = sum;
@@ -325,6 +392,12 @@ __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
 template <int NW, bool RM, int U, int MM>
 static void lin_launch_gemv(const LinParams& p, int epi, hipStream_t stream) {
     const dim3 grid(((p.N + 31) / 32) * lin_parts(p), p.S);
+    if constexpr (RM && MM == 1 && NW <= 8) {
+        if (p.norm_x) {
+            hipLaunchKernelGGL((lin_gemv<NW, LIN_STORE, true, U, 1, true>), grid, dim3(64 * NW), 0, stream, p);
+            return;
+        }
+    }
     if (epi == LIN_STORE) hipLaunchKernelGGL((lin_gemv<NW, LIN_STORE, RM, U, MM>), grid, dim3(64 * NW), 0, stream, p);
     else hipLaunchKernelGGL((lin_gemv<NW, LIN_PARTIAL, RM, U, MM>), grid, dim3(64 * NW), 0, stream, p);
 }
@@ -403,7 +476,7 @@ template <int MT>
 static void lin_launch_mt(const LinParams& p, int epi, hipStream_t stream) {
     constexpr int NWD = MT <= 2 ? MAMBA_LIN_NW : MAMBA_LIN_NW_BIGM;
     const int nw = p.NW ? p.NW : NWD;
-    const bool rm = p.X != nullptr;
+    const bool rm = p.X != nullptr || p.norm_x != nullptr;
     if constexpr (MT <= 2) {
         // 16 waves (1024 threads, at most 128 registers each) only for up to
         // two 32-row tiles, whose accumulators and operand stages fit
@@ -645,6 +718,41 @@ extern "C" int mamba_linear_fwd(const mamba_linear_args* a, void* ws, size_t ws_
     const int64_t nout = (int64_t)a->rows * a->d_out;
     hipLaunchKernelGGL(lin_reduce_kernel, dim3((int)std::min<int64_t>((nout + 255) / 256, 4096)), dim3(256), 0, s,
                        p.part, p.S, a->rows, a->d_out, a->bias, a->y, a->y_ld, a->y_dtype == MAMBA_BF16);
+    MAMBA_CHECK_LAUNCH();
+    return MAMBA_OK;
+}
+
+// One k-split always: the sum of planes would be a launch.  8 waves per column
+// tile, 4 where a CU has a tile of its own; weights not in the last-level cache, us
+// at 4 / 8 / 16 waves: normed 1024 x 5224 5.3 / 4.9 / 5.4, 2048 x 9576 10.4 / 11.6 /
+// 12.6 (norm and product apart 6.7, 15.6); 2048 x 1024 6.2 / 5.25 / 5.5, 4096 x
+// 2048 10.1 / 8.4 / 8.6 (8.6 in mamba_linear_fwd's plan).  Column parts gain at most 3 %.
+extern "C" int mamba_linear_row(const mamba_linear_row_args* a, mamba_stream_t stream) {
+    MAMBA_CHECK_ARG(a != nullptr, "args is NULL");
+    MAMBA_CHECK_ARG(a->d_in > 0 && a->d_in % 16 == 0 && a->d_in <= (1 << 20) && a->d_out > 0,
+                    "d_in must be a positive multiple of 16");
+    MAMBA_CHECK_ARG(a->x && a->packed_w && a->y, "x, packed_w and y are required");
+    MAMBA_CHECK_ARG(a->x_dtype == (a->norm_w ? MAMBA_F32 : MAMBA_BF16), "x must be f32 with norm_w, bf16 without");
+    MAMBA_CHECK_ARG(!a->norm_w || a->d_in <= kLinRowMaxK, "d_in must be at most 4096 with norm_w");
+    MAMBA_CHECK_ARG(a->y_dtype == MAMBA_F32 || (a->y_dtype == MAMBA_BF16 && !a->accumulate),
+                    "y must be f32 or bf16, f32 with accumulate");
+    MAMBA_CHECK_ARG(((uintptr_t)a->packed_w & 15u) == 0 && ((uintptr_t)a->x & 15u) == 0 &&
+                        ((uintptr_t)a->norm_w & 15u) == 0,
+                    "packed_w, x and norm_w must be 16-byte aligned");
+    LinParams p = {};
+    p.M = 1; p.N = a->d_out; p.K = a->d_in; p.MT = 1; p.S = 1;
+    p.NW = (a->d_out + 31) / 32 >= 256 ? 4 : 8;
+    p.W = static_cast<const lin_bf16x8_t*>(a->packed_w);
+    if (a->norm_w) {
+        p.norm_x = static_cast<const float*>(a->x);
+        p.norm_w = a->norm_w;
+    } else {
+        p.X = static_cast<const bf16_t*>(a->x);
+        p.x_ld = a->d_in;
+    }
+    p.bias = a->bias; p.out = a->y; p.out_ld = a->d_out; p.out_bf16 = a->y_dtype == MAMBA_BF16;
+    p.accumulate = a->accumulate != 0;
+    lin_launch(p, LIN_STORE, (hipStream_t)stream);
     MAMBA_CHECK_LAUNCH();
     return MAMBA_OK;
 }

@@ -270,6 +270,13 @@ class LinearArgs(ctypes.Structure):
     ]
 
 
+class LinearRowArgs(ctypes.Structure):
+    _fields_ = [
+        ("d_in", c_i32), ("d_out", c_i32), ("x_dtype", c_i32), ("y_dtype", c_i32),
+        ("x", c_vp), ("norm_w", c_vp), ("packed_w", c_vp), ("bias", c_vp), ("y", c_vp), ("accumulate", c_i32),
+    ]
+
+
 class MmF32Args(ctypes.Structure):
     _fields_ = [
         ("batch", c_i32), ("m", c_i32), ("n", c_i32), ("k", c_i32),
@@ -343,6 +350,7 @@ _SIGNATURES = {
     "mamba_linear_pack": ([c_vp, c_i32, c_i32, c_i64, c_i32, c_vp, c_vp], ctypes.c_int),
     "mamba_linear_workspace_size": ([ctypes.POINTER(LinearArgs)], ctypes.c_size_t),
     "mamba_linear_fwd": ([ctypes.POINTER(LinearArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
+    "mamba_linear_row": ([ctypes.POINTER(LinearRowArgs), c_vp], ctypes.c_int),
     "mamba_mm_f32": ([ctypes.POINTER(MmF32Args), c_vp], ctypes.c_int),
     "mamba2_layer_workspace_size": ([ctypes.POINTER(Mamba2LayerArgs)], ctypes.c_size_t),
     "mamba2_layer_step": ([ctypes.POINTER(Mamba2LayerArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),

@@ -584,9 +584,18 @@ class Mamba3Stack:
         return a
 
     def _run(self, x_res: torch.Tensor, caches, events, slot: int):
-        from .step import linear, rmsnorm
+        from .step import linear, linear_row, rmsnorm
         c = self.cfg
         bufs = self.buffers(x_res.shape[0], x_res.device, slot)
+        if x_res.shape[0] == 1 and c.d_model <= 4096 and \
+                all(t.data_ptr() % 16 == 0 for t in (x_res, *(l.norm_w for l in self.layers))):
+            # one row: the pre-norm inside in_proj, the residual add inside out_proj
+            for i, layer in enumerate(self.layers):
+                (pin, pout), (bin_, bout) = self._packed[i], self._bias[i]
+                linear_row(x_res, pin, bufs["proj"], norm_w=layer.norm_w, bias=bin_)
+                step_ssm(self._layer_args(i, slot, bufs, caches[i]), x_res.device, None if events is None else events[i])
+                linear_row(bufs["y"], pout, x_res, bias=bout, accumulate=True)
+            return x_res
         prev = None
         for i, layer in enumerate(self.layers):
             rmsnorm(x_res, layer.norm_w, out=bufs["normed"], add=prev)

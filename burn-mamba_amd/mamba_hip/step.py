@@ -226,6 +226,20 @@ def linear(x: torch.Tensor, packed_w: torch.Tensor, d_out: int, bias: Optional[t
     return out
 
 
+def linear_row(x: torch.Tensor, packed_w: torch.Tensor, out: torch.Tensor, norm_w: Optional[torch.Tensor] = None,
+               bias: Optional[torch.Tensor] = None, accumulate: bool = False) -> None:
+    """mamba_linear_row: out = x W (+ bias) for one row, x bf16, or f32 and
+    RMS-normed first (norm_w given); accumulate adds to an f32 out."""
+    a = _lib.LinearRowArgs()
+    a.d_in, a.d_out = x.numel(), out.numel()
+    a.x_dtype, a.y_dtype = _dtype_code(x), _dtype_code(out)
+    a.x, a.y, a.packed_w = x.data_ptr(), out.data_ptr(), packed_w.data_ptr()
+    a.norm_w = None if norm_w is None else norm_w.data_ptr()
+    a.bias = None if bias is None else bias.data_ptr()
+    a.accumulate = accumulate
+    check(_lib.lib().mamba_linear_row(ctypes.byref(a), _stream(x.device)), "mamba_linear_row")
+
+
 # every derived copy is kept on the weight under an attribute with this prefix
 _DERIVED_PREFIX = "_mamba_"
 

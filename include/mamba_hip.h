@@ -645,6 +645,25 @@ size_t mamba_linear_workspace_size(const mamba_linear_args* args);
 int mamba_linear_fwd(const mamba_linear_args* args, void* workspace, size_t workspace_bytes,
                      mamba_stream_t stream);
 
+/* The product for one row inside a pre-norm layer step (Layer::step_one,      */
+/* src/modules/layer.rs:224-232), without launches of their own for the norm   */
+/* and the residual: y = x W (+ bias), x a bf16 row, or with norm_w the        */
+/* RmsNorm (rms_norm.rs:53-98, rounded to bf16) of an f32 row of at most 4096; */
+/* accumulate: y (f32) += the product.  x, norm_w and packed_w are 16-byte     */
+/* aligned; y may not overlap x.                                               */
+typedef struct mamba_linear_row_args {
+    int32_t d_in, d_out;              /* d_in a multiple of 16                  */
+    int32_t x_dtype, y_dtype;         /* x: f32 with norm_w, bf16 without       */
+    const void* x;                    /* [d_in]                                 */
+    const float* norm_w;              /* [d_in] or NULL                         */
+    const void* packed_w;             /* mamba_linear_pack output               */
+    const float* bias;                /* [d_out] or NULL                        */
+    void* y;                          /* [d_out]                                */
+    int32_t accumulate;               /* y += ... (f32 y)                       */
+} mamba_linear_row_args;
+
+int mamba_linear_row(const mamba_linear_row_args* args, mamba_stream_t stream);
+
 /* Batched f32 products C[b] = A[b] B[b] for prefill blocks of few tokens, in  */
 /* any layout with one unit stride per operand (C's rows are contiguous): the  */
 /* Linears of Mamba1::forward (src/mamba1/mamba1.rs:278-399) formed time-major  */

@@ -633,6 +633,29 @@ impl Default for MambaLinearArgs {
 
 #[repr(C)]
 #[derive(Clone, Copy, Debug)]
+pub struct MambaLinearRowArgs {
+    pub d_in: i32,
+    pub d_out: i32,
+    pub x_dtype: i32,
+    pub y_dtype: i32,
+    pub x: *const c_void,
+    pub norm_w: *const f32,
+    pub packed_w: *const c_void,
+    pub bias: *const f32,
+    pub y: *mut c_void,
+    pub accumulate: i32,
+}
+
+impl Default for MambaLinearRowArgs {
+    /// Every size 0, every pointer null, every stride 0.
+    fn default() -> Self {
+        // SAFETY: all fields are integers, floats or raw pointers, for which zero is valid.
+        unsafe { core::mem::zeroed() }
+    }
+}
+
+#[repr(C)]
+#[derive(Clone, Copy, Debug)]
 pub struct MambaMmF32Args {
     pub batch: i32,
     pub m: i32,
@@ -834,6 +857,7 @@ extern "C" {
     pub fn mamba_linear_pack(weight: *const c_void, d_in: i32, d_out: i32, ld: i64, dtype: i32, packed: *mut c_void, stream: MambaStream) -> c_int;
     pub fn mamba_linear_workspace_size(args: *const MambaLinearArgs) -> usize;
     pub fn mamba_linear_fwd(args: *const MambaLinearArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
+    pub fn mamba_linear_row(args: *const MambaLinearRowArgs, stream: MambaStream) -> c_int;
     pub fn mamba_mm_f32(args: *const MambaMmF32Args, stream: MambaStream) -> c_int;
     pub fn mamba2_layer_workspace_size(args: *const Mamba2LayerArgs) -> usize;
     pub fn mamba2_layer_step(args: *const Mamba2LayerArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
