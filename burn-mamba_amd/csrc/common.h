@@ -225,6 +225,17 @@ __device__ __forceinline__ void dma16(u32x4_t rsrc, uint32_t lds, uint32_t voff,
         : "m0");
 }
 
+// The same with 4 bytes per lane, at LDS address lds + 4 * lane.
+__device__ __forceinline__ void dma4(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dword %1, %2, %3 offen lds"
+        :
+        : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff), "s"(rsrc), "s"(soff)
+        : "m0");
+}
+
 // two floats -> two bf16 (round to nearest even) in one dword, lo first
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));

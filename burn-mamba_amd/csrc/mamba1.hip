@@ -15,6 +15,7 @@
 // into registers before the current tile is computed); softplus, delta*u, D*u
 // and silu(z) are evaluated once per element in the staging pass.
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -34,6 +35,10 @@ struct Mamba1Params {
     const float* h0;
     float* y; int64_t y_sb, y_sd, y_sl;
     float* hT;
+    // time segments (mamba1_scan_tm16): seg_tiles tiles each; workspace planes of
+    // every segment's entry (0) or own end state [nseg][nb D][16] and sum of delta
+    int nseg, seg_tiles;
+    float* seg_h; float* seg_dl;
 };
 
 constexpr float kLog2eM1 = 1.4426950408889634f;
@@ -215,8 +220,7 @@ __global__ __launch_bounds__(16 * N, N <= 16 ? 3 : 1) void mamba1_scan_kernel(Ma
 }
 
 // ---------------------------------------------------------------------------
-// Time-major path for dstate 16 (u, delta, z and y contiguous along time, rows
-// 16-byte aligned): 64 channels x 32-token tiles, 4 lanes per channel holding 4
+// Time-major path for dstate 16 (u, delta, z and y contiguous along time): 64 channels x 32-token tiles, 4 lanes per channel holding 4
 // states each, as above.  A tile spans whole 128-byte lines of every row it
 // touches, so each line is read from HBM once (16-token tiles read half lines
 // and HBM fetched many lines twice) and y is written in whole lines.
@@ -235,9 +239,24 @@ __global__ __launch_bounds__(16 * N, N <= 16 ? 3 : 1) void mamba1_scan_kernel(Ma
 //    multiplies by silu(z) and stores.
 // Per tile one barrier, for the B/C tiles the waves share; everything else a
 // wave touches belongs to its own 16 channels.
+//
+// ALIGNED: rows start at multiples of 16 bytes.  Otherwise (odd lengths) the
+// direct-to-LDS loads take a word per lane instead of 16 bytes (16 instructions
+// per wave and tile instead of 4); 16-byte loads and stores of z and y need word
+// alignment only.  Against mamba1_scan_kernel, which such rows took before: 8 x
+// 5120 x 2047 758 -> 565 us (2048, aligned: 411), 1 x 1536 x 1001 160 -> 102 whole,
+// 24 in segments.
+//
+// Time segments, where (batch row, 64 channels) gives too few workgroups
+// (m1_segments): M1_STATE scans a segment from zero (the first from the initial
+// state) to its end state and sum of delta only; M1_OUT brings the entry state
+// forward over the segments before its own, h <- exp(A sum delta) h + end state,
+// and scans the segment.  The initial state is read by M1_STATE alone and handed
+// on through the workspace: final_state may be the same memory.
 constexpr int kTm16Tile = 32;
+enum M1Mode { M1_WHOLE, M1_STATE, M1_OUT };
 
-template <bool GATE>
+template <bool GATE, bool ALIGNED, int MODE>
 __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
     constexpr int N = 16, CPB = 64, TT = kTm16Tile, NQ = TT / 4;
     __shared__ __align__(16) float s_u[2][CPB][TT];  // u, then y + D u in place (swizzled pieces)
@@ -247,7 +266,9 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
 
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int nblk_d = (p.D + CPB - 1) / CPB;
-    const int b = blockIdx.x / nblk_d, d0 = (blockIdx.x % nblk_d) * CPB;
+    const int seg = MODE == M1_WHOLE ? 0 : blockIdx.x / (nblk_d * p.nb);
+    const int wg = blockIdx.x - seg * nblk_d * p.nb;
+    const int b = wg / nblk_d, d0 = (wg % nblk_d) * CPB;
     // scan mapping: channel c, states 4 ng .. 4 ng + 3
     const int c = tid >> 2, ng = tid & 3, d = d0 + c;
     const bool dvalid = d < p.D;
@@ -256,10 +277,28 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
     for (int k = 0; k < 4; ++k) {
         const int n = 4 * ng + k;
         A2[k] = dvalid ? p.A[(int64_t)d * p.A_sd + (int64_t)n * p.A_sn] * kLog2eM1 : 0.f;
-        h[k] = (dvalid && p.h0) ? p.h0[((int64_t)b * p.D + d) * N + n] : 0.f;
+        h[k] = (MODE != M1_OUT && seg == 0 && dvalid && p.h0) ? p.h0[((int64_t)b * p.D + d) * N + n] : 0.f;
     }
+    const int64_t seg_rows = (int64_t)p.nb * p.D, seg_row = (int64_t)b * p.D + d;
+    float4* const seg_h = reinterpret_cast<float4*>(p.seg_h);  // [nseg][row][4]
+    if (MODE == M1_STATE && seg == 0 && dvalid) seg_h[seg_row * 4 + ng] = make_float4(h[0], h[1], h[2], h[3]);
+    if (MODE == M1_OUT && dvalid) {
+        float4 e = seg_h[((seg ? seg_rows : 0) + seg_row) * 4 + ng];
+#pragma unroll 4
+        for (int j = 1; j < seg; ++j) {
+            const float4 q = seg_h[((int64_t)(j + 1) * seg_rows + seg_row) * 4 + ng];
+            const float dl = p.seg_dl[(int64_t)j * seg_rows + seg_row];
+            e.x = __builtin_fmaf(e.x, __builtin_amdgcn_exp2f(dl * A2[0]), q.x);
+            e.y = __builtin_fmaf(e.y, __builtin_amdgcn_exp2f(dl * A2[1]), q.y);
+            e.z = __builtin_fmaf(e.z, __builtin_amdgcn_exp2f(dl * A2[2]), q.z);
+            e.w = __builtin_fmaf(e.w, __builtin_amdgcn_exp2f(dl * A2[3]), q.w);
+        }
+        h[0] = e.x; h[1] = e.y; h[2] = e.z; h[3] = e.w;
+    }
+    float dl_sum = 0.f;
     const float Dd = (p.Dv && dvalid) ? p.Dv[d] : 0.f;
-    const int ntile = (p.L + TT - 1) / TT;
+    const int tk0 = MODE == M1_WHOLE ? 0 : seg * p.seg_tiles;
+    const int ntile = MODE == M1_WHOLE ? (p.L + TT - 1) / TT : min((p.L + TT - 1) / TT, tk0 + p.seg_tiles);
     // byte extents of the batch row's u / delta / z / y (u's strides for all);
     // lanes with nothing to move get an offset past the end (loads read zero,
     // stores are dropped)
@@ -283,6 +322,18 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
     // DMA mapping: wave w moves rows 16 w .. 16 w + 15 (its own channels) in
     // two instructions of 8 rows; lane i -> row + i / 8, slot i % 8
     auto dma_tile = [&](int tk, int buf) {
+        if (!ALIGNED) {
+            // 2 rows per instruction: lane i -> row + i / 32, word i % 32 of its slots
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int r0 = 16 * wave + 2 * k, r = r0 + (lane >> 5), w = lane & 31;
+                const int t = tk * TT + 4 * ((w >> 2) ^ (r & 7)) + (w & 3);
+                const uint32_t off = sel(d0 + r < p.D && t < p.L, ((uint32_t)(d0 + r) * sd + (uint32_t)t) * 4u);
+                dma4(ru, (uint32_t)(uintptr_t)&s_u[buf][r0][0], off, 0u);
+                dma4(rd, (uint32_t)(uintptr_t)&s_d[buf][r0][0], off, 0u);
+            }
+            return;
+        }
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int r0 = 16 * wave + 8 * k, r = r0 + (lane >> 3);
@@ -307,7 +358,8 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
         for (int e = 0; e < 2; ++e) {
             const int t = tk * TT + bt + e;
             rB[e] = buf_ld4(rb, sel(t < p.L, ((uint32_t)bn * (uint32_t)p.B_sn + (uint32_t)t * (uint32_t)p.B_sl) * 4u));
-            rC[e] = buf_ld4(rc, sel(t < p.L, ((uint32_t)bn * (uint32_t)p.C_sn + (uint32_t)t * (uint32_t)p.C_sl) * 4u));
+            if (MODE != M1_STATE)
+                rC[e] = buf_ld4(rc, sel(t < p.L, ((uint32_t)bn * (uint32_t)p.C_sn + (uint32_t)t * (uint32_t)p.C_sl) * 4u));
         }
     };
     // store mapping: thread -> channel tid / 4, tokens 8 (tid % 4) .. + 7
@@ -321,7 +373,7 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
         return sel(evalid && t < p.L, ((uint32_t)(d0 + ec) * sd + (uint32_t)t) * 4u);
     };
     auto load_z = [&](int tk) {
-        if (GATE) {
+        if (GATE && MODE != M1_STATE) {
 #pragma unroll
             for (int k = 0; k < 2; ++k) rzv[k] = buf_ld16(rz, eoff(tk, k));
         }
@@ -333,7 +385,7 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             s_B[buf][bt + e][bn] = rB[e];
-            s_C[buf][bt + e][bn] = rC[e];
+            if (MODE != M1_STATE) s_C[buf][bt + e][bn] = rC[e];
         }
         // this wave's direct-to-LDS loads of the tile: at most the previous
         // tile's two stores and this tile's two z loads were issued after them
@@ -346,8 +398,8 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
         // The count is exact only while no other vector-memory operation sits
         // between them: a register spill (scratch access) would break it, and
         // the build refuses a build of this kernel with scratch.
-        constexpr int kStoresPerTile = 2;          // the epilogue's two 16-byte stores
-        constexpr int kZLoadsPerTile = GATE ? 2 : 0;  // load_z
+        constexpr int kStoresPerTile = MODE == M1_STATE ? 0 : 2;  // the epilogue's two 16-byte stores
+        constexpr int kZLoadsPerTile = GATE && MODE != M1_STATE ? 2 : 0;  // load_z
         constexpr int kAfterDma = kStoresPerTile + kZLoadsPerTile;
         static_assert(kAfterDma < 16, "vmcnt immediate is 4 bits (low field)");
         // s_waitcnt: vmcnt in bits 3:0, expcnt(7) bits 6:4, lgkmcnt(15) bits 11:8
@@ -373,7 +425,7 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 bq[g] = *(const float4*)&s_B[buf][4 * q + g][4 * ng];
-                cq[g] = *(const float4*)&s_C[buf][4 * q + g][4 * ng];
+                if (MODE != M1_STATE) cq[g] = *(const float4*)&s_C[buf][4 * q + g][4 * ng];
             }
             float dv[4] = {dv4.x, dv4.y, dv4.z, dv4.w}, uv[4] = {uv4.x, uv4.y, uv4.z, uv4.w};
             if (partial) {
@@ -398,14 +450,17 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
                 h[1] = __builtin_fmaf(h[1], a1, du * bq[g].y);
                 h[2] = __builtin_fmaf(h[2], a2, du * bq[g].z);
                 h[3] = __builtin_fmaf(h[3], a3, du * bq[g].w);
-                yq[g] = __builtin_fmaf(cq[g].w, h[3], __builtin_fmaf(cq[g].z, h[2], __builtin_fmaf(cq[g].y, h[1], cq[g].x * h[0])));
+                if (MODE == M1_STATE) dl_sum += dv[g];
+                else yq[g] = __builtin_fmaf(cq[g].w, h[3], __builtin_fmaf(cq[g].z, h[2], __builtin_fmaf(cq[g].y, h[1], cq[g].x * h[0])));
             }
+            if (MODE == M1_STATE) continue;
 #pragma unroll
             for (int g = 0; g < 4; ++g) yq[g] = quad_sum(yq[g]);
             // every lane of the channel holds the sums: y + D u over u
             *(float4*)&s_u[buf][c][slot(c, q)] = make_float4(__builtin_fmaf(Dd, uv[0], yq[0]), __builtin_fmaf(Dd, uv[1], yq[1]),
                                                              __builtin_fmaf(Dd, uv[2], yq[2]), __builtin_fmaf(Dd, uv[3], yq[3]));
         }
+        if (MODE == M1_STATE) return;
         // ---- epilogue: y = (y + D u) silu(z), two 16-byte stores per thread
         // (the wave's own rows: its LDS accesses complete in program order)
 #pragma unroll
@@ -436,14 +491,21 @@ __global__ __launch_bounds__(256, 3) void mamba1_scan_tm16(Mamba1Params p) {
         load_z(tk + 1);
     };
 
-    load_bc(0);
-    dma_tile(0, 0);
-    load_z(0);
+    load_bc(tk0);
+    dma_tile(tk0, tk0 & 1);
+    load_z(tk0);
     __builtin_amdgcn_s_waitcnt(0);
-    const int nfull = p.L / TT;
-    for (int tk = 0; tk < nfull; ++tk) tile(tk, std::false_type{});
+    const int nfull = min(p.L / TT, ntile);
+    for (int tk = tk0; tk < nfull; ++tk) tile(tk, std::false_type{});
+    if (MODE == M1_STATE) {  // every segment but the last: whole tiles
+        if (dvalid) {
+            seg_h[((int64_t)(seg + 1) * seg_rows + seg_row) * 4 + ng] = make_float4(h[0], h[1], h[2], h[3]);
+            if (ng == 0) p.seg_dl[(int64_t)seg * seg_rows + seg_row] = dl_sum;
+        }
+        return;
+    }
     if (nfull < ntile) tile(nfull, std::true_type{});
-    if (dvalid && p.hT) {
+    if (dvalid && p.hT && (MODE == M1_WHOLE || seg == p.nseg - 1)) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) p.hT[((int64_t)b * p.D + d) * N + 4 * ng + k] = h[k];
     }
@@ -504,16 +566,52 @@ static int m1_make_params(const mamba1_scan_args* a, Mamba1Params* out) {
     return MAMBA_OK;
 }
 
-// the time-major tile path: dstate 16, time-contiguous rows at 16-byte
-// aligned addresses, byte offsets inside a batch row below 2^31
+// the time-major tile path: dstate 16, time-contiguous rows that do not
+// overlap, byte offsets inside a batch row below 2^31
 static bool tm16_ok(const Mamba1Params& p) {
-    auto al16 = [](const void* q) { return ((uintptr_t)q & 15u) == 0; };
-    return p.N == 16 && p.u_sl == 1 && p.u_sd % 4 == 0 && p.u_sd >= p.L && al16(p.u) && al16(p.dl) &&
-           al16(p.y) && (!p.z || al16(p.z)) && p.u_sb % 4 == 0 && p.dl_sb % 4 == 0 && p.y_sb % 4 == 0 &&
-           (!p.z || p.z_sb % 4 == 0) && (((int64_t)p.D - 1) * p.u_sd + p.L) * 4 < (1ll << 31) &&
+    return p.N == 16 && p.u_sl == 1 && p.u_sd >= p.L && (((int64_t)p.D - 1) * p.u_sd + p.L) * 4 < (1ll << 31) &&
            p.B_sn >= 0 && p.B_sl >= 0 && p.C_sn >= 0 && p.C_sl >= 0 &&
            ((int64_t)(p.N - 1) * p.B_sn + ((int64_t)p.L - 1) * p.B_sl + 1) * 4 < (1ll << 31) &&
            ((int64_t)(p.N - 1) * p.C_sn + ((int64_t)p.L - 1) * p.C_sl + 1) * 4 < (1ll << 31);
+}
+// ... every row at a 16-byte aligned address
+static bool tm16_aligned(const Mamba1Params& p) {
+    auto al16 = [](const void* q) { return ((uintptr_t)q & 15u) == 0; };
+    return p.u_sd % 4 == 0 && al16(p.u) && al16(p.dl) && al16(p.y) && (!p.z || al16(p.z)) && p.u_sb % 4 == 0 &&
+           p.dl_sb % 4 == 0 && p.y_sb % 4 == 0 && (!p.z || p.z_sb % 4 == 0);
+}
+
+// Time segments: none where (batch row, 64 channels) already gives a workgroup to
+// most CUs, else about 1280 workgroups (five per CU, three resident: the state pass
+// is half of the second one's work, and its chain is short), at least a tile each.
+// us whole / so split: 24 workgroups, 256 tokens 25.6 / 12.0, 2048 184 / 32; 40,
+// 1504: 136 / 38; 80, 2048: 185 / 77; 160, 2048: 180 / 146; 200, 2048: 180 / 185;
+// 320, 1024: 145 / 138; 480, 1024: 154 / 195.
+static int m1_segments(const Mamba1Params& p) {
+    const int tiles = (p.L + kTm16Tile - 1) / kTm16Tile;
+    const int64_t nblk = (int64_t)p.nb * ((p.D + 63) / 64);
+    return nblk > 160 ? 1 : (int)std::min<int64_t>(tiles, 1280 / nblk);
+}
+// workspace bytes of one segment
+static size_t m1_seg_bytes(const Mamba1Params& p) { return (size_t)p.nb * p.D * (16 + 1) * 4; }
+
+template <bool GATE, bool ALIGNED>
+static void launch_tm16(Mamba1Params& p, void* ws, size_t ws_bytes, hipStream_t s) {
+    const int nblk = p.nb * ((p.D + 63) / 64), tiles = (p.L + kTm16Tile - 1) / kTm16Tile;
+    int nseg = m1_segments(p);
+    if (nseg > 1) nseg = (int)std::min<size_t>(nseg, ws ? ws_bytes / m1_seg_bytes(p) : 0);
+    if (nseg > 1) {
+        p.seg_tiles = (tiles + nseg - 1) / nseg;
+        p.nseg = (tiles + p.seg_tiles - 1) / p.seg_tiles;
+    }
+    if (nseg <= 1 || p.nseg <= 1) {
+        hipLaunchKernelGGL((mamba1_scan_tm16<GATE, ALIGNED, M1_WHOLE>), dim3(nblk), dim3(256), 0, s, p);
+        return;
+    }
+    p.seg_h = static_cast<float*>(ws);
+    p.seg_dl = p.seg_h + (size_t)p.nseg * p.nb * p.D * 16;
+    hipLaunchKernelGGL((mamba1_scan_tm16<false, ALIGNED, M1_STATE>), dim3(nblk * (p.nseg - 1)), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((mamba1_scan_tm16<GATE, ALIGNED, M1_OUT>), dim3(nblk * p.nseg), dim3(256), 0, s, p);
 }
 
 template <int N>
@@ -526,21 +624,24 @@ static void launch_m1(const Mamba1Params& p, hipStream_t stream) {
         hipLaunchKernelGGL((mamba1_scan_kernel<N, false>), dim3(nblk), dim3(16 * N), 0, stream, p);
 }
 
-static int m1_dispatch(const mamba1_scan_args* a, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+static bool m1_tiled(const Mamba1Params& p) {
+    const bool same_strides = p.dl_sd == p.u_sd && p.dl_sl == p.u_sl && p.y_sd == p.u_sd &&
+                              p.y_sl == p.u_sl && (!p.z || (p.z_sd == p.u_sd && p.z_sl == p.u_sl));
+    return same_strides && (int64_t)p.D * std::abs(p.u_sd) + (int64_t)p.L * std::abs(p.u_sl) < (1ll << 31);
+}
+
+static int m1_dispatch(const mamba1_scan_args* a, void* ws, size_t ws_bytes, hipStream_t stream, hipEvent_t ev0,
+                       hipEvent_t ev1) {
     Mamba1Params p;
     int st = m1_make_params(a, &p);
     if (st != MAMBA_OK) return st;
-    const bool same_strides = p.dl_sd == p.u_sd && p.dl_sl == p.u_sl && p.y_sd == p.u_sd &&
-                              p.y_sl == p.u_sl && (!p.z || (p.z_sd == p.u_sd && p.z_sl == p.u_sl));
-    const bool fits32 = (int64_t)p.D * std::abs(p.u_sd) + (int64_t)p.L * std::abs(p.u_sl) < (1ll << 31);
-    int nfast = (same_strides && fits32) ? p.N : 0;
+    MAMBA_CHECK_ARG(((uintptr_t)ws & 15u) == 0, "the workspace must be 16-byte aligned");
+    int nfast = m1_tiled(p) ? p.N : 0;
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
     if (nfast == 16 && tm16_ok(p)) {
-        const int nblk = p.nb * ((p.D + 63) / 64);
-        if (p.z)
-            hipLaunchKernelGGL((mamba1_scan_tm16<true>), dim3(nblk), dim3(256), 0, stream, p);
-        else
-            hipLaunchKernelGGL((mamba1_scan_tm16<false>), dim3(nblk), dim3(256), 0, stream, p);
+        const bool al = tm16_aligned(p);
+        if (p.z) al ? launch_tm16<true, true>(p, ws, ws_bytes, stream) : launch_tm16<true, false>(p, ws, ws_bytes, stream);
+        else al ? launch_tm16<false, true>(p, ws, ws_bytes, stream) : launch_tm16<false, false>(p, ws, ws_bytes, stream);
         nfast = -1;
     }
     switch (nfast) {
@@ -562,8 +663,20 @@ static int m1_dispatch(const mamba1_scan_args* a, hipStream_t stream, hipEvent_t
 
 using namespace mamba;
 
+extern "C" size_t mamba1_scan_workspace_size(const mamba1_scan_args* a) {
+    Mamba1Params p;
+    if (m1_make_params(a, &p) != MAMBA_OK || !m1_tiled(p) || !tm16_ok(p)) return 0;
+    const int nseg = m1_segments(p);
+    return nseg > 1 ? nseg * m1_seg_bytes(p) : 0;
+}
+
+extern "C" int mamba1_scan_fwd_ws(const mamba1_scan_args* a, void* ws, size_t ws_bytes, mamba_stream_t stream,
+                                  void* ev_start, void* ev_stop) {
+    return m1_dispatch(a, ws, ws_bytes, (hipStream_t)stream, (hipEvent_t)ev_start, (hipEvent_t)ev_stop);
+}
+
 extern "C" int mamba1_scan_fwd(const mamba1_scan_args* a, mamba_stream_t stream) {
-    return m1_dispatch(a, (hipStream_t)stream, nullptr, nullptr);
+    return m1_dispatch(a, nullptr, 0, (hipStream_t)stream, nullptr, nullptr);
 }
 
 extern "C" int mamba1_scan_fwd_timed(const mamba1_scan_args* a, mamba_stream_t stream, void* ev_start,
@@ -572,5 +685,5 @@ extern "C" int mamba1_scan_fwd_timed(const mamba1_scan_args* a, mamba_stream_t s
         set_error("mamba1_scan_fwd_timed: both events are required");
         return MAMBA_ERR_INVALID_ARG;
     }
-    return m1_dispatch(a, (hipStream_t)stream, (hipEvent_t)ev_start, (hipEvent_t)ev_stop);
+    return m1_dispatch(a, nullptr, 0, (hipStream_t)stream, (hipEvent_t)ev_start, (hipEvent_t)ev_stop);
 }

@@ -326,6 +326,8 @@ _SIGNATURES = {
     "mamba_ssd3_double_fwd_generic": ([ctypes.POINTER(Ssd3DoubleArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
     "mamba1_scan_fwd": ([ctypes.POINTER(Mamba1ScanArgs), c_vp], ctypes.c_int),
     "mamba1_scan_fwd_timed": ([ctypes.POINTER(Mamba1ScanArgs), c_vp, c_vp, c_vp], ctypes.c_int),
+    "mamba1_scan_workspace_size": ([ctypes.POINTER(Mamba1ScanArgs)], ctypes.c_size_t),
+    "mamba1_scan_fwd_ws": ([ctypes.POINTER(Mamba1ScanArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp], ctypes.c_int),
     "mamba1_scan_step": ([ctypes.POINTER(Mamba1StepArgs), c_vp], ctypes.c_int),
     "mamba3_step_ssm": ([ctypes.POINTER(Mamba3StepArgs), c_vp], ctypes.c_int),
     "mamba2_conv_fwd": ([ctypes.POINTER(Mamba2ConvArgs), c_vp], ctypes.c_int),

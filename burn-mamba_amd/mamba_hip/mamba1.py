@@ -65,12 +65,11 @@ def mamba1_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta_softpl
     a.y = y.data_ptr(); a.y_sb, a.y_sd, a.y_sl = y.stride()
     a.final_state = final_state.data_ptr()
     L = _lib.lib()
-    st = _stream(u.device)
-    if events is not None:
-        e0, e1 = _raw_events(events, u.device)
-        check(L.mamba1_scan_fwd_timed(ctypes.byref(a), st, e0, e1), "mamba1_scan_fwd_timed")
-    else:
-        check(L.mamba1_scan_fwd(ctypes.byref(a), st), "mamba1_scan_fwd")
+    e0, e1 = _raw_events(events, u.device) if events is not None else (None, None)
+    need = L.mamba1_scan_workspace_size(ctypes.byref(a))
+    ws = torch.empty(need, dtype=torch.uint8, device=u.device) if need else None
+    check(L.mamba1_scan_fwd_ws(ctypes.byref(a), None if ws is None else ctypes.c_void_p(ws.data_ptr()), need,
+                               _stream(u.device), e0, e1), "mamba1_scan_fwd")
     return y, final_state
 
 

@@ -337,6 +337,13 @@ typedef struct mamba1_scan_args {
 } mamba1_scan_args;
 
 int mamba1_scan_fwd(const mamba1_scan_args* args, mamba_stream_t stream);
+/* The same with a 16-byte aligned workspace, in which a scan of few channels   */
+/* is split into time segments that run side by side.  mamba1_scan_workspace_size */
+/* gives the bytes for the best split (0 where none pays); with less the split  */
+/* is coarser, with none it is mamba1_scan_fwd.  The events may be NULL (both). */
+size_t mamba1_scan_workspace_size(const mamba1_scan_args* args);
+int mamba1_scan_fwd_ws(const mamba1_scan_args* args, void* workspace, size_t workspace_bytes, mamba_stream_t stream,
+                       void* event_start, void* event_stop);
 /* As mamba1_scan_fwd, recording the caller's HIP events around the scan      */
 /* kernel (benchmark timing; no counterpart in the reference).                */
 int mamba1_scan_fwd_timed(const mamba1_scan_args* args, mamba_stream_t stream, void* event_start,

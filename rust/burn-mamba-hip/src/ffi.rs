@@ -836,6 +836,8 @@ extern "C" {
     pub fn mamba_ssd3_bwd(args: *const MambaSsd3BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
     pub fn mamba_ssd3_bwd_timed(args: *const MambaSsd3BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
     pub fn mamba1_scan_fwd(args: *const Mamba1ScanArgs, stream: MambaStream) -> c_int;
+    pub fn mamba1_scan_workspace_size(args: *const Mamba1ScanArgs) -> usize;
+    pub fn mamba1_scan_fwd_ws(args: *const Mamba1ScanArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
     pub fn mamba1_scan_fwd_timed(args: *const Mamba1ScanArgs, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
     pub fn mamba1_scan_step(args: *const Mamba1StepArgs, stream: MambaStream) -> c_int;
     pub fn mamba1_scan_step_timed(args: *const Mamba1StepArgs, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
