@@ -9,8 +9,8 @@
 // products stay with the library, which reaches 154 TFLOP/s.
 //
 // Tilings: 64 x 64 (a 32 x 32 tile per wave of four, 32 of K per step), and, where
-// those would give fewer workgroups than CUs, 32 x 32 with 4 or 16 waves sharing
-// K (128 or 512 per step), their tiles summed through LDS at the end in a fixed
+// those would give fewer workgroups than CUs, 32 x 32 with 4, 8 or 16 waves sharing
+// K (128, 256 or 512 per step), their tiles summed through LDS at the end in a fixed
 // order.  Bound by launch and one load latency per step in the small; a lone
 // tile's MFMAs take 1.7 us per 512 of K.
 #include "bwd_core.h"
@@ -188,13 +188,15 @@ static int mm_run(MmParams p, hipStream_t s) {
 }
 
 // 64 x 64 tiles where they give every CU a workgroup; else 32 x 32 with K over 4
-// waves, or over 16 where K is long and the tiles are still few (one per CU: a
-// step's load latency, about 2 us, is paid K / 512 times instead of K / 128).
+// waves, or over 8 or 16 where K is long and the tiles are still few (a step's load
+// latency, about 2 us, is paid K / 256 or K / 512 times instead of K / 128; 512 x
+// 512 of K = 256: 7.1 us with 16 waves, half of them idle, 5.3 with 8).
 template <bool AK, bool BK>
 static int mm_launch(const MmParams& p, hipStream_t s) {
     auto tiles = [&](int w) { return (int64_t)p.Z * ((p.M + w - 1) / w) * ((p.N + w - 1) / w); };
     if (tiles(64) >= 256) return mm_run<AK, BK, 1>(p, s);
-    return p.K >= 256 && tiles(32) <= 512 ? mm_run<AK, BK, 16>(p, s) : mm_run<AK, BK, 4>(p, s);
+    if (p.K <= 128 || tiles(32) > 512) return mm_run<AK, BK, 4>(p, s);
+    return p.K <= 256 ? mm_run<AK, BK, 8>(p, s) : mm_run<AK, BK, 16>(p, s);
 }
 
 }  // namespace mamba

@@ -271,12 +271,15 @@ def mm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None)
 
 
 def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
-    """Where mamba_mm_f32 takes a block's x_proj and out_proj.  For at most 256
+    """Where mamba_mm_f32 takes a block's products.  For at most 256
     tokens per sequence and 512 channels the library picks 256-wide tiles (2 x 256
     tokens, 512 channels: out_proj 118 us, x_proj 25 us against 7.9 and 7.5; 1 x
     100: 62 and 28 against 7.3 and 7.5; 1 x 7: 12 and 6.8 against 7.5 and 6.4);
     past either bound it is the faster one (1 x 301: 6.8 against 9.0; 768 channels
-    and more: 8.6 against 11.8).  Calls that autograd follows, and operands
+    and more: 8.6 against 11.8).  dt_proj (K = dt_rank) takes the same time in either
+    (3.7 to 5 us) and in_proj up to 512 tokens in all (2 x 256: 5.2 against 5.2 and
+    5.8; 3 x 256: 7.2 against 6.7 and 5.7), for 9 us less of the host per call, which
+    is what bounds a block of this size.  Calls that autograd follows, and operands
     without a unit stride, stay with the library."""
     return L <= 256 and di <= 512 and all(1 in t.stride()[-2:] and t.dtype == torch.float32 for t in ts) and \
         not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
@@ -329,26 +332,31 @@ class Mamba1:
         di, r, n = c.d_inner, c.dt_rank, c.state_rank
         xf = x.float()
         x2 = xf.reshape(b * L, dm)
+        own = _mm_f32_pays(di, L, self.in_proj_w, self.x_proj_w, self.dt_proj_w, self.out_proj_w, xf)
         # The scan streams u, delta, z and y as time-contiguous rows [b, d, l]
         # (its tuned kernel reads 32-token tiles of whole 128-byte lines), so
         # the products around it are formed in that layout: z and delta as
         # W^T x^T per batch row, y consumed through its transposed view.
         # layer 1, in_proj: the conv half channels-last [b, l, d_inner], the
         # gate half z time-major [b, d_inner, l]
-        xs = torch.mm(x2, self.in_proj_w[:, :di]).view(b, L, di)
-        zt = torch.matmul(_wt(self.in_proj_w, "_mamba_t_res", di), xf.transpose(1, 2))
+        if own and b * L <= 512:
+            xs = mm_f32(x2[None], self.in_proj_w[None, :, :di]).view(b, L, di)
+            zt = mm_f32(self.in_proj_w[:, di:].t().expand(b, -1, -1), xf.transpose(1, 2))
+        else:
+            xs = torch.mm(x2, self.in_proj_w[:, :di]).view(b, L, di)
+            zt = torch.matmul(_wt(self.in_proj_w, "_mamba_t_res", di), xf.transpose(1, 2))
         # layer 2: causal conv over [cached window | xs] + SiLU; window updated
         u = conv1d_fwd(xs, cache.conv_bik, self.conv_w, self.conv_b)
         # ssm (mamba1.rs:366-399): x_proj, dt_proj (its bias and the softplus go
         # to the scan), then the selective scan with D u and the silu(res) gate
         # (x_proj and dt_proj time-major too: B and C then stream as whole rows)
         ut = u.transpose(1, 2).contiguous()
-        own = _mm_f32_pays(di, L, self.x_proj_w, self.out_proj_w, u)
         if own:  # reads u where the conv wrote it
-            x_dbl = mm_f32(self.x_proj_w.t().expand(b, -1, -1), u.transpose(1, 2))
+            x_dbl = mm_f32(self.x_proj_w.t().expand(b, -1, -1), u.transpose(1, 2))        # [b, r + 2n, l]
+            dt = mm_f32(self.dt_proj_w.t().expand(b, -1, -1), x_dbl[:, :r])               # [b, d_inner, l]
         else:
-            x_dbl = torch.matmul(_wt(self.x_proj_w, "_mamba_t", 0), ut)      # [b, r + 2n, l]
-        dt = torch.matmul(_wt(self.dt_proj_w, "_mamba_t", 0), x_dbl[:, :r])  # [b, d_inner, l]
+            x_dbl = torch.matmul(_wt(self.x_proj_w, "_mamba_t", 0), ut)
+            dt = torch.matmul(_wt(self.dt_proj_w, "_mamba_t", 0), x_dbl[:, :r])
         yt = torch.empty((b, di, L), device=x.device, dtype=torch.float32)
         # the scan reads a channel's initial state before it writes its final one
         mamba1_scan(ut, dt, self.A, x_dbl[:, r:r + n], x_dbl[:, r + n:],
