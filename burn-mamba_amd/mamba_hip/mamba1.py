@@ -281,8 +281,16 @@ def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
     5.8; 3 x 256: 7.2 against 6.7 and 5.7), for 9 us less of the host per call, which
     is what bounds a block of this size.  Calls that autograd follows, and operands
     without a unit stride, stay with the library."""
-    return L <= 256 and di <= 512 and all(1 in t.stride()[-2:] and t.dtype == torch.float32 for t in ts) and \
-        not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+    return L <= 256 and di <= 512 and _mm_f32_takes(*ts)
+
+
+def _mm_f32_takes(*ts: torch.Tensor) -> bool:
+    """Plain f32 tensors with a unit stride that no transform of the product's
+    operands (reverse or forward mode, vmap) has to see."""
+    return all(t.dtype == torch.float32 and 1 in t.stride()[-2:] and type(t) in (torch.Tensor, torch.nn.Parameter)
+               and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts) and \
+        not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)) and \
+        torch.autograd.forward_ad._current_level < 0
 
 
 def _wt(w: torch.Tensor, attr: str, col0: int) -> torch.Tensor:

@@ -25,7 +25,7 @@ import torch
 from . import _lib
 from ._lib import Mamba3FinishArgs, Mamba3FusedArgs, Mamba3PrepArgs, Mamba3StepArgs, check
 from .ssd import _dtype_code, _raw_events, _stream
-from .step import packed_weight, prefill_mm, prefill_mm_rows, step_mm, step_mm_ok
+from .step import out_mm, packed_weight, prefill_mm_rows, step_mm, step_mm_ok
 
 
 @dataclass
@@ -378,7 +378,7 @@ class Mamba3:
 
     def _out_proj(self, y: torch.Tensor, x: torch.Tensor):
         b, L, _ = y.shape
-        out = prefill_mm(y.reshape(b * L, -1), self.out_proj_w).reshape(b, L, -1)
+        out = out_mm(y.reshape(b * L, -1), self.out_proj_w).reshape(b, L, -1)
         if self.out_proj_b is not None:
             out = out + self.out_proj_b.to(self.in_proj_w.dtype)
         return out.to(x.dtype)

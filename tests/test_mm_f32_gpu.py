@@ -39,3 +39,27 @@ def test_mm_f32_refuses_operands_without_a_unit_stride():
     a, b = torch.zeros(1, 4, 8, device="cuda")[:, ::2, ::2], torch.zeros(1, 4, 4, device="cuda")
     with pytest.raises(mamba_hip.MambaHipError):
         mm_f32(a, b)
+
+
+# both sides of the rows, channels and columns at which the block's out_proj moves
+@pytest.mark.parametrize("rows,di,dm", [(1, 512, 256), (256, 512, 256), (257, 512, 256), (64, 528, 256), (64, 512, 264)])
+def test_out_mm_on_both_sides_of_its_rule(rows, di, dm):
+    import torch
+    from mamba_hip.step import out_mm
+    g = torch.Generator().manual_seed(rows + di)
+    y, w = torch.randn(rows, di, generator=g), torch.randn(di, dm, generator=g)
+    out = out_mm(y.cuda(), w.cuda())
+    np.testing.assert_allclose(out.cpu().numpy(), (y.double() @ w.double()).numpy(), rtol=1e-4, atol=1e-5 * di ** 0.5)
+
+
+def test_out_mm_under_autograd_and_forward_mode():
+    import torch
+    import torch.autograd.forward_ad as fw
+    from mamba_hip.step import out_mm
+    y, w, t = torch.randn(8, 64, device="cuda"), torch.randn(64, 32, device="cuda"), torch.randn(64, 32, device="cuda")
+    with fw.dual_level():
+        tangent = fw.unpack_dual(out_mm(y, fw.make_dual(w, t))).tangent
+    torch.testing.assert_close(tangent, y @ t, rtol=1e-4, atol=1e-4)
+    w.requires_grad_()
+    out_mm(y, w).sum().backward()
+    torch.testing.assert_close(w.grad, y.sum(0)[:, None].expand(64, 32), rtol=1e-4, atol=1e-4)
