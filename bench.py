@@ -995,7 +995,7 @@ def bench_ssd2_bwd(args):
     tflops = flops / (kern_ms * 1e-3) / 1e12
     roof = {"bound": "mfma", "achieved": tflops, "peak": F32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": tflops / F32_MFMA_PEAK_TFLOPS, "traffic": _profiled_traffic("mamba2_ssd_bwd_cfg1"),
-            "kernel_ms": kern_ms, "algorithmic_flops": flops, "kernel": "ssd2_bwd_chunks (reverse chunk loop)",
+            "kernel_ms": kern_ms, "algorithmic_flops": flops, "kernel": "ssd_f32_bwd_chunks (reverse chunk loop)",
             "timing": "HIP events around the reverse chunk-loop kernel on its stream, per call",
             "call_tflops": (flops + state_flops) / (ms_per_step * 1e-3) / 1e12,
             "call_compulsory_bytes": nbytes}
@@ -1075,10 +1075,10 @@ def bench_ssd3_bwd(args):
     tflops = flops / (kern_ms * 1e-3) / 1e12
     roof = {"bound": "mfma", "achieved": tflops, "peak": F32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": tflops / F32_MFMA_PEAK_TFLOPS, "traffic": _profiled_traffic("mamba3_ssd_bwd_cfg4"),
-            "kernel_ms": kern_ms, "algorithmic_flops": flops, "kernel": "ssd3_bwd_chunks (reverse chunk loop)",
+            "kernel_ms": kern_ms, "algorithmic_flops": flops, "kernel": "ssd_f32_bwd_chunks (reverse chunk loop)",
             "timing": "HIP events around the reverse chunk-loop kernel on its stream, per call",
             "call_tflops": (flops + state_flops) / (ms_per_step * 1e-3) / 1e12,
-            "grid": f"{cfg['batch'] * cfg['nheads']} workgroups (one per batch row and head) on 256 CUs"}
+            "grid": f"{cfg['batch'] * cfg['nheads']} (batch row, head) pairs x sequence segments on 256 CUs"}
     return {
         "metric": "Mamba-3 SSD backward tokens/s (B=4 L=8192 H=32 P=64 N=128 MIMO 4, f32) + % f32 MFMA roofline",
         "value": tokens / (ms_per_step * 1e-3), "unit": "tokens/s",
