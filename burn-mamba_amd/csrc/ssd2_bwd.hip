@@ -329,8 +329,9 @@ struct BwdLayout {
 
 // The call for the segment-parallel MFMA kernels: one rank, with sc = gm = dt
 // and the log-decay dt A.  False where they do not apply within `limit` bytes.
-static bool bwd_f32_params(const mamba_ssd2_bwd_args* a, size_t limit, SsdF32BwdParams* out) {
+static bool bwd_f32_params(const mamba_ssd2_bwd_args* a, bool bf16, size_t limit, SsdF32BwdParams* out) {
     SsdF32BwdParams f{};
+    f.bf16 = bf16;
     f.nb = a->batch; f.L = a->seqlen; f.M = 1; f.H = a->nheads; f.P = a->headdim; f.G = a->ngroups; f.N = a->dstate;
     f.v = a->x; f.v_sb = a->x_sb; f.v_sl = a->x_sl; f.v_sh = a->x_sh;
     f.da = a->dt; f.da_sb = a->dt_sb; f.da_sl = a->dt_sl; f.da_sh = a->dt_sh;
@@ -380,10 +381,10 @@ extern "C" size_t mamba_ssd2_bwd_workspace_size(const mamba_ssd2_bwd_args* a) {
     BwdLayout lay;
     if (bwd_validate(a, &lay) != MAMBA_OK) return 0;
     SsdF32BwdParams f;
-    return bwd_f32_params(a, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : lay.total;
+    return bwd_f32_params(a, false, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : lay.total;
 }
 
-static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, void* workspace, size_t workspace_bytes,
+static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, bool bf16, void* workspace, size_t workspace_bytes,
                         mamba_stream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
     BwdLayout lay;
     const int st = bwd_validate(a, &lay);
@@ -419,10 +420,13 @@ static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, void* workspace, size_t wo
     const dim3 grid(a->batch * a->nheads);
     p.npart = 1;
     SsdF32BwdParams f;
-    if (bwd_f32_params(a, workspace_bytes, &f)) {
+    if (bwd_f32_params(a, bf16, workspace_bytes, &f)) {
         const int fst = ssd_f32_bwd_launch(f, workspace, s, ev0, ev1);
         if (fst != MAMBA_OK) return fst;
         p.dBh = f.dBh; p.dCh = f.dCh; p.pA = f.pA; p.pD = f.pD; p.npart = f.S;
+    } else if (bf16) {
+        set_error("mamba_ssd2_bwd_bf16: these shapes, layouts or this workspace are not covered (use mamba_ssd2_bwd on f32)");
+        return MAMBA_ERR_UNSUPPORTED;
     } else {
         // dynamic LDS above the 64 KB default (up to the CU's 160 KB)
         MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd2_bwd_states, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -445,10 +449,22 @@ static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, void* workspace, size_t wo
 
 extern "C" int mamba_ssd2_bwd(const mamba_ssd2_bwd_args* a, void* workspace, size_t workspace_bytes,
                               mamba_stream_t stream) {
-    return ssd2_bwd_run(a, workspace, workspace_bytes, stream, nullptr, nullptr);
+    return ssd2_bwd_run(a, false, workspace, workspace_bytes, stream, nullptr, nullptr);
 }
 
 extern "C" int mamba_ssd2_bwd_timed(const mamba_ssd2_bwd_args* a, void* workspace, size_t workspace_bytes,
                                     mamba_stream_t stream, void* event_start, void* event_stop) {
-    return ssd2_bwd_run(a, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
+    return ssd2_bwd_run(a, false, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
+}
+
+extern "C" size_t mamba_ssd2_bwd_bf16_workspace_size(const mamba_ssd2_bwd_args* a) {
+    BwdLayout lay;
+    if (bwd_validate(a, &lay) != MAMBA_OK) return 0;
+    SsdF32BwdParams f;
+    return bwd_f32_params(a, true, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : 0;
+}
+
+extern "C" int mamba_ssd2_bwd_bf16(const mamba_ssd2_bwd_args* a, void* workspace, size_t workspace_bytes,
+                                  mamba_stream_t stream, void* event_start, void* event_stop) {
+    return ssd2_bwd_run(a, true, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
 }

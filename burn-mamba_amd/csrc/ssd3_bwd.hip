@@ -325,8 +325,9 @@ static size_t b3_chunks_lds(int P, int N) {
 
 // The call for the segment-parallel MFMA kernels.  False where they do not
 // apply within `limit` bytes.
-static bool b3_f32_params(const mamba_ssd3_bwd_args* a, size_t limit, SsdF32BwdParams* out) {
+static bool b3_f32_params(const mamba_ssd3_bwd_args* a, bool bf16, size_t limit, SsdF32BwdParams* out) {
     SsdF32BwdParams f{};
+    f.bf16 = bf16;
     f.nb = a->batch; f.L = a->seqlen; f.M = a->mimo; f.H = a->nheads; f.P = a->headdim; f.G = a->ngroups;
     f.N = a->dstate;
     f.v = a->v; f.v_sb = a->v_sb; f.v_sl = a->v_sl; f.v_sm = a->v_sm; f.v_sh = a->v_sh;
@@ -374,7 +375,7 @@ static int b3_validate(const mamba_ssd3_bwd_args* a, B3Layout* lay) {
     return MAMBA_OK;
 }
 
-static int ssd3_bwd_run(const mamba_ssd3_bwd_args* a, void* workspace, size_t workspace_bytes, mamba_stream_t stream,
+static int ssd3_bwd_run(const mamba_ssd3_bwd_args* a, bool bf16, void* workspace, size_t workspace_bytes, mamba_stream_t stream,
                         hipEvent_t ev0, hipEvent_t ev1) {
     B3Layout lay;
     const int st = b3_validate(a, &lay);
@@ -409,11 +410,14 @@ static int ssd3_bwd_run(const mamba_ssd3_bwd_args* a, void* workspace, size_t wo
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid(a->batch * a->nheads);
     SsdF32BwdParams f;
-    if (b3_f32_params(a, workspace_bytes, &f)) {
+    if (b3_f32_params(a, bf16, workspace_bytes, &f)) {
         const int fst = ssd_f32_bwd_launch(f, workspace, s, ev0, ev1);
         if (fst != MAMBA_OK) return fst;
         p.dBh = f.dBh;
         p.dCh = f.dCh;
+    } else if (bf16) {
+        set_error("mamba_ssd3_bwd_bf16: these shapes, layouts or this workspace are not covered (use mamba_ssd3_bwd on f32)");
+        return MAMBA_ERR_UNSUPPORTED;
     } else {
         MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd3_bwd_states, hipFuncAttributeMaxDynamicSharedMemorySize,
                                             (int)b3_states_lds(p.P, p.N)));
@@ -443,15 +447,27 @@ extern "C" size_t mamba_ssd3_bwd_workspace_size(const mamba_ssd3_bwd_args* a) {
     B3Layout lay;
     if (b3_validate(a, &lay) != MAMBA_OK) return 0;
     SsdF32BwdParams f;
-    return b3_f32_params(a, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : lay.total;
+    return b3_f32_params(a, false, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : lay.total;
 }
 
 extern "C" int mamba_ssd3_bwd(const mamba_ssd3_bwd_args* a, void* workspace, size_t workspace_bytes,
                               mamba_stream_t stream) {
-    return ssd3_bwd_run(a, workspace, workspace_bytes, stream, nullptr, nullptr);
+    return ssd3_bwd_run(a, false, workspace, workspace_bytes, stream, nullptr, nullptr);
 }
 
 extern "C" int mamba_ssd3_bwd_timed(const mamba_ssd3_bwd_args* a, void* workspace, size_t workspace_bytes,
                                     mamba_stream_t stream, void* event_start, void* event_stop) {
-    return ssd3_bwd_run(a, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
+    return ssd3_bwd_run(a, false, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
+}
+
+extern "C" size_t mamba_ssd3_bwd_bf16_workspace_size(const mamba_ssd3_bwd_args* a) {
+    B3Layout lay;
+    if (b3_validate(a, &lay) != MAMBA_OK) return 0;
+    SsdF32BwdParams f;
+    return b3_f32_params(a, true, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : 0;
+}
+
+extern "C" int mamba_ssd3_bwd_bf16(const mamba_ssd3_bwd_args* a, void* workspace, size_t workspace_bytes,
+                                  mamba_stream_t stream, void* event_start, void* event_stop) {
+    return ssd3_bwd_run(a, true, workspace, workspace_bytes, stream, (hipEvent_t)event_start, (hipEvent_t)event_stop);
 }

@@ -9,18 +9,19 @@ namespace mamba {
 struct SsdF32BwdParams {
     int nb, L, M, mshift, H, P, G, N;  // L counts steps; M = 1 << mshift ranks per step
     int nch, S, cps;                   // chunks of 64 fused rows, segments, chunks per segment
-    const float* v; int64_t v_sb, v_sl, v_sm, v_sh;
+    bool bf16;                         // v, B, C and dy are bf16 (f32 otherwise)
+    const void* v; int64_t v_sb, v_sl, v_sm, v_sh;
     // log-decay per step: da (A == NULL), or dt with A[h] (Mamba-2)
     const float* da; int64_t da_sb, da_sl, da_sh;
     const float* A;
     // source weights of earlier steps (sc) and of the row's own step (gm); NULL: 1
     const float* gm; int64_t gm_sb, gm_sl, gm_sh;
     const float* sc; int64_t sc_sb, sc_sl, sc_sh;
-    const float* B; int64_t B_sb, B_sl, B_sm, B_sg;
-    const float* C; int64_t C_sb, C_sl, C_sm, C_sg;
+    const void* B; int64_t B_sb, B_sl, B_sm, B_sg;
+    const void* C; int64_t C_sb, C_sl, C_sm, C_sg;
     const float* D;        // dv += D[h] dy (Mamba-2), or NULL
     const float* h0;       // [b, h, p, n] or NULL
-    const float* dy; int64_t dy_sb, dy_sl, dy_sm, dy_sh;
+    const void* dy; int64_t dy_sb, dy_sl, dy_sm, dy_sh;
     const float* dfin;     // [b, h, p, n] or NULL
     float* dv;             // [b, l, m, h, p]
     float* dda;            // [b, l, h]: d(da), or with A the whole d(dt)

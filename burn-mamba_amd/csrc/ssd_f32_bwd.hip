@@ -1,5 +1,5 @@
 // SSD backward with every product on f32 MFMA, split over sequence segments:
-// headdim 64, dstate 64 or 128, f32 throughout.
+// headdim 64, dstate 64 or 128, f32 arithmetic, f32 or bf16 inputs.
 //
 // Reference: the Autodiff arms of Mamba2BackendExt::ssd_serial_recalculated
 // (src/mamba2/ssd/serial_recalculated/backward.rs:29-321, gradient math
@@ -48,6 +48,10 @@
 // 32-row chunks, which it replaces; at 2 x 2048, 80 heads, rank 1, 0.98 -> 0.82
 // ms; and at dstate 64 (1 x 1024, 24 heads), where the SIMT kernels ran, 7.6 ms
 // -> 0.08 ms.
+// T: bf16 rows are widened on their way into LDS (the same values as an f32 copy,
+// half the bytes of three passes, and no spills in the reverse loop): a bf16
+// forward and backward at 2 x 2048, 80 heads, rank 1 943 -> 873 us with the four
+// conversion launches gone.
 #include <algorithm>
 #include <type_traits>
 
@@ -175,7 +179,7 @@ struct FBSegLds {
 // One workgroup per (batch, head, segment, direction): blocks of direction 0
 // form the state of segments 0 .. S - 2 from zero, those of direction 1 the
 // state gradient entering (from the right) segments 1 .. S - 1.
-template <int N>
+template <int N, typename T>
 __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
     __shared__ __align__(16) FBSegLds<N> S;
     constexpr int TILES = 2 * (N / 32), QT = TILES / 4, NT = 256;
@@ -183,26 +187,26 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
     const bool rev = blockIdx.x & 1;
     const int idx = blockIdx.x >> 1, u = idx / (p.S - 1), s0 = idx % (p.S - 1);
     const FBJob j = fb_job(p, u, rev ? s0 + 1 : s0);
-    const float* xb = rev ? p.dy + (int64_t)j.b * p.dy_sb + (int64_t)j.h * p.dy_sh
-                          : p.v + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
-    const float* rb = rev ? p.C + (int64_t)j.b * p.C_sb + (int64_t)j.grp * p.C_sg
-                          : p.B + (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg;
+    const T* xb = static_cast<const T*>(rev ? p.dy : p.v) +
+                  (rev ? (int64_t)j.b * p.dy_sb + (int64_t)j.h * p.dy_sh : (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh);
+    const T* rb = static_cast<const T*>(rev ? p.C : p.B) +
+                  (rev ? (int64_t)j.b * p.C_sb + (int64_t)j.grp * p.C_sg : (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg);
     const int64_t xsl = rev ? p.dy_sl : p.v_sl, xsm = rev ? p.dy_sm : p.v_sm;
     const int64_t rsl = rev ? p.C_sl : p.B_sl, rsm = rev ? p.C_sm : p.B_sm;
     const float A = p.A ? p.A[j.h] : 1.f;
-    FRaw<float> rr[kFR * N / 4 / NT], rx[kFR * kBP / 4 / NT];
+    FRaw<T> rr[kFR * N / 4 / NT], rx[kFR * kBP / 4 / NT];
     FBTab rt = {0.f, 0.f, 0.f};
     bwd_f32x16 acc[QT];
 #pragma unroll
     for (int q = 0; q < QT; ++q) acc[q] = fb_zero();
     auto fetch = [&](int c) {
-        f_fetch<float, N, NT>(rr, rb, rsl, rsm, p.L, p.mshift, c, tid);
-        f_fetch<float, kBP, NT>(rx, xb, xsl, xsm, p.L, p.mshift, c, tid);
+        f_fetch<T, N, NT>(rr, rb, rsl, rsm, p.L, p.mshift, c, tid);
+        f_fetch<T, kBP, NT>(rx, xb, xsl, xsm, p.L, p.mshift, c, tid);
         if (wv == 0) rt = fb_tab(p, j, c, lane);
     };
     auto commit = [&](int c) {
-        f_commit<float, N, NT, N + 4>(rr, S.R, p.L, p.mshift, c, tid);
-        f_commit<float, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
+        f_commit<T, N, NT, N + 4>(rr, S.R, p.L, p.mshift, c, tid);
+        f_commit<T, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
         if (wv == 0) {
             const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64);
             S.w[lane] = rev ? __expf(cs) : __expf(end - cs) * rt.sc;
@@ -239,26 +243,26 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
 
 // The chunk-entry states of one segment, as [p][n] tiles (pt + 2 nt) in
 // accumulator order: hs[(b h, chunk)][tile][r][lane].
-template <int N>
+template <int N, typename T>
 __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_states(SsdF32BwdParams p) {
     __shared__ __align__(16) FBSegLds<N> S;
     constexpr int TILES = 2 * (N / 32), QT = TILES / 4, NT = 256, NP = N + 4;
     const int tid = threadIdx.x, wv = wave_id(), lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
     const FBJob j = fb_job(p, blockIdx.x / p.S, blockIdx.x % p.S);
-    const float* vb = p.v + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
-    const float* Bb = p.B + (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg;
+    const T* vb = static_cast<const T*>(p.v) + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
+    const T* Bb = static_cast<const T*>(p.B) + (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg;
     const float A = p.A ? p.A[j.h] : 1.f;
-    FRaw<float> rr[kFR * N / 4 / NT], rx[kFR * kBP / 4 / NT];
+    FRaw<T> rr[kFR * N / 4 / NT], rx[kFR * kBP / 4 / NT];
     FBTab rt = {0.f, 0.f, 0.f};
     bwd_f32x16 acc[QT];
     auto fetch = [&](int c) {
-        f_fetch<float, N, NT>(rr, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
-        f_fetch<float, kBP, NT>(rx, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
+        f_fetch<T, N, NT>(rr, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
+        f_fetch<T, kBP, NT>(rx, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
         if (wv == 0) rt = fb_tab(p, j, c, lane);
     };
     auto commit = [&](int c) {
-        f_commit<float, N, NT, NP>(rr, S.R, p.L, p.mshift, c, tid);
-        f_commit<float, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
+        f_commit<T, N, NT, NP>(rr, S.R, p.L, p.mshift, c, tid);
+        f_commit<T, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
         if (wv == 0) {
             const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64);
             S.w[lane] = __expf(end - cs) * rt.sc;
@@ -325,7 +329,7 @@ struct FBLds {
     float dec;
 };
 
-template <int N>
+template <int N, typename T>
 __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) {
     extern __shared__ __align__(16) char fb_smem[];
     FBLds<N>& S = *reinterpret_cast<FBLds<N>*>(fb_smem);
@@ -333,31 +337,31 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
     constexpr int XT = N == 128 ? 2 : 1;  // row tiles of dB and dC per wave
     const int tid = threadIdx.x, wv = wave_id(), lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
     const FBJob j = fb_job(p, blockIdx.x / p.S, blockIdx.x % p.S);
-    const float* vb = p.v + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
-    const float* yb = p.dy + (int64_t)j.b * p.dy_sb + (int64_t)j.h * p.dy_sh;
-    const float* Bb = p.B + (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg;
-    const float* Cb = p.C + (int64_t)j.b * p.C_sb + (int64_t)j.grp * p.C_sg;
+    const T* vb = static_cast<const T*>(p.v) + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
+    const T* yb = static_cast<const T*>(p.dy) + (int64_t)j.b * p.dy_sb + (int64_t)j.h * p.dy_sh;
+    const T* Bb = static_cast<const T*>(p.B) + (int64_t)j.b * p.B_sb + (int64_t)j.grp * p.B_sg;
+    const T* Cb = static_cast<const T*>(p.C) + (int64_t)j.b * p.C_sb + (int64_t)j.grp * p.C_sg;
     const float A = p.A ? p.A[j.h] : 1.f;
     const float D = p.D ? p.D[j.h] : 0.f;
     const int ms = p.mshift, steps = kFR >> ms;
     const int pt = wv & 1;                                  // waves 0, 1, 6, 7
     const int nt = N == 128 ? wv - 2 : (wv - 2) & 1;        // waves 2-5
     const int own = N == 128 ? 0 : (wv - 2) >> 1;
-    FRaw<float> rB[kFR * N / 4 / NT], rC[kFR * N / 4 / NT], rv[kFR * kBP / 4 / NT], ry[kFR * kBP / 4 / NT];
+    FRaw<T> rB[kFR * N / 4 / NT], rC[kFR * N / 4 / NT], rv[kFR * kBP / 4 / NT], ry[kFR * kBP / 4 / NT];
     FBTab rt = {0.f, 0.f, 0.f};
     auto fetch = [&](int c, int tid) {
-        f_fetch<float, N, NT>(rB, Bb, p.B_sl, p.B_sm, p.L, ms, c, tid);
-        f_fetch<float, N, NT>(rC, Cb, p.C_sl, p.C_sm, p.L, ms, c, tid);
-        f_fetch<float, kBP, NT>(rv, vb, p.v_sl, p.v_sm, p.L, ms, c, tid);
-        f_fetch<float, kBP, NT>(ry, yb, p.dy_sl, p.dy_sm, p.L, ms, c, tid);
+        f_fetch<T, N, NT>(rB, Bb, p.B_sl, p.B_sm, p.L, ms, c, tid);
+        f_fetch<T, N, NT>(rC, Cb, p.C_sl, p.C_sm, p.L, ms, c, tid);
+        f_fetch<T, kBP, NT>(rv, vb, p.v_sl, p.v_sm, p.L, ms, c, tid);
+        f_fetch<T, kBP, NT>(ry, yb, p.dy_sl, p.dy_sm, p.L, ms, c, tid);
         if (wv == 1) rt = fb_tab(p, j, c, tid & 63);
     };
     auto commit = [&](int c, int tid) {
         const int lane = tid & 63;
-        f_commit<float, N, NT, NP>(rB, S.B, p.L, ms, c, tid);
-        f_commit<float, N, NT, NP>(rC, S.C, p.L, ms, c, tid);
-        f_commit<float, kBP, NT, kBVP>(rv, S.V, p.L, ms, c, tid);
-        f_commit<float, kBP, NT, kBVP>(ry, S.Y, p.L, ms, c, tid);
+        f_commit<T, N, NT, NP>(rB, S.B, p.L, ms, c, tid);
+        f_commit<T, N, NT, NP>(rC, S.C, p.L, ms, c, tid);
+        f_commit<T, kBP, NT, kBVP>(rv, S.V, p.L, ms, c, tid);
+        f_commit<T, kBP, NT, kBVP>(ry, S.Y, p.L, ms, c, tid);
         if (wv == 1) {
             const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64), a = __expf(end - cs);
             S.cs[lane] = cs;
@@ -742,8 +746,8 @@ bool ssd_f32_bwd_plan(SsdF32BwdParams* q, size_t limit) {
     if (p.P != kBP || (p.N != 64 && p.N != 128)) return false;
     // a step's ranks lie in one 32-row tile: its own-step block is on the diagonal
     if (p.M < 1 || p.M > 32 || (p.M & (p.M - 1)) != 0) return false;
-    for (const float* ptr : {p.v, p.B, p.C, p.dy})
-        if (((uintptr_t)ptr & 15u) != 0) return false;
+    for (const void* ptr : {p.v, p.B, p.C, p.dy})  // four values per load
+        if (((uintptr_t)ptr & (p.bf16 ? 7u : 15u)) != 0) return false;
     p.vec = true;
     for (const float* ptr : {p.dv, p.dBh, p.dCh, p.dh0})
         if (((uintptr_t)ptr & 15u) != 0) p.vec = false;
@@ -776,22 +780,22 @@ bool ssd_f32_bwd_plan(SsdF32BwdParams* q, size_t limit) {
     return best > 0. && units * p.S * 2 < (1ll << 31);
 }
 
-template <int N>
+template <int N, typename T>
 static int fb_run(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
     const int units = p.nb * p.H;
     // dynamic LDS above the 64 KB default (up to the CU's 160 KB)
     constexpr size_t lds = sizeof(FBLds<N>);
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N, T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)lds));
     if (p.S > 1) {
-        hipLaunchKernelGGL((ssd_f32_bwd_seg<N>), dim3(units * (p.S - 1) * 2), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((ssd_f32_bwd_seg<N, T>), dim3(units * (p.S - 1) * 2), dim3(256), 0, stream, p);
         MAMBA_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL((ssd_f32_bwd_states<N>), dim3(units * p.S), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((ssd_f32_bwd_states<N, T>), dim3(units * p.S), dim3(256), 0, stream, p);
     MAMBA_CHECK_LAUNCH();
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
-    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N>), dim3(units * p.S), dim3(512), lds, stream, p);
+    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N, T>), dim3(units * p.S), dim3(512), lds, stream, p);
     MAMBA_CHECK_LAUNCH();
     if (ev1) MAMBA_CHECK_HIP(hipEventRecord(ev1, stream));
     return MAMBA_OK;
@@ -821,7 +825,9 @@ int ssd_f32_bwd_launch(SsdF32BwdParams& p, void* ws, hipStream_t stream, hipEven
         p.pA = take(units * p.S * sizeof(float));
         p.pD = take(units * p.S * sizeof(float));
     }
-    return p.N == 128 ? fb_run<128>(p, stream, ev0, ev1) : fb_run<64>(p, stream, ev0, ev1);
+    if (p.bf16)
+        return p.N == 128 ? fb_run<128, bf16_t>(p, stream, ev0, ev1) : fb_run<64, bf16_t>(p, stream, ev0, ev1);
+    return p.N == 128 ? fb_run<128, float>(p, stream, ev0, ev1) : fb_run<64, float>(p, stream, ev0, ev1);
 }
 
 }  // namespace mamba

@@ -311,9 +311,13 @@ _SIGNATURES = {
                              ctypes.c_int),
     "mamba_ssd2_bwd_workspace_size": ([ctypes.POINTER(Ssd2BwdArgs)], ctypes.c_size_t),
     "mamba_ssd2_bwd": ([ctypes.POINTER(Ssd2BwdArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
+    "mamba_ssd2_bwd_bf16_workspace_size": ([ctypes.POINTER(Ssd2BwdArgs)], ctypes.c_size_t),
+    "mamba_ssd2_bwd_bf16": ([ctypes.POINTER(Ssd2BwdArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp], ctypes.c_int),
     "mamba_ssd2_bwd_timed": ([ctypes.POINTER(Ssd2BwdArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp], ctypes.c_int),
     "mamba_ssd3_bwd_workspace_size": ([ctypes.POINTER(Ssd3BwdArgs)], ctypes.c_size_t),
     "mamba_ssd3_bwd": ([ctypes.POINTER(Ssd3BwdArgs), c_vp, ctypes.c_size_t, c_vp], ctypes.c_int),
+    "mamba_ssd3_bwd_bf16_workspace_size": ([ctypes.POINTER(Ssd3BwdArgs)], ctypes.c_size_t),
+    "mamba_ssd3_bwd_bf16": ([ctypes.POINTER(Ssd3BwdArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp], ctypes.c_int),
     "mamba_ssd3_bwd_timed": ([ctypes.POINTER(Ssd3BwdArgs), c_vp, ctypes.c_size_t, c_vp, c_vp, c_vp], ctypes.c_int),
     "mamba_ssd3_workspace_size": ([ctypes.POINTER(Ssd3Args)], ctypes.c_size_t),
     "mamba_ssd3_fast_path": ([ctypes.POINTER(Ssd3Args)], ctypes.c_int),

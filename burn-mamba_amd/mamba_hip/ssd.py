@@ -138,17 +138,20 @@ def ssd2_bwd(dy, x, dt, A, B, C, D=None, initial_state=None, d_final_state=None,
     """The SSD forward's gradients through ``mamba_ssd2_bwd``: the Autodiff arm
     of Mamba2BackendExt::ssd_serial_recalculated
     (src/mamba2/ssd/serial_recalculated/backward.rs:29-321; gradient math
-    combined_backward.rs:126-593).  Inputs as ``ssd2_fwd`` (bf16 ones are read
-    as f32), dy[b,l,h,p], d_final_state[b,h,p,n] or None.  Returns a dict of f32
-    gradients: dx[b,l,h,p], ddt[b,l,h], dA[h], dB / dC[b,l,g,n] (summed over
+    combined_backward.rs:126-593).  Inputs as ``ssd2_fwd`` (the arithmetic is
+    f32 for bf16 ones too), dy[b,l,h,p], d_final_state[b,h,p,n] or None.
+    Returns a dict of f32 gradients: dx[b,l,h,p], ddt[b,l,h], dA[h], dB / dC[b,l,g,n] (summed over
     each group's heads), dD[h] (None without D), d_initial_state[b,h,p,n].
     events: optional (start, stop) torch events recorded around the reverse
     chunk-loop kernel (mamba_ssd2_bwd_timed)."""
     b, l, h, p = x.shape
     g, n = B.shape[2], B.shape[3]
     f = lambda t: None if t is None else (t if t.dtype == torch.float32 else t.float())  # noqa: E731
-    x, dy, B, C, dt, A, D, initial_state, d_final_state = map(f, (x, dy, B, C, dt, A, D, initial_state,
-                                                                d_final_state))
+    dt, A, D, initial_state, d_final_state = map(f, (dt, A, D, initial_state, d_final_state))
+    # bf16 rows are read in place where the kernels cover them
+    bf16 = all(t.dtype == torch.bfloat16 and t.stride(-1) == 1 for t in (x, dy, B, C))
+    if not bf16:
+        x, dy, B, C = map(f, (x, dy, B, C))
     for t, nm in ((x, "x"), (B, "B"), (C, "C"), (dy, "dy")):
         _check_inner(t, nm)
     for t in (A, D, initial_state, d_final_state):
@@ -174,6 +177,15 @@ def ssd2_bwd(dy, x, dt, A, B, C, D=None, initial_state=None, d_final_state=None,
         setattr(a, k, None if out[k] is None else out[k].data_ptr())
     a.d_initial_state = out["d_initial_state"].data_ptr()
     L = _lib.lib()
+    if bf16:
+        nbytes = L.mamba_ssd2_bwd_bf16_workspace_size(ctypes.byref(a))
+        if nbytes == 0:
+            return ssd2_bwd(dy.float(), x.float(), dt, A, B.float(), C.float(), D, initial_state, d_final_state, events)
+        ws = workspace(dev, nbytes)
+        e0, e1 = _raw_events(events, dev) if events is not None else (None, None)
+        check(L.mamba_ssd2_bwd_bf16(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(dev), e0, e1),
+              "mamba_ssd2_bwd_bf16")
+        return out
     nbytes = L.mamba_ssd2_bwd_workspace_size(ctypes.byref(a))
     if nbytes == 0:
         check(L.mamba_ssd2_bwd(ctypes.byref(a), None, 0, _stream(dev)), "mamba_ssd2_bwd")

@@ -185,7 +185,7 @@ def ssd3_bwd(dy, v, da, B, C, gamma=None, scale=None, initial_state=None, d_fina
     (src/mamba3/single_ssd/ssd/serial_recalculated/backward.rs:27-299; gradient
     math combined_backward.rs:74-536).  gamma = scale = None is the double-SSD
     seam's backward (double_ssd/ssd/serial_recalculated/backward.rs:27-275).
-    Inputs as ``ssd3_fwd`` (bf16 ones are read as f32), dy [b, l, m, h, p],
+    Inputs as ``ssd3_fwd`` (the arithmetic is f32 for bf16 ones too), dy [b, l, m, h, p],
     d_final_state [b, h, p, n] or None.  Returns a dict of f32 gradients: dv,
     dda, dgamma / dscale (None without the weights), dB / dC [b, l, m, g, n]
     (summed over each group's heads), d_initial_state [b, h, p, n].  events:
@@ -193,8 +193,11 @@ def ssd3_bwd(dy, v, da, B, C, gamma=None, scale=None, initial_state=None, d_fina
     b, l, m, h, p = v.shape
     g, n = B.shape[3], B.shape[4]
     f = lambda t: None if t is None else (t if t.dtype == torch.float32 else t.float())  # noqa: E731
-    v, dy, B, C, da, gamma, scale, initial_state, d_final_state = map(
-        f, (v, dy, B, C, da, gamma, scale, initial_state, d_final_state))
+    da, gamma, scale, initial_state, d_final_state = map(f, (da, gamma, scale, initial_state, d_final_state))
+    # bf16 rows are read in place where the kernels cover them
+    bf16 = all(t.dtype == torch.bfloat16 and t.stride(-1) == 1 for t in (v, dy, B, C))
+    if not bf16:
+        v, dy, B, C = map(f, (v, dy, B, C))
     if B.shape != C.shape or B.shape[:3] != (b, l, m) or dy.shape != v.shape:
         raise _lib.MambaHipError("B and C must be [b, l, m, g, n] and dy [b, l, m, h, p] matching v")
     for t, nm in ((v, "v"), (B, "B"), (C, "C"), (dy, "dy")):
@@ -228,6 +231,16 @@ def ssd3_bwd(dy, v, da, B, C, gamma=None, scale=None, initial_state=None, d_fina
     for k in ("dv", "dda", "dgamma", "dscale", "dB", "dC", "d_initial_state"):
         setattr(a, k, None if out[k] is None else out[k].data_ptr())
     L = _lib.lib()
+    if bf16:
+        need = L.mamba_ssd3_bwd_bf16_workspace_size(ctypes.byref(a))
+        if need == 0:
+            return ssd3_bwd(dy.float(), v.float(), da, B.float(), C.float(), gamma, scale, initial_state, d_final_state,
+                            events)
+        ws = workspace(dev, need)
+        e0, e1 = _raw_events(events, dev) if events is not None else (None, None)
+        check(L.mamba_ssd3_bwd_bf16(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(dev), e0, e1),
+              "mamba_ssd3_bwd_bf16")
+        return out
     need = L.mamba_ssd3_bwd_workspace_size(ctypes.byref(a))
     st = _stream(dev)
     if need == 0:

@@ -177,6 +177,13 @@ int mamba_ssd2_bwd(const mamba_ssd2_bwd_args* args, void* workspace, size_t work
 /* dominant kernel (the reverse chunk loop).  No counterpart in the reference. */
 int mamba_ssd2_bwd_timed(const mamba_ssd2_bwd_args* args, void* workspace, size_t workspace_bytes,
                          mamba_stream_t stream, void* event_start, void* event_stop);
+/* The same with bf16 x, B, C and dy behind their pointers (strides in elements; */
+/* the gradients stay f32), read without an f32 copy.  Covers headdim 64, dstate */
+/* 64 or 128, 8-byte aligned rows; the workspace size is 0 elsewhere.  The events */
+/* may be NULL (both).                                                         */
+size_t mamba_ssd2_bwd_bf16_workspace_size(const mamba_ssd2_bwd_args* args);
+int mamba_ssd2_bwd_bf16(const mamba_ssd2_bwd_args* args, void* workspace, size_t workspace_bytes,
+                       mamba_stream_t stream, void* event_start, void* event_stop);
 
 /* ------------------------------------------------------------------------- */
 /* Mamba-3 single-pass chunked SSD forward (trapezoidal discretisation, MIMO   */
@@ -302,6 +309,13 @@ int mamba_ssd3_bwd(const mamba_ssd3_bwd_args* args, void* workspace, size_t work
 /* dominant kernel (the reverse chunk loop).  No counterpart in the reference. */
 int mamba_ssd3_bwd_timed(const mamba_ssd3_bwd_args* args, void* workspace, size_t workspace_bytes,
                          mamba_stream_t stream, void* event_start, void* event_stop);
+/* The same with bf16 v, B, C and dy behind their pointers (strides in elements; */
+/* the gradients stay f32), read without an f32 copy.  Covers headdim 64, dstate */
+/* 64 or 128, 8-byte aligned rows; the workspace size is 0 elsewhere.  The events */
+/* may be NULL (both).                                                         */
+size_t mamba_ssd3_bwd_bf16_workspace_size(const mamba_ssd3_bwd_args* args);
+int mamba_ssd3_bwd_bf16(const mamba_ssd3_bwd_args* args, void* workspace, size_t workspace_bytes,
+                       mamba_stream_t stream, void* event_start, void* event_stop);
 
 /* ------------------------------------------------------------------------- */
 /* Mamba-1 selective scan (f32), with the optional dt bias + softplus of       */

@@ -823,6 +823,8 @@ extern "C" {
     pub fn mamba_ssd2_bwd_workspace_size(args: *const MambaSsd2BwdArgs) -> usize;
     pub fn mamba_ssd2_bwd(args: *const MambaSsd2BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
     pub fn mamba_ssd2_bwd_timed(args: *const MambaSsd2BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
+    pub fn mamba_ssd2_bwd_bf16_workspace_size(args: *const MambaSsd2BwdArgs) -> usize;
+    pub fn mamba_ssd2_bwd_bf16(args: *const MambaSsd2BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
     pub fn mamba_ssd3_workspace_size(args: *const MambaSsd3Args) -> usize;
     pub fn mamba_ssd3_fast_path(args: *const MambaSsd3Args) -> c_int;
     pub fn mamba_ssd3_fwd(args: *const MambaSsd3Args, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
@@ -835,6 +837,8 @@ extern "C" {
     pub fn mamba_ssd3_bwd_workspace_size(args: *const MambaSsd3BwdArgs) -> usize;
     pub fn mamba_ssd3_bwd(args: *const MambaSsd3BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream) -> c_int;
     pub fn mamba_ssd3_bwd_timed(args: *const MambaSsd3BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
+    pub fn mamba_ssd3_bwd_bf16_workspace_size(args: *const MambaSsd3BwdArgs) -> usize;
+    pub fn mamba_ssd3_bwd_bf16(args: *const MambaSsd3BwdArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
     pub fn mamba1_scan_fwd(args: *const Mamba1ScanArgs, stream: MambaStream) -> c_int;
     pub fn mamba1_scan_workspace_size(args: *const Mamba1ScanArgs) -> usize;
     pub fn mamba1_scan_fwd_ws(args: *const Mamba1ScanArgs, workspace: *mut c_void, workspace_bytes: usize, stream: MambaStream, event_start: *mut c_void, event_stop: *mut c_void) -> c_int;
