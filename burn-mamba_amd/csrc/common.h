@@ -136,6 +136,17 @@ __device__ __forceinline__ float wave_incl_scan(float v) {
     return v;
 }
 
+// The same over each half of the wave by itself.
+__device__ __forceinline__ float half_incl_scan(float v) {
+    asm volatile("" : "+v"(v));
+    v += dpp_term(v, 0x111, 0xf);  // row_shr:1
+    v += dpp_term(v, 0x112, 0xf);  // row_shr:2
+    v += dpp_term(v, 0x114, 0xf);  // row_shr:4
+    v += dpp_term(v, 0x118, 0xf);  // row_shr:8
+    v += dpp_term(v, 0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+    return v;
+}
+
 // Wave index inside the workgroup, as a wave-uniform (scalar) value: branches
 // and loops on it stay scalar, so waits on memory counters remain exact.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }

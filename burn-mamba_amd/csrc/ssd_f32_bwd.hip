@@ -558,13 +558,21 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 gh += S.ghc[k];
             }
             const float xg = lane < 32 ? S.xg[0][lane] + S.xg[1][lane] : S.xg[1][lane];
-            const float rowm = lane < 32 ? S.rowm[0][lane] : S.rowm[0][lane] + S.rowm[1][lane];
             const float sc = S.sc[lane];
-            const float z = S.w[lane] * xu, d = sc * xg - rowm;
-            const float pz = wave_incl_scan(z) - z, pd = wave_incl_scan(d) - d;
+            const float z = S.w[lane] * xu, pz = wave_incl_scan(z) - z;
+            // T's pairs j before t <= i: those of t's own 32-row tile as column
+            // less row sums before t (a pair wholly before t cancels); those of
+            // the tile below the diagonal one-sided, with nothing to cancel, as
+            // columns before t or rows from t on.  One scan of 64 rows instead
+            // left dA 1.4 times as far from 64 bits.
+            const float d = sc * S.xg[lane >> 5][lane] - S.rowm[lane >> 5][lane];
+            const float pd = half_incl_scan(d) - d;
+            const int rl = lane < 32 ? lane : 95 - lane;  // rows 32 .. 63 from the last
+            const float x = lane < 32 ? sc * S.xg[1][lane] : S.rowm[0][rl];
+            const float sx = __shfl(half_incl_scan(x), rl, 64), px = lane < 32 ? sx - x : sx;
             // suffix sums of b_i uh_i: the scan runs from the last lane
             const float su = __shfl(wave_incl_scan(__shfl(S.bv[lane] * uh, 63 - lane, 64)), 63 - lane, 64);
-            const float dda = S.dec * gh + pz + su + pd;
+            const float dda = S.dec * gh + pz + su + (px + pd);
             float ds = xg + S.av[lane] * xu, dg = S.dg[lane];
             for (int o = 1; o < p.M; o <<= 1) {
                 ds += __shfl_xor(ds, o, 64);
