@@ -136,7 +136,31 @@ __device__ __forceinline__ float wave_incl_scan(float v) {
     return v;
 }
 
-// The same over each half of the wave by itself.
+// The same in 64 bits.
+__device__ __forceinline__ double dpp_term64(double v, int ctrl, int row_mask) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __float_as_uint(dpp_term(__uint_as_float((uint32_t)u), ctrl, row_mask));
+    const uint32_t hi = __float_as_uint(dpp_term(__uint_as_float((uint32_t)(u >> 32)), ctrl, row_mask));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_incl_scan64(double v) {
+    v += dpp_term64(v, 0x111, 0xf);
+    v += dpp_term64(v, 0x112, 0xf);
+    v += dpp_term64(v, 0x114, 0xf);
+    v += dpp_term64(v, 0x118, 0xf);
+    v += dpp_term64(v, 0x142, 0xa);
+    v += dpp_term64(v, 0x143, 0xc);
+    return v;
+}
+
+__device__ __forceinline__ double wave_lane64(double v, int lane) {  // lane: a constant
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// wave_incl_scan over each half of the wave by itself.
 __device__ __forceinline__ float half_incl_scan(float v) {
     asm volatile("" : "+v"(v));
     v += dpp_term(v, 0x111, 0xf);  // row_shr:1

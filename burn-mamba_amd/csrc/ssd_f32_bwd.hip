@@ -42,6 +42,8 @@
 // What bounds it: the f32 MFMA rate (157 TFLOP/s) and, close behind, HBM (inputs
 // read three times, the entry states written and read, dB / dC per head).
 // 64-row chunks halve the entry states and the barriers against 32-row ones.
+// Sums over rows whose weights fall with the row (g, dv, dB) run from the last
+// row: a term rounds at the size of the sum it meets, so the small ones go first.
 // Measured: the backward at 2 x 4096 steps, 32 heads 64 x 128, rank 4, 5.6 ms ->
 // 2.4 ms (reverse loop 4.53 -> 1.70 ms)
 // against one workgroup per (batch, head, half of dstate) on
@@ -130,8 +132,8 @@ __device__ __forceinline__ FBTab fb_tab(const SsdF32BwdParams& p, const FBJob& j
     return r;
 }
 // a step's decay counts once, at its first rank
-__device__ __forceinline__ float fb_cumsum(const SsdF32BwdParams& p, const FBTab& r, float A, int lane) {
-    return wave_incl_scan((lane & (p.M - 1)) == 0 ? r.da * A : 0.f);
+__device__ __forceinline__ FDecay fb_decay(const SsdF32BwdParams& p, const FBTab& r, float A, int lane) {
+    return f_decay((lane & (p.M - 1)) == 0 ? (double)r.da * A : 0.);
 }
 
 // The state entering segment s as [n][p] tiles (columns p on lanes), or as
@@ -158,7 +160,7 @@ __device__ __forceinline__ void fb_entry(const SsdF32BwdParams& p, const FBJob& 
     const int n = grad ? p.S - 1 - j.s : j.s;
     for (int k = 0; k < n; ++k) {
         const int u = grad ? p.S - 1 - k : k;
-        const float d = __expf(dec[j.bh * p.S + u]);
+        const float d = f_exp(dec[j.bh * p.S + u]);
         const float* q = seg + (j.bh * p.S + u) * (kBP * N) + ln * kBP + lp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -185,6 +187,7 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
     constexpr int TILES = 2 * (N / 32), QT = TILES / 4, NT = 256;
     const int tid = threadIdx.x, wv = wave_id(), lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
     const bool rev = blockIdx.x & 1;
+    const int flip = rev ? kFR - 1 : 0;
     const int idx = blockIdx.x >> 1, u = idx / (p.S - 1), s0 = idx % (p.S - 1);
     const FBJob j = fb_job(p, u, rev ? s0 + 1 : s0);
     const T* xb = static_cast<const T*>(rev ? p.dy : p.v) +
@@ -205,14 +208,14 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
         if (wv == 0) rt = fb_tab(p, j, c, lane);
     };
     auto commit = [&](int c) {
-        f_commit<T, N, NT, N + 4>(rr, S.R, p.L, p.mshift, c, tid);
-        f_commit<T, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
+        f_commit<T, N, NT, N + 4>(rr, S.R, p.L, p.mshift, c, tid, flip);
+        f_commit<T, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid, flip);
         if (wv == 0) {
-            const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64);
-            S.w[lane] = rev ? __expf(cs) : __expf(end - cs) * rt.sc;
+            const FDecay d = fb_decay(p, rt, A, lane);
+            S.w[lane ^ flip] = rev ? d.b : d.a * rt.sc;
             if (lane == 63) {
-                S.dec = __expf(end);
-                S.end = end;
+                S.dec = d.b;
+                S.end = d.end;
             }
         }
     };
@@ -264,9 +267,9 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_states(SsdF32BwdParams p) 
         f_commit<T, N, NT, NP>(rr, S.R, p.L, p.mshift, c, tid);
         f_commit<T, kBP, NT, kBVP>(rx, S.X, p.L, p.mshift, c, tid);
         if (wv == 0) {
-            const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64);
-            S.w[lane] = __expf(end - cs) * rt.sc;
-            if (lane == 63) S.dec = __expf(end);
+            const FDecay d = fb_decay(p, rt, A, lane);
+            S.w[lane] = d.a * rt.sc;
+            if (lane == 63) S.dec = d.b;
         }
     };
     fetch(j.c0);
@@ -317,7 +320,7 @@ struct FBLds {
     float Y[kFR * kBVP];      // dy
     float E1[kFR * kBVP];     // [i][j] W CB
     float E2[kFR * kBVP];     // [i][j] W DV
-    float cs[kFR], gm[kFR], sc[kFR], av[kFR], bv[kFR], w[kFR];
+    float cs[kFR], lo[kFR], gm[kFR], sc[kFR], av[kFR], bv[kFR], w[kFR];
     float P[4][16 * 64];      // [pt, nh] its share of g B for the other row tile, accumulator order
     float xu[4][kFR];         // v_j . g B_j over 32 columns of p and half of n
     float uh[4][kFR];         // C_i . h^T dy_i over 32 columns of n
@@ -349,6 +352,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
     const int own = N == 128 ? 0 : (wv - 2) >> 1;
     FRaw<T> rB[kFR * N / 4 / NT], rC[kFR * N / 4 / NT], rv[kFR * kBP / 4 / NT], ry[kFR * kBP / 4 / NT];
     FBTab rt = {0.f, 0.f, 0.f};
+    FDecay rd = {0.f, 0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](int c, int tid) {
         f_fetch<T, N, NT>(rB, Bb, p.B_sl, p.B_sm, p.L, ms, c, tid);
         f_fetch<T, N, NT>(rC, Cb, p.C_sl, p.C_sm, p.L, ms, c, tid);
@@ -363,19 +367,20 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
         f_commit<T, kBP, NT, kBVP>(rv, S.V, p.L, ms, c, tid);
         f_commit<T, kBP, NT, kBVP>(ry, S.Y, p.L, ms, c, tid);
         if (wv == 1) {
-            const float cs = fb_cumsum(p, rt, A, lane), end = __shfl(cs, 63, 64), a = __expf(end - cs);
-            S.cs[lane] = cs;
+            S.cs[lane] = rd.cs;
+            S.lo[lane] = rd.lo;
             S.gm[lane] = rt.gm;
             S.sc[lane] = rt.sc;
-            S.av[lane] = a;
-            S.bv[lane] = __expf(cs);
-            S.w[lane] = a * rt.sc;
-            if (lane == 63) S.dec = __expf(end);
+            S.av[lane] = rd.a;
+            S.bv[lane] = rd.b;
+            S.w[lane] = rd.a * rt.sc;
+            if (lane == 63) S.dec = rd.b;
         }
     };
     // Each role runs its own loop over the chunks, with the same barriers (A |
     // B | commit |), so that no wave holds another role's accumulators.
     fetch(j.c1 - 1, tid);
+    if (wv == 1) rd = fb_decay(p, rt, A, lane);
     if (wv < 2 || wv >= 6) {
         // 32 columns of p (pt) and half of n (nh): its share of g B for both row
         // tiles, a pair tile, then dv of row tile nh
@@ -430,29 +435,40 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Bc = S.B + (32 * jt + i32) * NP + 4 * hf;
                 const float* Ay = S.Y + (32 * it + i32) * kBVP + 4 * hf;
                 const float* Bv = S.V + (32 * jt + i32) * kBVP + 4 * hf;
+                const int jj = 32 * jt + i32, sj = jj >> ms, row0 = 32 * it + 4 * hf;
+                float* e1 = S.E1 + row0 * kBVP + jj;
+                float* e2 = S.E2 + row0 * kBVP + jj;
                 bwd_f32x16 cb = fb_zero(), dx = fb_zero();
 #pragma unroll
                 for (int s = 0; s < N / 8; ++s) {
                     cb = fb_row4(fb_ld4(Ac + 8 * s), fb_ld4(Bc + 8 * s), cb);
                     if ((s & 3) == 3) fb_fence();
+                    if (s == 7 && N == 128) {
+                        // two sums of 64 products instead of one of 128; the first
+                        // waits where the lane's W CB will go
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) e1[(8 * (r >> 2) + (r & 3)) * kBVP] = cb[r];
+                        cb = fb_zero();
+                    }
                 }
 #pragma unroll
                 for (int s = 0; s < kBP / 8; ++s) {
                     dx = fb_row4(fb_ld4(Ay + 8 * s), fb_ld4(Bv + 8 * s), dx);
                     if ((s & 3) == 3) fb_fence();
                 }
-                const int jj = 32 * jt + i32, sj = jj >> ms, row0 = 32 * it + 4 * hf;
-                const float csj = S.cs[jj], scj = S.sc[jj];
+                const float csj = S.cs[jj], loj = S.lo[jj], scj = S.sc[jj];
                 float rl[16], rs[16], xg = 0.f, dd = 0.f;
-                float* e1 = S.E1 + row0 * kBVP + jj;
-                float* e2 = S.E2 + row0 * kBVP + jj;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const float4 c4 = fb_ld4(&S.cs[row0 + 8 * q]), g4 = fb_ld4(&S.gm[row0 + 8 * q]);
-                    const float ci[4] = {c4.x, c4.y, c4.z, c4.w}, gi[4] = {g4.x, g4.y, g4.z, g4.w};
+                    const float4 c4 = fb_ld4(&S.cs[row0 + 8 * q]), l4 = fb_ld4(&S.lo[row0 + 8 * q]);
+                    const float4 g4 = fb_ld4(&S.gm[row0 + 8 * q]);
+                    const float d[4] = {(c4.x - csj) + (l4.x - loj), (c4.y - csj) + (l4.y - loj),
+                                        (c4.z - csj) + (l4.z - loj), (c4.w - csj) + (l4.w - loj)};
+                    const float gi[4] = {g4.x, g4.y, g4.z, g4.w};
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const int r = 4 * q + k;
+                        if constexpr (N == 128) cb[r] += e1[(8 * q + k) * kBVP];
                         const float t = cb[r] * dx[r];
                         float e, W;
                         if constexpr (DIAG) {
@@ -460,7 +476,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                             // dropped pair's values never enter a sum)
                             const int si = (row0 + 8 * q + k) >> ms;
                             const bool lower = si > sj, same = si == sj;
-                            e = __expf(lower ? ci[k] - csj : 0.f);
+                            e = f_exp(lower ? d[k] : 0.f);
                             W = lower ? e * scj : gi[k];
                             rl[r] = lower ? W * t : 0.f;
                             rs[r] = same ? t : 0.f;
@@ -469,7 +485,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                             e1[(8 * q + k) * kBVP] = lower || same ? W * cb[r] : 0.f;
                             e2[(8 * q + k) * kBVP] = lower || same ? W * dx[r] : 0.f;
                         } else {
-                            e = __expf(ci[k] - csj);
+                            e = f_exp(d[k]);
                             W = e * scj;
                             rl[r] = W * t;
                             xg = __builtin_fmaf(e, t, xg);
@@ -496,6 +512,8 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 tile(std::false_type{}, 1, 0);
             else if (wv == 7)
                 tile(std::true_type{}, 1, 1);
+            else if (c > j.c0)  // wave 1 has no pair tile: the next chunk's decays
+                rd = fb_decay(p, rt, A, lane);
             __syncthreads();
             {
                 const float* in = S.P[2 * pt + 1 - nh] + lane;
@@ -505,11 +523,11 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Ap = S.Y + 4 * hf * kBVP + 32 * pt + i32;
                 const float* Bp = S.E1 + 4 * hf * kBVP + 32 * nh + i32;
 #pragma unroll
-                for (int s = 0; s < 8; ++s)
+                for (int s = 7; s >= 0; --s)
                     if (s >= 4 * nh) {
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) a = bwd_mfma(Ap[(8 * s + k) * kBVP], Bp[(8 * s + k) * kBVP], a);
-                        if (s & 1) fb_fence();
+                        for (int k = 3; k >= 0; --k) a = bwd_mfma(Ap[(8 * s + k) * kBVP], Bp[(8 * s + k) * kBVP], a);
+                        if ((s & 1) == 0) fb_fence();
                     }
                 const int row = 32 * nh + i32, t = t0 + (row >> ms);
                 if (t < p.L) {
@@ -536,16 +554,16 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * GT * nh + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + 32 * pt + i32;
 #pragma unroll
-                for (int s = 0; s < 8; ++s) {
+                for (int s = 7; s >= 0; --s) {
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
+                    for (int e = 3; e >= 0; --e) {
                         const float y = bi[e] * Yp[(8 * s + e) * kBVP];
 #pragma unroll
                         for (int k = 0; k < GT; ++k) G[k] = bwd_mfma(Cp[(8 * s + e) * NP + 32 * k], y, G[k]);
                     }
-                    if (s & 1) fb_fence();
+                    if ((s & 1) == 0) fb_fence();
                 }
             }
             if (wv == 7) {
@@ -678,12 +696,12 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Ep = S.E2 + 4 * hf * kBVP + 32 * xt + i32;
 #pragma unroll
-                for (int s = 0; s < 8; ++s)
+                for (int s = 7; s >= 0; --s)
                     if (s >= 4 * xt) {
 #pragma unroll
-                        for (int k = 0; k < 4; ++k)
+                        for (int k = 3; k >= 0; --k)
                             acc[x] = bwd_mfma(Cp[(8 * s + k) * NP], Ep[(8 * s + k) * kBVP], acc[x]);
-                        if (s & 1) fb_fence();
+                        if ((s & 1) == 0) fb_fence();
                     }
                 const float* Bp = S.B + 4 * hf * NP + 32 * nt + i32;
                 const float* Er = S.E2 + row * kBVP + 4 * hf;
@@ -718,16 +736,16 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + i32;
 #pragma unroll
-                for (int s = 0; s < 8; ++s) {
+                for (int s = 7; s >= 0; --s) {
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
+                    for (int e = 3; e >= 0; --e) {
                         const float cv = bi[e] * Cp[(8 * s + e) * NP];
 #pragma unroll
                         for (int k = 0; k < 2; ++k) G[k] = bwd_mfma(Yp[(8 * s + e) * kBVP + 32 * k], cv, G[k]);
                     }
-                    if (s & 1) fb_fence();
+                    if ((s & 1) == 0) fb_fence();
                 }
             }
             __syncthreads();

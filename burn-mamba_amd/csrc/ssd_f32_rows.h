@@ -9,6 +9,31 @@
 namespace mamba {
 
 constexpr int kFR = 64;  // fused rows per chunk
+constexpr double kFLog2e = 1.4426950408889634;
+
+// The decays of a chunk's rows (lane = row) in log2 units, summed in 64 bits: the
+// decay between two rows is a difference of sums that may be far larger than
+// itself, and with sums in f32 it is off by their rounding (under strong decays
+// that left dv and dB up to 1.8 times as far from 64 bits as sums taken row by row
+// over 32).  cs + lo is the sum up to the row; the difference of two rows is
+// (cs_i - cs_j) + (lo_i - lo_j), and f_exp of it costs less than an __expf.
+struct FDecay {
+    float cs, lo;
+    float a, b;  // decay factors from the row to the chunk's end, and up to the row
+    float end;   // the whole chunk's, in log2 units
+};
+__device__ __forceinline__ float f_exp(float x) { return __builtin_amdgcn_exp2f(x); }
+// x: the row's log-decay
+__device__ __forceinline__ FDecay f_decay(double x) {
+    const double cs = wave_incl_scan64(x * kFLog2e), end = wave_lane64(cs, 63);
+    FDecay d;
+    d.cs = (float)cs;
+    d.lo = fabsf(d.cs) < INFINITY ? (float)(cs - (double)d.cs) : 0.f;
+    d.a = f_exp((float)(end - cs));
+    d.b = f_exp(d.cs);
+    d.end = (float)end;
+    return d;
+}
 
 // four values of a row, as f32
 template <typename T>
@@ -41,16 +66,17 @@ __device__ __forceinline__ void f_fetch(FRaw<T> (&raw)[kFR * W / 4 / NT], const 
         raw[q].v = *reinterpret_cast<const decltype(raw[q].v)*>(base + at);
     }
 }
+// flip: 0, or kFR - 1 for the rows in reverse
 template <typename T, int W, int NT, int PITCH>
 __device__ __forceinline__ void f_commit(const FRaw<T> (&raw)[kFR * W / 4 / NT], float* dst, int L, int mshift, int c,
-                                         int tid) {
+                                         int tid, int flip = 0) {
     constexpr int RW = W / 4;
 #pragma unroll
     for (int q = 0; q < kFR * W / 4 / NT; ++q) {
         const int e = tid + NT * q, row = e / RW, col = (e % RW) * 4;
         const int t = c * (kFR >> mshift) + (row >> mshift);
         const float4 z = {0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<float4*>(dst + row * PITCH + col) = t < L ? raw[q].get() : z;
+        *reinterpret_cast<float4*>(dst + (row ^ flip) * PITCH + col) = t < L ? raw[q].get() : z;
     }
 }
 

@@ -78,6 +78,33 @@ def test_ssd3(case):
         _close(out["dscale"], want["dscale"], "dscale")
 
 
+@pytest.mark.parametrize("l,h", [(64, 2), (200, 2), (200, 300)])
+def test_ssd2_decays_after_a_reset(l, h):
+    """A first half of 32 positions whose decays sum to 3200, then weak ones: the
+    decay between two late positions is no difference of sums of that size
+    (spacing 2^-12: 1e-4 off).  The late rows' own sums stay below 1, so that an
+    exp is 2^-23 off and a gradient a few times that: 2e-6 of its 2-norm, on
+    whole and on split sequences."""
+    import torch
+    import mamba_hip
+    b, g, n, p = 1, 1, 64, 64
+    rng = np.random.default_rng(l)
+    r = lambda *s: rng.standard_normal(s, dtype=np.float32)  # noqa: E731
+    x, dy, B, C = r(b, l, h, p), r(b, l, h, p), r(b, l, g, n) / 8, r(b, l, g, n) / 8
+    dt = rng.uniform(0.01, 0.03, (b, l, h)).astype(np.float32)
+    dt[:, np.arange(l) % 64 < 32] = 100.0
+    A = np.full(h, -1.0, np.float32)
+    x[:, np.arange(l) % 64 < 32] *= 1e-4  # dt weighs them
+    out = mamba_hip.ssd2_bwd(_t(dy), _t(x), _t(dt), _t(A), _t(B), _t(C))
+    torch.cuda.synchronize()
+    want = oracle.ssd2_bwd(dy, None, x, dt, A, B, C, None, None)
+    late = np.arange(l) % 64 >= 32
+    for k in ("dx", "dB", "dC"):
+        got, ref = out[k].cpu().numpy()[:, late].astype(np.float64), want[k][:, late]
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert err < 2e-6, (k, err)
+
+
 def test_ssd2_any_segment_count_gives_the_same_gradients():
     """A workspace that holds fewer segments (as small as the SIMT kernels', one
     entry state per 32 positions) is used with fewer; both agree to f32 rounding."""
