@@ -26,7 +26,7 @@ struct SsdF32Params {
     void* y; int64_t y_sb, y_sl, y_sm, y_sh;
     float* hT;
     float* seg;             // [b h pblock][S][N * PB] segment-local final states
-    float* segd;            // [b h pblock][S] segment log-decays
+    float* segd;            // [b h pblock][S] segment log2-decays
 };
 
 // Whether the kernels cover these shapes and layouts; fills nch, S and cps.

@@ -47,7 +47,7 @@ struct FTabRaw {
 };
 
 struct FTables {
-    float cs[kFR], gm[kFR], sc[kFR];
+    float cs[kFR], lo[kFR], gm[kFR], sc[kFR];  // cs, lo: FDecay
     float w[kFR];  // sc exp(cs_end - cs): the weights of the state update
     float dec, end;
 };
@@ -82,20 +82,23 @@ __device__ __forceinline__ FTabRaw f_tab_fetch(const SsdF32Params& p, const FJob
     r.sc = p.sc ? p.sc[(int64_t)j.b * p.sc_sb + (int64_t)t * p.sc_sl + (int64_t)j.h * p.sc_sh] : 1.f;
     return r;
 }
-__device__ __forceinline__ void f_tab_commit(const SsdF32Params& p, const FTabRaw& r, FTables& T, float A, int c,
-                                             int lane) {
+__device__ __forceinline__ FDecay f_tab_decay(const SsdF32Params& p, const FTabRaw& r, float A, int c, int lane) {
     const bool ok = c * (kFR >> p.mshift) + (lane >> p.mshift) < p.L;
     // a step's decay counts once, at its first rank
-    const float cs = wave_incl_scan(ok && (lane & (p.M - 1)) == 0 ? r.da * A : 0.f);
-    const float end = __shfl(cs, 63, 64);
+    return f_decay(ok && (lane & (p.M - 1)) == 0 ? (double)r.da * A : 0.);
+}
+__device__ __forceinline__ void f_tab_commit(const SsdF32Params& p, const FTabRaw& r, const FDecay& d, FTables& T, int c,
+                                             int lane) {
+    const bool ok = c * (kFR >> p.mshift) + (lane >> p.mshift) < p.L;
     const float sc = ok ? r.sc : 0.f;
-    T.cs[lane] = cs;
+    T.cs[lane] = d.cs;
+    T.lo[lane] = d.lo;
     T.gm[lane] = ok ? r.gm : 0.f;
     T.sc[lane] = sc;
-    T.w[lane] = __expf(end - cs) * sc;
+    T.w[lane] = d.a * sc;
     if (lane == 63) {
-        T.dec = __expf(end);
-        T.end = end;
+        T.dec = d.b;
+        T.end = d.end;
     }
 }
 
@@ -103,7 +106,8 @@ template <int PB, int N>
 struct FStateLds {
     float B[kFR * (N + 4)];
     float V[kFR * (PB + 8)];
-    FTables T;
+    float w[kFR];  // as FTables
+    float dec, end;
 };
 
 template <typename T, int PB, int N>
@@ -131,7 +135,14 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_state(SsdF32Params p) {
     auto commit = [&](int c) {
         f_commit<T, N, NT, N + 4>(rb, S.B, p.L, p.mshift, c, tid);
         f_commit<T, PB, NT, PB + 8>(rv, S.V, p.L, p.mshift, c, tid);
-        if (wv == 0) f_tab_commit(p, rt, S.T, A, c, lane);
+        if (wv == 0) {
+            const FDecay d = f_tab_decay(p, rt, A, c, lane);
+            S.w[lane] = c * (kFR >> p.mshift) + (lane >> p.mshift) < p.L ? d.a * rt.sc : 0.f;
+            if (lane == 63) {
+                S.dec = d.b;
+                S.end = d.end;
+            }
+        }
     };
     fetch(j.c0);
     commit(j.c0);
@@ -139,8 +150,8 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_state(SsdF32Params p) {
     float total = 0.f;
     for (int c = j.c0; c < j.c1; ++c) {
         if (c + 1 < j.c1) fetch(c + 1);
-        total += S.T.end;
-        f_update<PB, N, QT, PB + 8>(acc, S.B, S.V, S.T.w, S.T.dec, wv, i32, hf);
+        total += S.end;
+        f_update<PB, N, QT, PB + 8>(acc, S.B, S.V, S.w, S.dec, wv, i32, hf);
         __syncthreads();
         if (c + 1 < j.c1) commit(c + 1);
         __syncthreads();
@@ -183,17 +194,18 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
     const int steps = kFR >> p.mshift;
     FRaw<T> rb[kFR * N / 4 / NT], rc[kFR * N / 4 / NT], rv[kFR * PB / 4 / NT];
     FTabRaw rt = {0.f, 0.f, 0.f};
+    FDecay rd = {0.f, 0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](int c) {
         f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
         f_fetch<T, N, NT>(rc, Cb, p.C_sl, p.C_sm, p.L, p.mshift, c, tid);
         f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
-        if (wv == 0) rt = f_tab_fetch(p, j, c, lane);
+        if (wv == 7) rt = f_tab_fetch(p, j, c, lane);
     };
     auto commit = [&](int c) {
         f_commit<T, N, NT, NP>(rb, S.B, p.L, p.mshift, c, tid);
         f_commit<T, N, NT, NP>(rc, S.C, p.L, p.mshift, c, tid);
         f_commit<T, PB, NT, VP>(rv, S.V, p.L, p.mshift, c, tid);
-        if (wv == 0) f_tab_commit(p, rt, S.T, A, c, lane);
+        if (wv == 7) f_tab_commit(p, rt, rd, S.T, c, lane);
     };
     const bool st = wv >= 4;  // wave-uniform
     const int w4 = wv & 3;
@@ -230,7 +242,7 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
             const float* sp = p.seg + j.hp * p.S * (int64_t)(N * PB) + t * 1024 + lane;
 #pragma unroll 4
             for (int u = 0; u < j.s; ++u) {
-                const float dec = __expf(p.segd[j.hp * p.S + u]);
+                const float dec = f_exp(p.segd[j.hp * p.S + u]);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     acc[q][r] = __builtin_fmaf(acc[q][r], dec, sp[(int64_t)u * (N * PB) + r * 64]);
@@ -238,6 +250,7 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
         }
         publish();
     }
+    if (wv == 7) rd = f_tab_decay(p, rt, A, j.c0, lane);
     commit(j.c0);
     __syncthreads();
     // y waves: rows 32 it, columns 32 pt
@@ -259,7 +272,7 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) ya = bwd_mfma(Ap[(8 * s + k) * VP], cj[k], ya);
             }
-            const float e = __expf(S.T.cs[32 * it + i32]);
+            const float e = f_exp(S.T.cs[32 * it + i32]);
 #pragma unroll
             for (int r = 0; r < 16; ++r) ya[r] *= e;
         }
@@ -281,15 +294,17 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
                 a = bwd_mfma(bv.w, cv.w, a);
             }
             const int i = 32 * wi + i32, si = i >> p.mshift;
-            const float csi = S.T.cs[i], gmi = S.T.gm[i];
+            const float csi = S.T.cs[i], loi = S.T.lo[i], gmi = S.T.gm[i];
             float* Wp = S.W + 32 * jt * WP + i;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int jr = bwd_row(r, hf), jj = 32 * jt + jr, sj = jj >> p.mshift;
-                const float k = sj < si ? __expf(csi - S.T.cs[jj]) * S.T.sc[jj] : gmi;
+                const float k = sj < si ? f_exp((csi - S.T.cs[jj]) + (loi - S.T.lo[jj])) * S.T.sc[jj] : gmi;
                 Wp[jr * WP] = sj <= si ? a[r] * k : 0.f;
             }
         }
+        // wave 7 has no tile of C.B^T: the next chunk's decays
+        if (wv == 7 && c + 1 < j.c1) rd = f_tab_decay(p, rt, A, c + 1, lane);
         __syncthreads();
         if (yw) {
             // += sum_j v[j][p] W[j][i]

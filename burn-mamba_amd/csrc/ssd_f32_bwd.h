@@ -32,7 +32,7 @@ struct SsdF32BwdParams {
     // workspace
     float* hs;             // [b h][chunk][tile][16][64] states entering the chunks
     float* fs; float* gs;  // [b h][S][n][p] segment-local states and state gradients
-    float* fd; float* gd;  // [b h][S] segment log-decays
+    float* fd; float* gd;  // [b h][S] segment log2-decays
     float* pA; float* pD;  // [b h][S] partial dA, dD (Mamba-2)
 };
 

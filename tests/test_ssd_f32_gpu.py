@@ -3,7 +3,7 @@ Mamba-3 seams at the edges of its chunks (64 fused rows), segments, headdim
 blocks and ranks, vs the f64 oracle.
 
 Tolerance: a result is a sum of at most a few hundred f32 products of O(1)
-terms, each off by 2^-24 relative and by the ~2^-21 of an exp of |x| <= 8, so
+terms, each off by 2^-24 relative and by the 2^-22 of an exp of its decay, so
 1e-5 of the row's scale bounds it; rtol 1e-4 is the f32 bar of the other tests.
 bf16 results are rounded once, 2^-9."""
 
@@ -81,6 +81,31 @@ def test_ssd3(case, double):
     tol = dict(rtol=1e-4, atol=2e-5 * max(1.0, m ** 0.5))
     np.testing.assert_allclose(y.cpu().numpy(), yr, **tol)
     np.testing.assert_allclose(hT.cpu().numpy(), hr, **tol)
+
+
+@pytest.mark.parametrize("l", [64, 200])
+def test_ssd2_decays_after_a_reset(l):
+    """A first half of 32 positions whose decays sum to 3200, then weak ones: the
+    decay between two late positions is no difference of sums of that size
+    (spacing 2^-12: 1e-4 off).  The late positions' own sums stay below 1, so that
+    an exp is 2^-22 off and y a few times that: 1e-6 of its 2-norm, on whole and
+    on split sequences."""
+    import torch
+    import mamba_hip
+    import oracle
+    b, h, p, n = 1, 2, 64, 64
+    inp = ssd2_inputs(seed=l, b=b, l=l, h=h, p=p, g=1, n=n, h0=False)
+    strong = np.arange(l) % 64 < 32
+    inp["A"][:] = -1.0
+    inp["dt"][:] = np.random.default_rng(l).uniform(0.01, 0.03, (b, l, h))
+    inp["dt"][:, strong] = 100.0
+    inp["x"][:, strong] *= np.float32(1e-4)  # dt weighs them
+    t = {k: _dev(v) for k, v in inp.items()}
+    y, hT = mamba_hip.ssd2_fwd(t["x"], t["dt"], t["A"], t["B"], t["C"], chunk_len=64)
+    torch.cuda.synchronize()
+    yr, hr = oracle.ssd2(inp["x"], inp["dt"], inp["A"], inp["B"], inp["C"], None, None, chunk=64)
+    for got, ref in ((y.cpu().numpy()[:, ~strong], yr[:, ~strong]), (hT.cpu().numpy(), hr)):
+        assert np.linalg.norm(got - ref) < 1e-6 * np.linalg.norm(ref)
 
 
 def test_ssd2_workspace_of_the_generic_path_still_serves():
