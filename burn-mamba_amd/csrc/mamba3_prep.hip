@@ -746,9 +746,7 @@ __global__ __launch_bounds__(256) void mamba3_finish_vec(M3FinishParams p) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float zv = M > 1 ? z[e] * mz[w][e] : z[e];
-                const float den = 1.f + __expf(-zv);
-                // a bf16 result takes the hardware reciprocal (1 ulp of f32)
-                const float sz = sizeof(T) == 2 ? zv * __builtin_amdgcn_rcpf(den) : zv / den;
+                const float sz = zv / (1.f + __expf(-zv));
                 float gv = p.onw ? (o[m][e] * inv) * on[e] * sz : o[m][e] * sz;
                 if (M > 1) gv *= mo[w][e];
                 acc[e] += gv;

@@ -39,3 +39,21 @@ def test_finish(case, dtype):
                                                                  out_norm_w=onw if norm else None))
     tol = dict(rtol=1e-4, atol=2e-5) if dtype == "f32" else dict(rtol=1e-2, atol=1e-2)
     np.testing.assert_allclose(out.float().cpu().numpy(), want, **tol)
+
+
+def test_gate_divides_as_the_general_kernel_does():
+    """bf16, one rank, no norm: both kernels form y z / (1 + exp(-z)) in f32 and
+    round once, so that they agree bit for bit (a reciprocal 1 ulp off would turn
+    about one bf16 rounding in 2^17: some 60 of these 8 million)."""
+    import torch
+    import mamba_hip
+    b, L, H, P = 2, 8192, 8, 64
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    y = torch.randn(b, L, 1, H, P, device="cuda", generator=gen).bfloat16()
+    z = (4 * torch.randn(b, L, H * P, device="cuda", generator=gen)).bfloat16()
+    cfg = mamba_hip.Mamba3Config(d_model=H * P // 2, per_head_dim=P, mimo_rank=1)
+    out = mamba_hip.mamba3_finish_fwd(cfg, y, None, z)
+    odd = torch.empty(b * L * H * P + 1, device="cuda", dtype=torch.bfloat16)[1:].view(b, L, H * P)
+    mamba_hip.mamba3_finish_fwd(cfg, y, None, z, out=odd)  # rows off 16 bytes: the general kernel
+    torch.cuda.synchronize()
+    assert torch.equal(out, odd)
