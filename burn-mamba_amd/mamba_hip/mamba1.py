@@ -258,9 +258,16 @@ def mm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None)
     """mamba_mm_f32: a [z, m, k] @ b [z, k, n] -> [z, m, n] (f32; a unit stride in
     one of the last two axes of each; expanded batch axes are read in place)."""
     z, m, k = a.shape
-    n = b.shape[2]
+    n = b.shape[-1]
+    # the kernel is handed pointers: what a matmul would refuse is refused here
+    if b.shape != (z, k, n) or (out is not None and (out.shape != (z, m, n) or out.stride(2) != 1)):
+        raise _lib.MambaHipError(f"mm_f32: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not match, or out's rows")
     if out is None:
         out = torch.empty((z, m, n), device=a.device, dtype=torch.float32)
+    if not (a.dtype == b.dtype == out.dtype == torch.float32):
+        raise _lib.MambaHipError("mm_f32: float32 required")
+    if not (a.is_cuda and a.device == b.device == out.device):
+        raise _lib.MambaHipError(f"mm_f32: operands on {a.device}, {b.device}, {out.device}: one GPU device required")
     g = _lib.MmF32Args()
     g.batch, g.m, g.n, g.k = z, m, n, k
     g.a, (g.a_sb, g.a_sm, g.a_sk) = a.data_ptr(), a.stride()
