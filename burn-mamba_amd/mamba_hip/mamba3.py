@@ -611,7 +611,8 @@ class Mamba3Stack:
         """In-place step of the whole stack: x_res [b, d_model] f32 becomes the
         stack output.  ``events``: optional list of one torch.cuda.Event pair per
         layer, recorded around that layer's mamba3_step_ssm (one stream)."""
-        if x_res.dtype != torch.float32 or x_res.dim() != 2 or x_res.stride(1) != 1:
+        if x_res.dtype != torch.float32 or x_res.dim() != 2 or x_res.stride(1) != 1 or \
+                x_res.shape[1] != self.cfg.d_model:
             raise _lib.MambaHipError("x_res must be a row-contiguous [b, d_model] float32 tensor")
         b = x_res.shape[0]
         K = self.parts(b) if events is None else 1

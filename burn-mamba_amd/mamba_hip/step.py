@@ -231,6 +231,14 @@ def linear_row(x: torch.Tensor, packed_w: torch.Tensor, out: torch.Tensor, norm_
                bias: Optional[torch.Tensor] = None, accumulate: bool = False) -> None:
     """mamba_linear_row: out = x W (+ bias) for one row, x bf16, or f32 and
     RMS-normed first (norm_w given); accumulate adds to an f32 out."""
+    ts = [t for t in (x, out, norm_w, bias, packed_w) if t is not None]
+    if not all(t.is_contiguous() for t in ts) or any(t.device != x.device for t in ts):
+        raise _lib.MambaHipError("linear_row: contiguous operands on one device required")
+    for t, like in ((norm_w, x), (bias, out)):
+        if t is not None and (t.dtype != torch.float32 or t.numel() != like.numel()):
+            raise _lib.MambaHipError("linear_row: norm_w and bias must be float32 of x's and out's sizes")
+    if packed_w.numel() != _lib.lib().mamba_linear_packed_size(x.numel(), out.numel()):
+        raise _lib.MambaHipError(f"linear_row: packed_w is not a packed {x.numel()} x {out.numel()} weight")
     a = _lib.LinearRowArgs()
     a.d_in, a.d_out = x.numel(), out.numel()
     a.x_dtype, a.y_dtype = _dtype_code(x), _dtype_code(out)
