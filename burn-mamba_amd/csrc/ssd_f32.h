@@ -25,7 +25,7 @@ struct SsdF32Params {
     const float* init_hpr;  // [h, p, n] or NULL
     void* y; int64_t y_sb, y_sl, y_sm, y_sh;
     float* hT;
-    float* seg;             // [b h pblock][S][N * PB] segment-local final states
+    float* seg;             // [b h pblock][S][N * PB] segments' end states (0: from the initial state, which S - 1 holds)
     float* segd;            // [b h pblock][S] segment log2-decays
 };
 

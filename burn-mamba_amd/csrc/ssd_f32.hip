@@ -15,9 +15,14 @@
 //
 // Two launches (one when a (batch, head) is not split):
 //   1. ssd_f32_state: one 4-wave workgroup per (batch, head, 64 columns of
-//      headdim, segment but the last) forms the segment's state from zero.
+//      headdim, segment but the last) forms the segment's state, the first from
+//      the initial state, the others from zero.
 //   2. ssd_f32_scan: one 8-wave workgroup per (.., segment) sums the earlier
 //      segments' states into its entry state and walks the segment's chunks.
+//      Segment 0 finds the initial state in the last segment's place in the
+//      workspace, which has no state of its own there: only the first launch
+//      reads it from its memory, which the scan may write (final_state may be
+//      the same memory).
 //      Waves 0-3 each form a 32 x 32 tile of y; waves 4-7 form C.B^T, then
 //      update the state, which stays in their accumulators, so that on every
 //      SIMD one wave's y tile runs beside another's update.
@@ -102,6 +107,24 @@ __device__ __forceinline__ void f_tab_commit(const SsdF32Params& p, const FTabRa
     }
 }
 
+// The initial state's tile t (rows n 32 (t / (PB / 32)), columns p 32 (t % (PB / 32))).
+template <int PB, int N>
+__device__ __forceinline__ void f_h0(const SsdF32Params& p, const FJob& j, int t, int i32, int hf, bwd_f32x16& a) {
+    constexpr int PT = PB / 32;
+    const int64_t at = (int64_t)(j.p0 + 32 * (t % PT) + i32) * N + 32 * (t / PT) + 4 * hf;
+    const int64_t bh = (int64_t)j.b * p.H + j.h, pn = (int64_t)p.P * N;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        float4 x = {0.f, 0.f, 0.f, 0.f};
+        if (p.h0) x = *reinterpret_cast<const float4*>(p.h0 + bh * pn + at + 8 * k);
+        if (p.init_hpr) {
+            const float4 i = *reinterpret_cast<const float4*>(p.init_hpr + j.h * pn + at + 8 * k);
+            x.x += i.x; x.y += i.y; x.z += i.z; x.w += i.w;
+        }
+        a[4 * k] = x.x; a[4 * k + 1] = x.y; a[4 * k + 2] = x.z; a[4 * k + 3] = x.w;
+    }
+}
+
 template <int PB, int N>
 struct FStateLds {
     float B[kFR * (N + 4)];
@@ -123,10 +146,21 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_state(SsdF32Params p) {
     FRaw<T> rb[kFR * N / 4 / NT], rv[kFR * PB / 4 / NT];
     FTabRaw rt = {0.f, 0.f, 0.f};
     bwd_f32x16 acc[QT];
+    float* const seg = p.seg + j.hp * p.S * (int64_t)(N * PB) + lane;
 #pragma unroll
-    for (int q = 0; q < QT; ++q)
+    for (int q = 0; q < QT; ++q) {
+        const int t = wv + 4 * q;
+        if (t >= TILES) break;
+        if (j.s == 0 && (p.h0 || p.init_hpr)) {
+            f_h0<PB, N>(p, j, t, i32, hf, acc[q]);
+            float* out = seg + (p.S - 1) * (int64_t)(N * PB) + t * 1024;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+            for (int r = 0; r < 16; ++r) out[r * 64] = acc[q][r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+        }
+    }
     auto fetch = [&](int c) {
         f_fetch<T, N, NT>(rb, Bb, p.B_sl, p.B_sm, p.L, p.mshift, c, tid);
         f_fetch<T, PB, NT>(rv, vb, p.v_sl, p.v_sm, p.L, p.mshift, c, tid);
@@ -156,13 +190,13 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_state(SsdF32Params p) {
         if (c + 1 < j.c1) commit(c + 1);
         __syncthreads();
     }
-    float* out = p.seg + (j.hp * p.S + j.s) * (int64_t)(N * PB);
+    float* out = seg + j.s * (int64_t)(N * PB);
 #pragma unroll
     for (int q = 0; q < QT; ++q) {
         const int t = wv + 4 * q;
         if (t >= TILES) break;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[t * 1024 + r * 64 + lane] = acc[q][r];
+        for (int r = 0; r < 16; ++r) out[t * 1024 + r * 64] = acc[q][r];
     }
     if (tid == 0) p.segd[j.hp * p.S + j.s] = total;
 }
@@ -222,26 +256,22 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
     };
     fetch(j.c0);
     if (st) {
-        // the entering state: h0 through the earlier segments, oldest first
+        // the entering state: segment 0's end through the later ones, oldest first
 #pragma unroll
         for (int q = 0; q < QT; ++q) {
             const int t = w4 + 4 * q;
             if (t >= TILES) break;
-            const int64_t at = (int64_t)(j.p0 + 32 * (t % PT) + i32) * N + 32 * (t / PT) + 4 * hf;
-            const int64_t bh = (int64_t)j.b * p.H + j.h, pn = (int64_t)p.P * N;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float4 x = {0.f, 0.f, 0.f, 0.f};
-                if (p.h0) x = *reinterpret_cast<const float4*>(p.h0 + bh * pn + at + 8 * k);
-                if (p.init_hpr) {
-                    const float4 i = *reinterpret_cast<const float4*>(p.init_hpr + j.h * pn + at + 8 * k);
-                    x.x += i.x; x.y += i.y; x.z += i.z; x.w += i.w;
-                }
-                acc[q][4 * k] = x.x; acc[q][4 * k + 1] = x.y; acc[q][4 * k + 2] = x.z; acc[q][4 * k + 3] = x.w;
-            }
             const float* sp = p.seg + j.hp * p.S * (int64_t)(N * PB) + t * 1024 + lane;
+            if (p.S == 1) {
+                f_h0<PB, N>(p, j, t, i32, hf, acc[q]);
+                continue;
+            }
+            const bool zero = j.s == 0 && !p.h0 && !p.init_hpr;
+            const int64_t first = j.s == 0 ? p.S - 1 : 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[q][r] = zero ? 0.f : sp[first * (N * PB) + r * 64];
 #pragma unroll 4
-            for (int u = 0; u < j.s; ++u) {
+            for (int u = 1; u < j.s; ++u) {
                 const float dec = f_exp(p.segd[j.hp * p.S + u]);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)

@@ -107,7 +107,7 @@ typedef struct mamba_ssd2_args {
     const float* initial_state;                     /* [b, h, p, n] f32 or NULL */
     const float* init_state_hpr;                    /* [h, p, n] f32 or NULL (learnable h0) */
     void* y;        int64_t y_sb, y_sl, y_sh;      /* [b, l, h, p]          */
-    float* final_state;                             /* [b, h, p, n] f32      */
+    float* final_state;                             /* [b, h, p, n] f32; may be initial_state */
 } mamba_ssd2_args;
 
 size_t mamba_ssd2_workspace_size(const mamba_ssd2_args* args);
@@ -213,7 +213,7 @@ typedef struct mamba_ssd3_args {
     const void* C;      int64_t C_sb, C_sl, C_sm, C_sg;      /* [b, l, m, g, n]      */
     const float* initial_state;                              /* [b, h, p, n] or NULL */
     void* y;            int64_t y_sb, y_sl, y_sm, y_sh;      /* [b, l, m, h, p]      */
-    float* final_state;                                      /* [b, h, p, n] f32     */
+    float* final_state;                     /* [b, h, p, n] f32; may be initial_state */
 } mamba_ssd3_args;
 
 size_t mamba_ssd3_workspace_size(const mamba_ssd3_args* args);
@@ -253,7 +253,7 @@ typedef struct mamba_ssd3_double_args {
     const void* C;      int64_t C_sb, C_sl, C_sm, C_sg;      /* [b, l, m, g, n]      */
     const float* initial_state;                              /* [b, h, p, n] or NULL */
     void* y;            int64_t y_sb, y_sl, y_sm, y_sh;      /* [b, l, m, h, p]      */
-    float* final_state;                                      /* [b, h, p, n] f32     */
+    float* final_state;                     /* [b, h, p, n] f32; may be initial_state */
 } mamba_ssd3_double_args;
 
 size_t mamba_ssd3_double_workspace_size(const mamba_ssd3_double_args* args);
