@@ -9,8 +9,8 @@
 //      C_c.B_c^T tiles (K2, computed once per group instead of once per head,
 //      f32 accumulation rounded to bf16), C_c and B_c in bf16, written as one
 //      packed run of 1 KB MFMA operand fragments per (batch, chunk, group).
-//   (ssd2_seg_state: the segments' states from zero, where (batch, head) alone
-//      leaves the chip idle.)
+//   (ssd2_seg_state: the segments' end states, where (batch, head) alone leaves
+//      the chip idle.)
 //   2. ssd2_scan_wu: one wave per (batch, head, 32-wide headdim half) walks
 //      the chunks in order, with the running state in its MFMA accumulators
 //      for the whole sequence (K4 needs no HBM round trip).  The HPW waves of
@@ -79,14 +79,40 @@ __device__ __forceinline__ f32x16_t zero16() {
     return z;
 }
 
-// Segments of a launch: chunks [s cps, (s + 1) cps) each, with the states of all
-// but the last from zero ([b h, headdim half][S][tile][16][64], accumulator
-// order) and their log2 decays ([b h][S]).
+// Segments of a launch: chunks [s cps, (s + 1) cps) each, with the end states of
+// all but the last ([b h, headdim half][S][tile][16][64], accumulator order; the
+// first from the initial state, the others from zero) and their log2 decays
+// ([b h][S]).  The last segment's place holds the initial state for segment 0:
+// the state pass alone reads it from its memory, which the scan may write
+// (final_state may be the same memory).
 struct Ssd2Seg {
     int S, cps;
     float* state;
     float* decay;
 };
+
+// The initial state of a (batch, head, headdim half) in accumulator order: tile
+// nt, register v holds (n = 32 nt + 8 (v/4) + 4 half + v%4, p = p0 + r).
+template <int NTN>
+__device__ __forceinline__ void ssd2_h0(const Ssd2Params& p, int b, int h, int p0, int lane, f32x16_t (&hacc)[NTN]) {
+    const int r = lane & 31, half = lane >> 5, N = 32 * NTN;
+    const float* hin = p.h0 ? p.h0 + (((int64_t)b * p.H + h) * 64 + p0 + r) * N : nullptr;
+    const float* hid = p.init_hpr ? p.init_hpr + ((int64_t)h * 64 + p0 + r) * N : nullptr;
+#pragma unroll
+    for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int n = 32 * nt + 8 * q + 4 * half;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (hin) v = *(const float4*)(hin + n);
+            if (hid) {
+                const float4 u = *(const float4*)(hid + n);
+                v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+            }
+            hacc[nt][4 * q] = v.x; hacc[nt][4 * q + 1] = v.y;
+            hacc[nt][4 * q + 2] = v.z; hacc[nt][4 * q + 3] = v.w;
+        }
+}
 
 // Fragments per (batch, chunk, group), in the order the scan kernel stages them:
 //   CB  it*(it+1) + ks         (C.B^T)[i = 32 it + lane%32][j = 16 ks + 8 (lane/32) + e],
@@ -243,8 +269,8 @@ __global__ __launch_bounds__(256) void ssd2_prep_pack(Ssd2Params p, bf16_t* frag
 // The launch bound caps a wave at 256 registers (two waves per SIMD), which
 // keeps the accumulators in VGPRs next to the VALU work that scales them.
 //
-// SEG: blockIdx.y is a segment of sg.cps chunks, whose entry state is the
-// initial state carried through the earlier segments' (ssd2_seg_state).
+// SEG: blockIdx.y is a segment of sg.cps chunks, whose entry state is the end of
+// segment 0 carried through the later ones before it (ssd2_seg_state).
 template <int N, int Q, int HPW, bool SEG>
 __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu(Ssd2Params p, const bf16_t* frag,
                                                                                 Ssd2Seg sg) {
@@ -288,40 +314,27 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
     const int c_lo = SEG ? (int)blockIdx.y * sg.cps : 0;
     const int c_hi = SEG ? min(p.nch, c_lo + sg.cps) : p.nch;
 
-    // ---- the state h^T: tile nt, register v holds (n = 32 nt + 8 (v/4) + 4 half + v%4, p = p0 + r)
-    f32x16_t hacc[NTN];
-    {
-        const int r = lane0 & 31, half = lane0 >> 5;
-        const int64_t hrow = (((int64_t)b * p.H + h) * 64 + p0 + r) * N;
-        const float* hin = p.h0 ? p.h0 + hrow : nullptr;
-        const float* hid = p.init_hpr ? p.init_hpr + ((int64_t)h * 64 + p0 + r) * N : nullptr;
+    f32x16_t hacc[NTN];  // the state h^T
+    if constexpr (SEG) {
+        const int64_t bh = (int64_t)b * p.H + h;
+        const float* st = sg.state + (bh * 2 + ph) * sg.S * (NTN * 1024) + lane0;
+        const bool zero = blockIdx.y == 0 && !p.h0 && !p.init_hpr;
+        const int64_t first = blockIdx.y == 0 ? sg.S - 1 : 0;
 #pragma unroll
         for (int nt = 0; nt < NTN; ++nt)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = 32 * nt + 8 * q + 4 * half;
-                float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (hin) v = *(const float4*)(hin + n);
-                if (hid) {
-                    const float4 u = *(const float4*)(hid + n);
-                    v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
-                }
-                hacc[nt][4 * q] = v.x; hacc[nt][4 * q + 1] = v.y;
-                hacc[nt][4 * q + 2] = v.z; hacc[nt][4 * q + 3] = v.w;
-            }
-        if constexpr (SEG) {
-            const int64_t bh = (int64_t)b * p.H + h;
-            const float* st = sg.state + (bh * 2 + ph) * sg.S * (NTN * 1024) + lane0;
+            for (int v = 0; v < 16; ++v) hacc[nt][v] = zero ? 0.f : st[first * (NTN * 1024) + nt * 1024 + v * 64];
 #pragma unroll 2
-            for (int u = 0; u < (int)blockIdx.y; ++u) {
-                const float dec = __builtin_amdgcn_exp2f(sg.decay[bh * sg.S + u]);
+        for (int u = 1; u < (int)blockIdx.y; ++u) {
+            const float dec = __builtin_amdgcn_exp2f(sg.decay[bh * sg.S + u]);
 #pragma unroll
-                for (int nt = 0; nt < NTN; ++nt)
+            for (int nt = 0; nt < NTN; ++nt)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        hacc[nt][v] = __builtin_fmaf(hacc[nt][v], dec, st[(int64_t)u * (NTN * 1024) + nt * 1024 + v * 64]);
-            }
+                for (int v = 0; v < 16; ++v)
+                    hacc[nt][v] = __builtin_fmaf(hacc[nt][v], dec, st[(int64_t)u * (NTN * 1024) + nt * 1024 + v * 64]);
         }
+    } else {
+        ssd2_h0<NTN>(p, b, h, p0, lane0, hacc);
     }
 
     const bf16_t* xhead = (const bf16_t*)p.x + (int64_t)b * p.x_sb + (int64_t)h * p.x_sh + p0;
@@ -690,8 +703,8 @@ __global__ __launch_bounds__(64 * HPW, HPW >= 5 ? 1 : 8 / HPW) void ssd2_scan_wu
 }
 
 // ------------------------------------------------- segment states (K3 + K4) --
-// The state of each segment but the last from zero, one wave per (batch, head,
-// 32-wide headdim half, segment): the scan's state recurrence alone, with the
+// The end state of each segment but the last, one wave per (batch, head, 32-wide
+// headdim half, segment): the scan's state recurrence alone, with the
 // chunk's whole decay applied to the accumulators (xg_j = x_j dt_j exp(cs_end -
 // cs_j) <= x_j dt_j).  Waves share nothing, so there is no barrier; the B
 // fragments come straight from L2 as MFMA operands, a chunk ahead.
@@ -735,10 +748,21 @@ __global__ __launch_bounds__(256, 2) void ssd2_seg_state(Ssd2Params p, const bf1
         for (int f = 0; f < NB; ++f) bq[f] = *(const uint4*)(gfrag + (int64_t)cc * grp_stride + f * 512);
     };
     f32x16_t hacc[NTN];
-#pragma unroll
-    for (int nt = 0; nt < NTN; ++nt) hacc[nt] = zero16();
+    const int64_t bh = (int64_t)b * p.H + h;
+    float* const states = sg.state + (bh * 2 + ph) * sg.S * (NTN * 1024) + lane;
     float total = 0.f;
     fetch(c0);
+    if (s == 0 && (p.h0 || p.init_hpr)) {
+        ssd2_h0<NTN>(p, b, h, p0, lane, hacc);
+        float* out = states + (int64_t)(sg.S - 1) * (NTN * 1024);
+#pragma unroll
+        for (int nt = 0; nt < NTN; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) out[nt * 1024 + v * 64] = hacc[nt][v];
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < NTN; ++nt) hacc[nt] = zero16();
+    }
     for (int c = c0; c < c1; ++c) {
         const float cs2 = wave_incl_scan(dtq * A2);
         const float end = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cs2), 63));
@@ -775,8 +799,7 @@ __global__ __launch_bounds__(256, 2) void ssd2_seg_state(Ssd2Params p, const bf1
             for (int nt = 0; nt < NTN; ++nt) hacc[nt] = mfma32x32x16(as_bf16x8(bc[nt * KS + ks]), bx, hacc[nt]);
         }
     }
-    const int64_t bh = (int64_t)b * p.H + h;
-    float* out = sg.state + ((bh * 2 + ph) * sg.S + s) * (NTN * 1024) + lane;
+    float* out = states + (int64_t)s * (NTN * 1024);
 #pragma unroll
     for (int nt = 0; nt < NTN; ++nt)
 #pragma unroll
