@@ -31,7 +31,7 @@ struct SsdF32BwdParams {
     bool vec;              // every output is 16-byte aligned
     // workspace
     float* hs;             // [b h][chunk][tile][16][64] states entering the chunks
-    float* fs; float* gs;  // [b h][S][n][p] segment-local states and state gradients
+    float* fs; float* gs;  // [b h][S][n][p] segments' states and state gradients (0: dfin)
     float* fd; float* gd;  // [b h][S] segment log2-decays
     float* pA; float* pD;  // [b h][S] partial dA, dD (Mamba-2)
 };

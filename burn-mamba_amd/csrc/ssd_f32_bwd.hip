@@ -138,7 +138,10 @@ __device__ __forceinline__ FDecay fb_decay(const SsdF32BwdParams& p, const FBTab
 
 // The state entering segment s as [n][p] tiles (columns p on lanes), or as
 // [p][n] tiles (columns n): four consecutive values of the row axis per load.
-// Horner over the earlier segments (h), or over the later ones (g).
+// Horner over the earlier segments (h), or over the later ones (g).  Of several
+// segments the first launch alone reads d(final state), and copies it into the
+// place of segment 0, which has no gradient of its own there: d(initial state),
+// written by the last launch, may be the same memory.
 template <int N, bool PN>
 __device__ __forceinline__ void fb_entry(const SsdF32BwdParams& p, const FBJob& j, bool grad, int pt, int nt, int i32,
                                          int hf, bwd_f32x16& a) {
@@ -150,7 +153,7 @@ __device__ __forceinline__ void fb_entry(const SsdF32BwdParams& p, const FBJob& 
     // h0 and dfin are [p][n]; segments [n][p]
     const int lp = 32 * pt + (PN ? 4 * hf : i32), ln = 32 * nt + (PN ? i32 : 4 * hf);
     if (h0) {
-        const float* q = h0 + j.bh * (kBP * N) + lp * N + ln;
+        const float* q = (grad && p.S > 1 ? p.gs + j.bh * p.S * (kBP * N) : h0 + j.bh * (kBP * N)) + lp * N + ln;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int k = 8 * (r >> 2) + (r & 3);
@@ -180,7 +183,7 @@ struct FBSegLds {
 
 // One workgroup per (batch, head, segment, direction): blocks of direction 0
 // form the state of segments 0 .. S - 2 from zero, those of direction 1 the
-// state gradient entering (from the right) segments 1 .. S - 1.
+// state gradient that segments 1 .. S - 1 hand to the left, from zero.
 template <int N, typename T>
 __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
     __shared__ __align__(16) FBSegLds<N> S;
@@ -222,7 +225,18 @@ __global__ __launch_bounds__(256, 3) void ssd_f32_bwd_seg(SsdF32BwdParams p) {
     const int nc = j.c1 - j.c0;
     auto at = [&](int k) { return rev ? j.c1 - 1 - k : j.c0 + k; };
     fetch(at(0));
-    commit(at(0));
+    if (rev && j.s == p.S - 1 && p.dfin) {
+        const float* in = p.dfin + j.bh * (kBP * N) + tid;
+        float* to = p.gs + j.bh * p.S * (kBP * N) + tid;
+        float v[kBP * N / NT];
+#pragma unroll
+        for (int e = 0; e < kBP * N / NT; ++e) v[e] = in[e * NT];
+        commit(at(0));
+#pragma unroll
+        for (int e = 0; e < kBP * N / NT; ++e) to[e * NT] = v[e];
+    } else {
+        commit(at(0));
+    }
     __syncthreads();
     float total = 0.f;
     for (int k = 0; k < nc; ++k) {

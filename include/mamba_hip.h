@@ -165,7 +165,7 @@ typedef struct mamba_ssd2_bwd_args {
     float* dB;                                       /* [b, l, g, n] contiguous */
     float* dC;                                       /* [b, l, g, n] contiguous */
     float* dD;                                       /* [h] or NULL            */
-    float* d_initial_state;                          /* [b, h, p, n]           */
+    float* d_initial_state;                 /* [b, h, p, n]; may be d_final_state */
 } mamba_ssd2_bwd_args;
 
 /* Workspace bytes (chunk states, per-head dB / dC when ngroups < nheads,     */
@@ -297,7 +297,7 @@ typedef struct mamba_ssd3_bwd_args {
     float* dscale;                                                /* [b, l, h] or NULL    */
     float* dB;                                                    /* [b, l, m, g, n] contiguous */
     float* dC;                                                    /* [b, l, m, g, n] contiguous */
-    float* d_initial_state;                                       /* [b, h, p, n]         */
+    float* d_initial_state;                     /* [b, h, p, n]; may be d_final_state   */
 } mamba_ssd3_bwd_args;
 
 /* Workspace bytes (chunk states; per-head dB / dC when ngroups < nheads);     */

@@ -1,6 +1,6 @@
-"""final_state may be the memory of initial_state: a cache updated in place.  Where a
-sequence is split into segments that run side by side, the last one writes while
-others still start; the result is bit for bit that of separate tensors.  Each
+"""final_state may be the memory of initial_state (a cache updated in place), and
+d_initial_state that of d_final_state.  Where a sequence is split into segments
+that run side by side, one writes while others still start; the result is bit for bit that of separate tensors.  Each
 case is sized to split, which its workspace or its rounding shows."""
 
 import ctypes
@@ -92,3 +92,55 @@ def test_ssd2_bf16(case, hpr):
     assert not torch.equal(hT, split[1])
     _in_place(lambda h0, hT: mamba_hip.ssd2_fwd(t["x"], t["dt"], t["A"], t["B"], t["C"], t["D"], h0, add, chunk_len=q,
                                                 final_state=hT), t["h0"])
+
+
+# (b, l, h, n): segments of one chunk and of several
+@pytest.mark.parametrize("case", [(1, 1000, 2, 64), (2, 2500, 6, 128)])
+def test_ssd2_bwd(case):
+    import torch
+    from mamba_hip import _lib
+    from mamba_hip.ssd import _stream
+    b, l, h, n = case
+    p = 64
+    rng = np.random.default_rng(l)
+    r = lambda *s: _dev(rng.standard_normal(s, dtype=np.float32))  # noqa: E731
+    t = dict(dy=r(b, l, h, p), x=r(b, l, h, p), dt=_dev(rng.uniform(0.01, 0.3, (b, l, h)).astype(np.float32)),
+             A=-torch.ones(h, device="cuda"), B=r(b, l, 1, n) / 8, C=r(b, l, 1, n) / 8, initial_state=r(b, h, p, n))
+    dF = r(b, h, p, n)
+    a = _lib.Ssd2BwdArgs()
+    a.batch, a.seqlen, a.nheads, a.headdim, a.ngroups, a.dstate = b, l, h, p, 1, n
+    for k in ("x", "dy"):
+        for nm, v in (("sb", l * h * p), ("sl", h * p), ("sh", p)):
+            setattr(a, f"{k}_{nm}", v)
+    for k in ("B", "C"):
+        for nm, v in (("sb", l * n), ("sl", n), ("sg", n)):
+            setattr(a, f"{k}_{nm}", v)
+    a.dt_sb, a.dt_sl, a.dt_sh = l * h, h, 1
+    for k, v in t.items():
+        setattr(a, k, v.data_ptr())
+    L = _lib.lib()
+
+    def run(d_final, d_initial, nbytes):
+        out = {k: torch.empty_like(t[s]) for k, s in (("dx", "x"), ("ddt", "dt"), ("dA", "A"), ("dB", "B"), ("dC", "C"))}
+        for k, v in out.items():
+            setattr(a, k, v.data_ptr())
+        a.d_final_state, a.d_initial_state = d_final.data_ptr(), d_initial.data_ptr()
+        _lib.check(L.mamba_ssd2_bwd(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), nbytes, _stream("cuda")), "bwd")
+        torch.cuda.synchronize()
+        return dict(out, dh0=d_initial)
+
+    for k in ("dx", "ddt", "dA", "dB", "dC", "d_initial_state"):  # the size query wants every pointer
+        setattr(a, k, dF.data_ptr())
+    full = L.mamba_ssd2_bwd_workspace_size(ctypes.byref(a))
+    ws = torch.empty(full, dtype=torch.uint8, device="cuda")
+    want = run(dF, torch.empty_like(dF), full)
+    cache = dF.clone()
+    got = run(cache, cache, full)
+    for k in want:
+        assert torch.equal(got[k], want[k]), k
+    # the SIMT kernels' size (a state per 32 positions, dB and dC per head, partial
+    # sums) holds fewer segments: rounded elsewhere, so that full does split
+    nch = -(-l // 32)
+    fewer = (b * h * nch * p * n + 2 * b * l * h * n) * 4 + 4 * 256 + 2 * b * h * 4
+    assert fewer < full
+    assert not torch.equal(run(dF, torch.empty_like(dF), fewer)["dx"], want["dx"])
