@@ -40,17 +40,11 @@ def _stream(device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-_WS = {}
-
-
 def workspace(device, nbytes: int) -> torch.Tensor:
-    """A cached per-device byte buffer of at least ``nbytes`` (stream-ordered use)."""
-    key = str(device)
-    buf = _WS.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
-        _WS[key] = buf
-    return buf
+    """A byte buffer for one call on the current stream.  Allocated for each: calls
+    on several streams or threads, and graphs that hold the address, share none,
+    and torch's allocator hands the memory on in stream order."""
+    return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
 
 
 def _check_inner(t: torch.Tensor, name: str):
