@@ -389,8 +389,15 @@ static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, bool bf16, void* workspace
     BwdLayout lay;
     const int st = bwd_validate(a, &lay);
     if (st != MAMBA_OK) return st;
-    if (workspace == nullptr || workspace_bytes < lay.total || ((uintptr_t)workspace & 255u) != 0) {
-        set_error("mamba_ssd2_bwd: a 256-byte aligned workspace of mamba_ssd2_bwd_workspace_size() bytes is required");
+    SsdF32BwdParams f;
+    if (bf16 && !bwd_f32_params(a, true, SIZE_MAX, &f)) {
+        set_error("mamba_ssd2_bwd_bf16: these shapes or layouts are not covered (use mamba_ssd2_bwd on f32)");
+        return MAMBA_ERR_UNSUPPORTED;
+    }
+    // with a workspace too small for the MFMA kernels the SIMT ones serve f32
+    const bool mfma = bwd_f32_params(a, bf16, workspace_bytes, &f);
+    if (workspace == nullptr || (!mfma && (bf16 || workspace_bytes < lay.total)) || ((uintptr_t)workspace & 255u) != 0) {
+        set_error("mamba_ssd2_bwd: a 256-byte aligned workspace of the *_workspace_size() bytes is required");
         return MAMBA_ERR_WORKSPACE;
     }
     Ssd2BwdParams p;
@@ -419,14 +426,10 @@ static int ssd2_bwd_run(const mamba_ssd2_bwd_args* a, bool bf16, void* workspace
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid(a->batch * a->nheads);
     p.npart = 1;
-    SsdF32BwdParams f;
-    if (bwd_f32_params(a, bf16, workspace_bytes, &f)) {
+    if (mfma) {
         const int fst = ssd_f32_bwd_launch(f, workspace, s, ev0, ev1);
         if (fst != MAMBA_OK) return fst;
         p.dBh = f.dBh; p.dCh = f.dCh; p.pA = f.pA; p.pD = f.pD; p.npart = f.S;
-    } else if (bf16) {
-        set_error("mamba_ssd2_bwd_bf16: these shapes, layouts or this workspace are not covered (use mamba_ssd2_bwd on f32)");
-        return MAMBA_ERR_UNSUPPORTED;
     } else {
         // dynamic LDS above the 64 KB default (up to the CU's 160 KB)
         MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd2_bwd_states, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -461,7 +464,7 @@ extern "C" size_t mamba_ssd2_bwd_bf16_workspace_size(const mamba_ssd2_bwd_args* 
     BwdLayout lay;
     if (bwd_validate(a, &lay) != MAMBA_OK) return 0;
     SsdF32BwdParams f;
-    return bwd_f32_params(a, true, SIZE_MAX, &f) ? std::max(lay.total, ssd_f32_bwd_workspace(f)) : 0;
+    return bwd_f32_params(a, true, SIZE_MAX, &f) ? ssd_f32_bwd_workspace(f) : 0;
 }
 
 extern "C" int mamba_ssd2_bwd_bf16(const mamba_ssd2_bwd_args* a, void* workspace, size_t workspace_bytes,
