@@ -292,12 +292,12 @@ def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
 
 
 def _mm_f32_takes(*ts: torch.Tensor) -> bool:
-    """Plain f32 tensors with a unit stride that no transform of the product's
-    operands (reverse or forward mode, vmap) has to see."""
-    return all(t.dtype == torch.float32 and 1 in t.stride()[-2:] and type(t) in (torch.Tensor, torch.nn.Parameter)
+    """Plain f32 tensors with values and a unit stride that no transform of the
+    product's operands (reverse or forward mode, vmap, autocast) has to see."""
+    return all(t.dtype == torch.float32 and t.numel() and 1 in t.stride()[-2:] and type(t) in (torch.Tensor, torch.nn.Parameter)
                and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts) and \
         not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)) and \
-        torch.autograd.forward_ad._current_level < 0
+        torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda")
 
 
 def _wt(w: torch.Tensor, attr: str, col0: int) -> torch.Tensor:

@@ -7,7 +7,7 @@ import torch
 
 import mamba_hip
 from mamba_hip import _lib
-from mamba_hip.mamba1 import mm_f32
+from mamba_hip.mamba1 import _mm_f32_takes, mm_f32
 from mamba_hip.step import linear_row
 
 
@@ -40,6 +40,17 @@ def test_mm_f32_types_and_rows_of_out():
         mm_f32(a, b.double())
     with pytest.raises(mamba_hip.MambaHipError, match="out"):
         mm_f32(a, b, torch.zeros(1, 4, 10)[:, :, ::2])
+
+
+def test_the_library_keeps_empty_and_autocast_products():
+    a, b = torch.zeros(4, 8), torch.zeros(8, 5)
+    assert _mm_f32_takes(a, b)
+    assert not _mm_f32_takes(a[:0], b)  # no rows: an empty product, not an error
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        assert not _mm_f32_takes(a, b)
+    finally:
+        torch.set_autocast_enabled("cuda", False)
 
 
 def test_mamba1_forward_width():
