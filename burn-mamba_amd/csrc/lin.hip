@@ -234,7 +234,7 @@ template <int NW, int EPI, bool RM, int U, int MM, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
     static_assert(!NORM || (MM == 1 && RM), "one row");
     __shared__ float s_red[NW][MM][32];
-    __shared__ __align__(16) bf16_t s_x[NORM ? kLinRowMaxK : 8];
+    __shared__ __align__(16) bf16_t s_x[NORM ? kLinRowMaxK + 16 : 8];
     __shared__ float s_ss[NORM ? NW : 1];
     const int cs = lin_parts(p);
     const int j = blockIdx.x / cs, z = blockIdx.y;
@@ -326,12 +326,14 @@ __global__ __launch_bounds__(64 * NW) void lin_gemv(LinParams p) {
                                (uint32_t)f32_to_bf16((xv[i].z / rms) * nv[i].z) |
                                    ((uint32_t)f32_to_bf16((xv[i].w / rms) * nv[i].w) << 16));
         }
+        if (threadIdx.x < 16) s_x[p.K + threadIdx.x] = 0;
         __syncthreads();
-        // k-steps past the wave's end meet zero weights: any k of the row will do
+        // k-steps past the wave's end: the zeros after the row (zero weights alone
+        // would make NaN of an infinite operand)
         auto operand = [&](Stage& st, int s) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                st.a[u][0] = *reinterpret_cast<const uint4*>(s_x + 16 * min(s + u, KS - 1) + 8 * h);
+                st.a[u][0] = *reinterpret_cast<const uint4*>(s_x + 16 * (s + u < s1 ? s + u : KS) + 8 * h);
         };
         for (int st = 0; st < nstage; st += 2) {
             const int s = s0 + U * st;

@@ -35,6 +35,26 @@ def test_linear_row(d_in, d_out, norm, accumulate):
     assert bool(((out.cpu().double() - want).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("d_in", [48, 784, 1040])
+def test_an_infinite_norm_weight_stays_in_its_products(d_in):
+    """inf times a weight that is not zero is that infinity, not the NaN of a zero
+    weight in the padding of some wave's last stage."""
+    import torch
+    from mamba_hip.step import linear_row, pack_linear
+    d_out = 70
+    g = torch.Generator().manual_seed(d_in)
+    w = (torch.rand(d_in, d_out, generator=g) + 0.5).bfloat16() * (torch.randint(0, 2, (d_out,), generator=g) * 2 - 1)
+    x = torch.rand(d_in, generator=g) + 0.5
+    packed = pack_linear(w.cuda())
+    for k in range(0, d_in, 16):
+        gam = torch.ones(d_in)
+        gam[k] = float("inf")
+        out = torch.empty(d_out, device="cuda")
+        linear_row(x.cuda(), packed, out, norm_w=gam.cuda())
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), w[k].float().sign() * float("inf")), k
+
+
 def test_linear_row_refuses():
     import torch
     import mamba_hip
