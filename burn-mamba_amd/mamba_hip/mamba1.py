@@ -262,12 +262,13 @@ def mm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None)
     # the kernel is handed pointers: what a matmul would refuse is refused here
     if b.shape != (z, k, n) or (out is not None and (out.shape != (z, m, n) or out.stride(2) != 1)):
         raise _lib.MambaHipError(f"mm_f32: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not match, or out's rows")
+    dev = a.get_device()  # below 0: not a GPU
+    if dev < 0 or b.get_device() != dev or (out is not None and out.get_device() != dev):
+        raise _lib.MambaHipError("mm_f32: operands on one GPU device required")
     if out is None:
         out = torch.empty((z, m, n), device=a.device, dtype=torch.float32)
-    if not (a.dtype == b.dtype == out.dtype == torch.float32):
+    if a.dtype != torch.float32 or b.dtype != torch.float32 or out.dtype != torch.float32:
         raise _lib.MambaHipError("mm_f32: float32 required")
-    if not (a.is_cuda and a.device == b.device == out.device):
-        raise _lib.MambaHipError(f"mm_f32: operands on {a.device}, {b.device}, {out.device}: one GPU device required")
     g = _lib.MmF32Args()
     g.batch, g.m, g.n, g.k = z, m, n, k
     g.a, (g.a_sb, g.a_sm, g.a_sk) = a.data_ptr(), a.stride()
@@ -291,13 +292,20 @@ def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
     return L <= 256 and di <= 512 and _mm_f32_takes(*ts)
 
 
+_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+
+
 def _mm_f32_takes(*ts: torch.Tensor) -> bool:
     """Plain f32 tensors with values and a unit stride that no transform of the
     product's operands (reverse or forward mode, vmap, autocast) has to see."""
-    return all(t.dtype == torch.float32 and t.numel() and 1 in t.stride()[-2:] and type(t) in (torch.Tensor, torch.nn.Parameter)
-               and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in ts) and \
-        not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)) and \
-        torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled("cuda")
+    if torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
+        return False
+    grad, f32 = torch.is_grad_enabled(), torch.float32
+    for t in ts:
+        if t.dtype != f32 or (grad and t.requires_grad) or type(t) not in (torch.Tensor, torch.nn.Parameter) or \
+                _wrapped(t) or 1 not in t.stride()[-2:] or not t.numel():
+            return False
+    return True
 
 
 def _wt(w: torch.Tensor, attr: str, col0: int) -> torch.Tensor:
