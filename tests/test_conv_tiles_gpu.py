@@ -1,7 +1,8 @@
 """The prefill conv at every tile length its launch takes (8 to 64 positions per
-workgroup), ragged ends and sequences shorter than the window, with the window
-updated in place by the first tile's workgroups, vs the oracle (f32: rtol 1e-4;
-the window holds input values: exact)."""
+workgroup) and every kernel length whose margin to the second tile differs,
+ragged ends and sequences shorter than the window, with the window updated in
+place by the first tile's workgroups, vs the oracle (f32: rtol 1e-4; the window
+holds input values: exact)."""
 
 import numpy as np
 import pytest
@@ -9,18 +10,29 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# (b, l, channels): tiles of 64, 32, 16 and 8 positions; scalar channels; l < kernel
+# (b, l, channels): tiles of 64 (twice), 32 and 8 positions; scalar channels; l < kernel
 CASES = [(8, 4101, 8), (4, 4101, 8), (2, 4101, 8), (1, 500, 16), (2, 300, 7), (3, 2, 24), (1, 1, 8)]
+# tiles of 32, 16 (the first of 8 positions) and 8, where a kernel of 8 leaves the
+# second tile one position past the old window
+KERNELS = [(2, 4101, 8), (1, 4101, 8), (1, 500, 16), (1, 4101, 7)]
 
 
 @pytest.mark.parametrize("case", CASES)
 def test_conv1d_fwd(case):
+    _check(*case, 4)
+
+
+@pytest.mark.parametrize("K", [2, 4, 8])
+@pytest.mark.parametrize("case", KERNELS)
+def test_conv1d_fwd_kernels(case, K):
+    _check(*case, K)
+
+
+def _check(b, L, c, K):
     import torch
     import mamba_hip
     import oracle
-    b, L, c = case
-    K = 4
-    rng = np.random.default_rng(sum(case))
+    rng = np.random.default_rng(b + L + c)
     x, st = rng.standard_normal((b, L, c), dtype=np.float32), rng.standard_normal((b, c, K), dtype=np.float32)
     w, bias = rng.standard_normal((c, K), dtype=np.float32), rng.standard_normal(c, dtype=np.float32)
     s = torch.from_numpy(st).cuda()

@@ -11,9 +11,10 @@ pytestmark = pytest.mark.gpu
 
 
 # (z, m, n, k): one element, ragged 32-tiles, K over 4, 8 and 16 waves with
-# ragged ends, odd rows (no 16-byte loads), 64-tiles
+# ragged ends, odd rows (no 16-byte loads), 64-tiles with odd rows and with 16-byte
+# loads up to ragged edges
 SHAPES = [(1, 1, 1, 1), (3, 33, 31, 5), (2, 48, 250, 128), (2, 48, 250, 130),
-          (2, 47, 251, 513), (1, 256, 100, 512), (5, 530, 515, 65)]
+          (2, 47, 251, 513), (1, 256, 100, 512), (5, 530, 515, 65), (4, 516, 508, 68)]
 
 
 @pytest.mark.parametrize("ta,tb", list(itertools.product([False, True], repeat=2)))
