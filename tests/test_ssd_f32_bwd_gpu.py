@@ -23,9 +23,10 @@ def _close(got, want, name):
 
 
 # (b, l, h, g, n, optional): one row, a chunk +- 1, many segments (one head),
-# per-head and grouped B / C, with and without D, h0 and d(final state)
+# segments of two chunks, per-head and grouped B / C, with and without D, h0 and
+# d(final state)
 CASES2 = [(1, 1, 2, 1, 64, True), (2, 63, 2, 2, 64, False), (1, 64, 3, 1, 128, True), (1, 65, 2, 1, 64, True),
-          (1, 700, 1, 1, 128, True), (2, 333, 4, 2, 64, True), (1, 130, 300, 1, 64, False)]
+          (1, 700, 1, 1, 128, True), (2, 333, 4, 2, 64, True), (1, 130, 300, 1, 64, False), (1, 2500, 12, 2, 64, True)]
 
 
 @pytest.mark.parametrize("case", CASES2)
@@ -49,10 +50,10 @@ def test_ssd2(case):
         _close(out["dD"], want["dD"], "dD")
 
 
-# (b, l, m, h, g, n, optional): 64 / m steps per chunk, ragged ends, the double
-# seam's unit weights (optional False)
+# (b, l, m, h, g, n, optional): 64 / m steps per chunk, ragged ends, segments of
+# two chunks, the double seam's unit weights (optional False)
 CASES3 = [(1, 33, 4, 2, 2, 64, True), (1, 3, 32, 2, 1, 64, True), (2, 100, 2, 2, 1, 128, True),
-          (1, 400, 4, 1, 1, 64, True), (1, 129, 1, 3, 3, 64, False), (1, 17, 16, 2, 2, 128, False)]
+          (1, 400, 4, 1, 1, 64, True), (1, 129, 1, 3, 3, 64, False), (1, 17, 16, 2, 2, 128, False), (1, 710, 4, 12, 1, 64, True)]
 
 
 @pytest.mark.parametrize("case", CASES3)

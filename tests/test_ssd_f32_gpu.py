@@ -24,9 +24,10 @@ def _dev(a, dtype=None):
 
 
 # (b, l, h, p, g, n): one row, a chunk +- 1, several segments (few heads, long
-# sequences), one segment (many heads), headdim blocks of 32 and of 64
+# sequences), one segment (many heads), segments of two chunks, headdim blocks of
+# 32 and of 64
 CASES2 = [(1, 1, 2, 64, 1, 64), (1, 63, 4, 32, 2, 32), (2, 64, 2, 96, 1, 64), (1, 65, 2, 128, 2, 128),
-          (1, 1500, 3, 64, 1, 128), (2, 640, 5, 192, 5, 32), (2, 130, 160, 64, 1, 64)]
+          (1, 1500, 3, 64, 1, 128), (2, 640, 5, 192, 5, 32), (2, 130, 160, 64, 1, 64), (1, 4700, 3, 64, 1, 64)]
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
@@ -56,9 +57,10 @@ def test_ssd2(case, dtype):
     np.testing.assert_allclose(hT.cpu().numpy(), hr, **F32_TOL)
 
 
-# (b, l, m, h, p, n): ranks that fill a chunk with 64 / m steps, ragged ends
+# (b, l, m, h, p, n): ranks that fill a chunk with 64 / m steps, ragged ends,
+# segments of two chunks
 CASES3 = [(1, 33, 4, 2, 64, 64), (2, 15, 4, 2, 32, 128), (1, 300, 2, 3, 64, 128), (1, 3, 64, 2, 64, 64),
-          (1, 257, 1, 4, 128, 32), (1, 70, 16, 2, 64, 128)]
+          (1, 257, 1, 4, 128, 32), (1, 70, 16, 2, 64, 128), (1, 710, 4, 12, 64, 128)]
 
 
 @pytest.mark.parametrize("double", [False, True])
