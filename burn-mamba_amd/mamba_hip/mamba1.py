@@ -278,7 +278,7 @@ def mm_f32(a: torch.Tensor, b: torch.Tensor, out: Optional[torch.Tensor] = None)
     return out
 
 
-def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
+def _mm_f32_pays(di: int, b: int, L: int, *ts: torch.Tensor) -> bool:
     """Where mamba_mm_f32 takes a block's products.  For at most 256
     tokens per sequence and 512 channels the library picks 256-wide tiles (2 x 256
     tokens, 512 channels: out_proj 118 us, x_proj 25 us against 7.9 and 7.5; 1 x
@@ -287,9 +287,14 @@ def _mm_f32_pays(di: int, L: int, *ts: torch.Tensor) -> bool:
     and more: 8.6 against 11.8).  dt_proj (K = dt_rank) takes the same time in either
     (3.7 to 5 us) and in_proj up to 512 tokens in all (2 x 256: 5.2 against 5.2 and
     5.8; 3 x 256: 7.2 against 6.7 and 5.7), for 9 us less of the host per call, which
-    is what bounds a block of this size.  Calls that autograd follows, and operands
-    without a unit stride, stay with the library."""
-    return L <= 256 and di <= 512 and _mm_f32_takes(*ts)
+    is what bounds a block of this size.  Up to 128 sequences: the library's tiles
+    fill the chip as they become many (512 channels, the whole block and, in
+    brackets, the three products on the GPU, against the library's: 64 x 256 280 and
+    372 [87, 169], 128 x 256 496 and 544 [142, 179], 256 x 256 927 and 884 [264,
+    197]; 64 x 8 tokens 109 and 172 [32, 25], 128 x 8 143 and 172 [42, 25], 512 x 8
+    250 and 177 [130, 51]).  Calls that autograd follows, and operands without a unit
+    stride, stay with the library."""
+    return b <= 128 and L <= 256 and di <= 512 and _mm_f32_takes(*ts)
 
 
 _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
@@ -355,7 +360,7 @@ class Mamba1:
         di, r, n = c.d_inner, c.dt_rank, c.state_rank
         xf = x.float()
         x2 = xf.reshape(b * L, dm)
-        own = _mm_f32_pays(di, L, self.in_proj_w, self.x_proj_w, self.dt_proj_w, self.out_proj_w, xf)
+        own = _mm_f32_pays(di, b, L, self.in_proj_w, self.x_proj_w, self.dt_proj_w, self.out_proj_w, xf)
         # The scan streams u, delta, z and y as time-contiguous rows [b, d, l]
         # (its tuned kernel reads 32-token tiles of whole 128-byte lines), so
         # the products around it are formed in that layout: z and delta as

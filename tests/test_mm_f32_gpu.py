@@ -53,6 +53,25 @@ def test_out_mm_on_both_sides_of_its_rule(rows, di, dm):
     np.testing.assert_allclose(out.cpu().numpy(), (y.double() @ w.double()).numpy(), rtol=1e-4, atol=1e-5 * di ** 0.5)
 
 
+def test_mamba1_block_on_both_sides_of_its_batch_rule(monkeypatch):
+    """128 sequences on the own product, 129 on the library: the same rows."""
+    import torch
+    import mamba_hip
+    from mamba_hip import mamba1
+    calls = []
+    own = mamba1.mm_f32
+    monkeypatch.setattr(mamba1, "mm_f32", lambda *a: calls.append(1) or own(*a))
+    m = mamba_hip.Mamba1Config(64).init("cuda", torch.Generator(device="cuda").manual_seed(2))
+    x = torch.randn(129, 9, 64, generator=torch.Generator().manual_seed(3)).cuda()
+    y, cache = m.forward(x[:128])
+    assert calls
+    n = len(calls)
+    z, cache2 = m.forward(x)
+    assert len(calls) == n
+    torch.testing.assert_close(y, z[:128], rtol=1e-4, atol=1e-5)
+    torch.testing.assert_close(cache.ssm_bir, cache2.ssm_bir[:128], rtol=1e-4, atol=1e-5)
+
+
 def test_out_mm_under_autograd_and_forward_mode():
     import torch
     import torch.autograd.forward_ad as fw
