@@ -312,16 +312,18 @@ __global__ __launch_bounds__(NT) void mamba3_step_kernel(M3StepParams p) {
 }
 
 // 512 threads per workgroup where the launch has at most one workgroup per CU
-// (two at rank 4): the CU has nothing else to hide the step's serial chain of
-// loads, norms and readout behind.  us per step at state 64 x 128, 256 against
-// 512 threads, by workgroups: rank 4, 32: 8.05 / 6.92, 256: 9.2 / 8.2, 512: 11.7 /
-// 11.0, 768: 14.5 / 16.6; rank 1, 32: 5.5 / 5.1, 256: 7.4 / 7.1, 384: 8.4 / 8.9;
-// rank 8, 32: 10.5 / 8.8, 256: 12.7 / 10.6, 384: 15.0 / 17.6.  (1024 threads: a
-// further 0.2 us below 256 workgroups up to rank 4, far slower above.)
+// (two at rank 4, for states of 2048 values or more): the CU has nothing else to
+// hide the step's serial chain of loads, norms and readout behind.  us per step at
+// state 64 x 128, 256 against 512 threads, by workgroups: rank 4, 32: 8.05 / 6.92,
+// 256: 9.2 / 8.2, 512: 11.7 / 11.0, 768: 14.5 / 16.6; rank 1, 32: 5.5 / 5.1, 256:
+// 7.4 / 7.1, 384: 8.4 / 8.9; rank 2, 32: 6.5 / 5.9, 256: 7.7 / 7.3, 384: 9.1 / 9.3;
+// rank 8, 32: 10.5 / 8.8, 256: 12.7 / 10.6, 384: 15.0 / 17.6.  Rank 4, 512: state 16
+// x 16 5.0 / 5.4, 32 x 32 5.2 / 5.6, 32 x 64 6.0 / 6.0, 64 x 64 7.2 / 7.1.  (1024
+// threads: a further 0.2 us below 256 workgroups up to rank 4, far slower above.)
 template <int N4, int MM>
 static void m3_launch_nt(const M3StepParams& p, hipStream_t s) {
     const int grid = p.nb * p.H;
-    if (grid <= (MM == 4 ? 512 : 256))
+    if (grid <= (MM == 4 && p.P * 4 * N4 >= 2048 ? 512 : 256))
         hipLaunchKernelGGL((mamba3_step_kernel<N4, MM, 512>), dim3(grid), dim3(512), 0, s, p);
     else
         hipLaunchKernelGGL((mamba3_step_kernel<N4, MM, 256>), dim3(grid), dim3(256), 0, s, p);
