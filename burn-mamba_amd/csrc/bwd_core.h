@@ -46,11 +46,5 @@ __device__ __forceinline__ float bwd_half_sum16(const float (&v)[16], int i32) {
     const float z = (b1 ? y[1] : y[0]) + bwd_xor2(b1 ? y[0] : y[1]);
     return z + bwd_xor1(z);
 }
-__device__ __forceinline__ void bwd_put4(float* dst, float4 v) {
-    dst[0] = v.x;
-    dst[1] = v.y;
-    dst[2] = v.z;
-    dst[3] = v.w;
-}
 
 }  // namespace mamba

@@ -409,10 +409,12 @@ bool ssd_f32_plan(SsdF32Params* q) {
     p.mshift = __builtin_ctz(p.M);
     const int64_t steps = kFR >> p.mshift;
     p.nch = (int)((p.L + steps - 1) / steps);
-    // Segments per (batch, head, block): the scan takes rounds of 256
-    // workgroups (one per CU: 87-142 KB of LDS), each as long as a segment's
-    // chunks plus the entry state; the state pass half a chunk's time per chunk
-    // at two workgroups per CU and another launch (about half a chunk's time).
+    // Segments per (batch, head, block): the scan takes rounds of 256 workgroups
+    // (one per CU at dstate 64 and 128, by 75 to 143 KB of LDS and up to 240
+    // registers; at dstate 32, 53 to 66 KB, two fit, which is not counted), each as
+    // long as a segment's chunks plus the entry state; the state pass half a chunk's
+    // time per chunk at two workgroups per CU and another launch (about half a
+    // chunk's time).
     const int64_t units = (int64_t)p.nb * p.H * (p.P / f_pblock(p));
     double best = 0.;
     for (int n = 1; n <= std::min(p.nch, 64); ++n) {
