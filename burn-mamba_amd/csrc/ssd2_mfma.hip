@@ -855,14 +855,17 @@ static size_t seg_bytes(const Ssd2Params& p, int S) {
 // of a group) and segments per sequence.  The scan's LDS (two chunks of group
 // fragments) allows one workgroup per CU, so a launch of nwg workgroups takes
 // ceil(nwg / 256) rounds on MI355X's 256 CUs, each as long as a segment's
-// chunks; five waves share four SIMDs, which costs a chunk about a fifth.  In
-// units of a chunk (about 4.5 us): a segment adds its entry state (0.5 and 0.1
-// per earlier segment) and the state pass a third of a chunk per chunk for
-// every 2048 waves, and a launch (1).  Measured at 80 heads x 64 x 128: batch 1,
-// 3001 positions 191 -> 73 us, batch 2 x 2048 (the forward of a training
-// step) 160 -> 87 us; batch 8 x 4096 fills the chip and stays whole.  Ties
-// go to the larger head set, which stages each fragment for more heads, and to
-// fewer segments.  MAMBA_SSD2_HPW (read on every call) forces a valid head set.
+// chunks; five waves share four SIMDs, which costs a chunk about a fifth.  A
+// chunk takes 1.1 / 2.0 us at dstate 64 (32 / 64 positions) and 1.3 / 2.4 at 128.
+// Splitting adds a launch, 0.24 / 0.31 us of entry state per segment, the state
+// pass (a chunk's time per chunk for every 2048 waves) and the states' bytes: each
+// segment's written and read, and read again by every later one.  These were fitted
+// to 372 calls of 1 to 4 sequences of 65 to 2600 positions, 1 to 80 heads, whole
+// and split (5 to 6 % rms).  Measured at 80 heads x 64 x 128, whole against
+// split: 1 x 3001 positions 191 / 73 us, 2 x 2048 160 / 87, 1 x 400 25.9 / 31.2 and 2
+// x 200 19.5 / 28.9 (whole); 8 x 4096 fills the chip and stays whole.  Ties go to the
+// larger head set, which stages each fragment for more heads, and to fewer
+// segments.  MAMBA_SSD2_HPW (read on every call) forces a valid head set.
 struct Ssd2Plan {
     int hpw, S, cps;
 };
@@ -874,6 +877,9 @@ static Ssd2Plan choose_plan(const Ssd2Params& p, size_t ws_bytes) {
         if ((v == 1 || v == 2 || v == 4 || v == 5) && hpg % v == 0) forced = v;
     }
     constexpr int kCUs = 256;
+    const bool n128 = p.N == 128, q64 = p.Q == 64;
+    const double chunk_us = n128 ? (q64 ? 2.4 : 1.3) : (q64 ? 2.0 : 1.1);
+    const double launch_us = n128 ? (q64 ? 2.9 : 4.2) : (q64 ? 2.0 : 2.5), entry_us = n128 ? 0.31 : 0.24;
     Ssd2Plan best{1, 1, p.nch};
     double best_cost = 0.;
     for (int hpw : {5, 4, 2, 1}) {
@@ -884,9 +890,11 @@ static Ssd2Plan choose_plan(const Ssd2Params& p, size_t ws_bytes) {
             if (S != n || (S > 1 && frag_bytes(p) + seg_bytes(p, S) > ws_bytes)) continue;
             const int64_t rounds = (nwg * S + kCUs - 1) / kCUs;
             const int64_t pass = ((int64_t)p.nb * p.H * 2 * (S - 1) + 2047) / 2048;
-            const double chunk = hpw == 5 ? 1.2 : 1.;
-            const double cost =
-                rounds * chunk * (cps + (S > 1 ? 0.5 + 0.1 * S : 0.)) + (S > 1 ? pass * 0.33 * cps + 1. : 0.);
+            double cost = (double)rounds * cps * (hpw == 5 ? 1.2 : 1.) * chunk_us;
+            if (S > 1) {
+                const double mb = (double)p.nb * p.H * 64 * p.N * 4e-6 * ((S - 1) * S * 0.5 + 2. * (S - 1));
+                cost += launch_us + entry_us * S + chunk_us * (double)pass * cps + 0.1 * mb;
+            }
             if (best_cost == 0. || cost < best_cost) {
                 best_cost = cost;
                 best = {hpw, S, cps};
