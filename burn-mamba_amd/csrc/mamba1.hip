@@ -581,16 +581,31 @@ static bool tm16_aligned(const Mamba1Params& p) {
            p.dl_sb % 4 == 0 && p.y_sb % 4 == 0 && (!p.z || p.z_sb % 4 == 0);
 }
 
+// Rows at odd addresses, which take a word per direct-to-LDS load, long
+// enough: mamba1_scan_kernel's 16-token tiles waste less on a last half-tile.
+// us there against here: 1 x 5120 channels, 7 tokens 5.1 / 6.7, 15 5.1 / 6.8, 31 7.6 /
+// 7.1, 33 9.9 / 10.0, 49 12.2 / 9.9, 65 15.0 / 13.1; 8 x 5120, 15 7.5 / 10.7, 33 15.0 /
+// 18.3, 49 19.4 / 19.0, 65 23.6 / 25.1, 97 32.1 / 32.1.
+static bool tm16_pays(const Mamba1Params& p) {
+    if (tm16_aligned(p)) return true;
+    const bool half = (p.L - 1) % kTm16Tile < kTm16Tile / 2;  // the last tile
+    const int64_t nblk = (int64_t)p.nb * ((p.D + 63) / 64);
+    return !(half && p.L <= (nblk >= 512 ? 80 : 48));
+}
+
 // Time segments: none where (batch row, 64 channels) already gives a workgroup to
-// most CUs, else about 1280 workgroups (five per CU, three resident: the state pass
-// is half of the second one's work, and its chain is short), at least a tile each.
-// us whole / so split: 24 workgroups, 256 tokens 25.6 / 12.0, 2048 184 / 32; 40,
-// 1504: 136 / 38; 80, 2048: 185 / 77; 160, 2048: 180 / 146; 200, 2048: 180 / 185;
-// 320, 1024: 145 / 138; 480, 1024: 154 / 195.
+// most CUs or the sequence is a few tiles, else about 1280 workgroups (five per CU,
+// three resident: the state pass is half of the second one's work, and its chain is
+// short), at least a tile each.  us whole / so split: 24 workgroups, 64 tokens 8.6 /
+// 10.5, 96 11.3 / 10.8, 256 24.9 / 11.6, 2048 186 / 33; 80, 96 11.5 / 11.0, 2048 184 / 76;
+// 100, 96 11.5 / 13.0, 128 14.2 / 15.0, 160 17.0 / 15.6; 160, 256 26.5 / 28.0, 320 32.6 /
+// 32.7, 384 38.2 / 36.2, 2048 180 / 140; 200, 2048 180 / 185; 320, 1024 145 / 138; 480,
+// 1024 154 / 195.
 static int m1_segments(const Mamba1Params& p) {
     const int tiles = (p.L + kTm16Tile - 1) / kTm16Tile;
     const int64_t nblk = (int64_t)p.nb * ((p.D + 63) / 64);
-    return nblk > 160 ? 1 : (int)std::min<int64_t>(tiles, 1280 / nblk);
+    const int least = nblk <= 80 ? 3 : nblk <= 128 ? 5 : 11;
+    return nblk > 160 || tiles < least ? 1 : (int)std::min<int64_t>(tiles, 1280 / nblk);
 }
 // workspace bytes of one segment
 static size_t m1_seg_bytes(const Mamba1Params& p) { return (size_t)p.nb * p.D * (16 + 1) * 4; }
@@ -638,7 +653,7 @@ static int m1_dispatch(const mamba1_scan_args* a, void* ws, size_t ws_bytes, hip
     MAMBA_CHECK_ARG(((uintptr_t)ws & 15u) == 0, "the workspace must be 16-byte aligned");
     int nfast = m1_tiled(p) ? p.N : 0;
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
-    if (nfast == 16 && tm16_ok(p)) {
+    if (nfast == 16 && tm16_ok(p) && tm16_pays(p)) {
         const bool al = tm16_aligned(p);
         if (p.z) al ? launch_tm16<true, true>(p, ws, ws_bytes, stream) : launch_tm16<true, false>(p, ws, ws_bytes, stream);
         else al ? launch_tm16<false, true>(p, ws, ws_bytes, stream) : launch_tm16<false, false>(p, ws, ws_bytes, stream);
@@ -665,7 +680,7 @@ using namespace mamba;
 
 extern "C" size_t mamba1_scan_workspace_size(const mamba1_scan_args* a) {
     Mamba1Params p;
-    if (m1_make_params(a, &p) != MAMBA_OK || !m1_tiled(p) || !tm16_ok(p)) return 0;
+    if (m1_make_params(a, &p) != MAMBA_OK || !m1_tiled(p) || !tm16_ok(p) || !tm16_pays(p)) return 0;
     const int nseg = m1_segments(p);
     return nseg > 1 ? nseg * m1_seg_bytes(p) : 0;
 }

@@ -47,3 +47,20 @@ def test_segments_match_oracle(l, ws, gate, monkeypatch):
     np.testing.assert_allclose(y.cpu().numpy(), yr, **TOL)
     np.testing.assert_allclose(hT.cpu().numpy(), hr, **TOL)
     assert hT.data_ptr() == state.data_ptr()
+
+
+# rows at odd addresses on both sides of the rule between the two tiled kernels:
+# last half-tiles up to 48 tokens, and up to 80 where the launch is large
+@pytest.mark.parametrize("b,d,l", [(2, 70, 1), (2, 70, 15), (2, 70, 17), (1, 70, 33), (1, 70, 47), (1, 70, 49),
+                                   (1, 70, 65), (8, 4100, 49), (8, 4100, 65), (8, 4100, 79), (8, 4100, 81)])
+def test_odd_rows_match_oracle(b, d, l):
+    import torch
+    import mamba_hip
+    import oracle
+    inp = mamba1_inputs(seed=l, b=b, d=d, l=l, n=16, h0=True)
+    t = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in inp.items()}
+    y, hT = mamba_hip.mamba1_scan(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], initial_state=t["h0"])
+    torch.cuda.synchronize()
+    yr, hr = oracle.mamba1_scan(inp["u"], inp["delta"], inp["A"], inp["B"], inp["C"], inp["D"], h0=inp["h0"])
+    np.testing.assert_allclose(y.cpu().numpy(), yr, **TOL)
+    np.testing.assert_allclose(hT.cpu().numpy(), hr, **TOL)
