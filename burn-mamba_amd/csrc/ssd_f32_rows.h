@@ -23,8 +23,11 @@ struct FDecay {
     float end;   // the whole chunk's, in log2 units
 };
 __device__ __forceinline__ float f_exp(float x) { return __builtin_amdgcn_exp2f(x); }
-// x: the row's log-decay
+// x: the row's log-decay.  At the least -2^14, whose exp is 0 as that of all below: a
+// mask's lowest value or -inf, kept, would make the sums infinite in log2 units and
+// every difference after it NaN (a NaN stays one).
 __device__ __forceinline__ FDecay f_decay(double x) {
+    x = x < -16384. ? -16384. : x;
     const double cs = wave_incl_scan64(x * kFLog2e), end = wave_lane64(cs, 63);
     FDecay d;
     d.cs = (float)cs;

@@ -106,6 +106,31 @@ def test_ssd2_decays_after_a_reset(l, h):
         assert err < 2e-6, (k, err)
 
 
+@pytest.mark.parametrize("low", [np.finfo(np.float32).min, -np.inf])
+@pytest.mark.parametrize("l", [40, 400])
+def test_ssd3_decays_of_the_lowest_value(l, low):
+    """Steps that forget everything before them, as masks set them, two of them in
+    a chunk: the gradients are those of a decay of exp(-1e4), which is 0."""
+    import torch
+    import mamba_hip
+    b, m, h, g, n, p = 1, 2, 2, 1, 64, 64
+    rng = np.random.default_rng(l)
+    r = lambda *s: rng.standard_normal(s, dtype=np.float32)  # noqa: E731
+    v, dy, B, C = r(b, l, m, h, p), r(b, l, m, h, p), r(b, l, m, g, n) / 8, r(b, l, m, g, n) / 8
+    da = -rng.uniform(0.01, 0.5, (b, l, h)).astype(np.float32)
+    gam, scl = (rng.uniform(0.01, 0.3, (b, l, h)).astype(np.float32) for _ in range(2))
+    h0, dF = 0.3 * r(b, h, p, n), r(b, h, p, n)
+    reset = np.isin(np.arange(l) % 64, (5, 21))
+    da[:, reset] = low
+    out = mamba_hip.ssd3_bwd(_t(dy), _t(v), _t(da), _t(B), _t(C), _t(gam), _t(scl), _t(h0), _t(dF))
+    torch.cuda.synchronize()
+    da[:, reset] = -1e4
+    want = oracle.ssd3_bwd(dy, dF, v, da, B, C, gam, scl, h0)
+    for k, w in (("dv", "dv"), ("dda", "dda"), ("dB", "dB"), ("dC", "dC"), ("d_initial_state", "dh0"),
+                 ("dgamma", "dgamma"), ("dscale", "dscale")):
+        _close(out[k], want[w], k)
+
+
 def test_ssd2_any_segment_count_gives_the_same_gradients():
     """A workspace that holds fewer segments (as small as the SIMT kernels', one
     entry state per 32 positions) is used with fewer; both agree to f32 rounding."""

@@ -110,6 +110,28 @@ def test_ssd2_decays_after_a_reset(l):
         assert np.linalg.norm(got - ref) < 1e-6 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("low", [np.finfo(np.float32).min, -np.inf])
+@pytest.mark.parametrize("l,h", [(40, 2), (400, 2), (400, 160)])
+def test_ssd3_decays_of_the_lowest_value(l, h, low):
+    """Steps that forget everything before them, as masks set them, two of them in
+    a chunk: their decay is 0 as exp(-1e4)'s is, and the rows after them have
+    their own.  Whole and split sequences."""
+    import torch
+    import mamba_hip
+    import oracle
+    b, m, p, n = 1, 2, 64, 64
+    inp = ssd3_inputs(l + h, b, l, m, h, p, n)
+    reset = np.isin(np.arange(l) % 64, (5, 21))
+    inp["da"][:, reset] = low
+    t = {k: _dev(v) for k, v in inp.items()}
+    y, hT = mamba_hip.ssd3_fwd(t["v"], t["da"], t["B"], t["C"], t["gamma"], t["scale"], t["h0"], chunk_len=64)
+    torch.cuda.synchronize()
+    inp["da"][:, reset] = -1e4
+    yr, hr = oracle.ssd3(inp["v"], inp["da"], inp["B"], inp["C"], inp["gamma"], inp["scale"], inp["h0"], 16)
+    np.testing.assert_allclose(y.cpu().numpy(), yr, rtol=1e-4, atol=3e-5)
+    np.testing.assert_allclose(hT.cpu().numpy(), hr, rtol=1e-4, atol=3e-5)
+
+
 def test_ssd2_workspace_of_the_generic_path_still_serves():
     """A workspace of the SIMT kernels' size, without room for segment states,
     is accepted: the call then takes those kernels."""
