@@ -131,6 +131,23 @@ def test_ssd3_decays_of_the_lowest_value(l, low):
         _close(out[k], want[w], k)
 
 
+def test_ssd3_infinite_dy_of_the_first_step():
+    """An infinite dy gives infinities in its own step's dv, as its product with
+    C.B has it, and leaves the other columns of dv alone."""
+    import torch
+    import mamba_hip
+    b, l, m, h, g, n, p = 1, 1, 1, 1, 1, 64, 64
+    rng = np.random.default_rng(1)
+    r = lambda *s: rng.standard_normal(s, dtype=np.float32)  # noqa: E731
+    v, dy, B, C = r(b, l, m, h, p), r(b, l, m, h, p), r(b, l, m, g, n), r(b, l, m, g, n)
+    dy[..., 9] = np.inf
+    da, gam, scl = (-np.ones((b, l, h), np.float32), np.ones((b, l, h), np.float32), np.ones((b, l, h), np.float32))
+    out = mamba_hip.ssd3_bwd(_t(dy), _t(v), _t(da), _t(B), _t(C), _t(gam), _t(scl))
+    torch.cuda.synchronize()
+    dv = out["dv"].cpu().numpy().reshape(p)
+    assert dv[9] == np.sign(float((B * C).sum())) * np.inf and np.isfinite(np.delete(dv, 9)).all()
+
+
 def test_ssd2_any_segment_count_gives_the_same_gradients():
     """A workspace that holds fewer segments (as small as the SIMT kernels', one
     entry state per 32 positions) is used with fewer; both agree to f32 rounding."""

@@ -132,6 +132,22 @@ def test_ssd3_decays_of_the_lowest_value(l, h, low):
     np.testing.assert_allclose(hT.cpu().numpy(), hr, rtol=1e-4, atol=3e-5)
 
 
+def test_ssd3_infinite_value_of_the_last_step():
+    """An infinite v gives infinities at its own row, as its product with C.B has
+    it, and leaves the other columns alone."""
+    import torch
+    import mamba_hip
+    b, l, m, h, p, n = 1, 3, 1, 1, 64, 64
+    inp = ssd3_inputs(7, b, l, m, h, p, n)
+    inp["v"][0, -1, 0, 0, 9] = np.inf
+    t = {k: _dev(v) for k, v in inp.items()}
+    y, _ = mamba_hip.ssd3_fwd(t["v"], t["da"], t["B"], t["C"], t["gamma"], t["scale"], t["h0"], chunk_len=16)
+    torch.cuda.synchronize()
+    y = y.cpu().numpy()[0, -1, 0, 0]
+    cb = float(np.dot(inp["B"].reshape(l, n)[-1], inp["C"].reshape(l, n)[-1]))
+    assert y[9] == np.sign(cb) * np.inf and np.isfinite(np.delete(y, 9)).all()
+
+
 def test_ssd2_workspace_of_the_generic_path_still_serves():
     """A workspace of the SIMT kernels' size, without room for segment states,
     is accepted: the call then takes those kernels."""
