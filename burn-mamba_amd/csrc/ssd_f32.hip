@@ -356,14 +356,14 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
                 const float* vr = S.V + i * VP + 32 * pt + 4 * hf;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    float o0 = ya[4 * k], o1 = ya[4 * k + 1], o2 = ya[4 * k + 2], o3 = ya[4 * k + 3];
-                    if (p.D) {  // without one no 0 v: an infinite v stays what its product is
-                        const float4 x = *reinterpret_cast<const float4*>(vr + 8 * k);
-                        o0 = __builtin_fmaf(D, x.x, o0);
-                        o1 = __builtin_fmaf(D, x.y, o1);
-                        o2 = __builtin_fmaf(D, x.z, o2);
-                        o3 = __builtin_fmaf(D, x.w, o3);
-                    }
+                    const float4 x = *reinterpret_cast<const float4*>(vr + 8 * k);
+                    // without D no 0 v: an infinite v stays what its product is (selects, here
+                    // and in the backward: a training step at 2 x 4096, 32 heads, rank 4 takes
+                    // 0.7 % longer than with D = 0, with branches 1.1 %)
+                    const float o0 = p.D ? __builtin_fmaf(D, x.x, ya[4 * k]) : ya[4 * k];
+                    const float o1 = p.D ? __builtin_fmaf(D, x.y, ya[4 * k + 1]) : ya[4 * k + 1];
+                    const float o2 = p.D ? __builtin_fmaf(D, x.z, ya[4 * k + 2]) : ya[4 * k + 2];
+                    const float o3 = p.D ? __builtin_fmaf(D, x.w, ya[4 * k + 3]) : ya[4 * k + 3];
                     if constexpr (sizeof(T) == 4)
                         *reinterpret_cast<float4*>(yr + 8 * k) = make_float4(o0, o1, o2, o3);
                     else

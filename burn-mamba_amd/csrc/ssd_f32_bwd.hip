@@ -547,16 +547,15 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 if (t < p.L) {
                     float* out = p.dv + ((((int64_t)j.b * p.L + t) * p.M + (row & (p.M - 1))) * p.H + j.h) * kBP +
                                  32 * pt + 4 * hf;
-                    if (p.D) {  // without one no 0 dy: an infinite dy stays what its product is
-                        const float* yr = S.Y + row * kBVP + 32 * pt + 4 * hf;
+                    // without D no 0 dy: an infinite dy stays what its product is
+                    const float* yr = S.Y + row * kBVP + 32 * pt + 4 * hf;
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const float4 y = fb_ld4(yr + 8 * q);
-                            a[4 * q] = __builtin_fmaf(D, y.x, a[4 * q]);
-                            a[4 * q + 1] = __builtin_fmaf(D, y.y, a[4 * q + 1]);
-                            a[4 * q + 2] = __builtin_fmaf(D, y.z, a[4 * q + 2]);
-                            a[4 * q + 3] = __builtin_fmaf(D, y.w, a[4 * q + 3]);
-                        }
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 y = fb_ld4(yr + 8 * q);
+                        a[4 * q] = p.D ? __builtin_fmaf(D, y.x, a[4 * q]) : a[4 * q];
+                        a[4 * q + 1] = p.D ? __builtin_fmaf(D, y.y, a[4 * q + 1]) : a[4 * q + 1];
+                        a[4 * q + 2] = p.D ? __builtin_fmaf(D, y.z, a[4 * q + 2]) : a[4 * q + 2];
+                        a[4 * q + 3] = p.D ? __builtin_fmaf(D, y.w, a[4 * q + 3]) : a[4 * q + 3];
                     }
                     fb_put(out, p.vec, a);
                 }
