@@ -134,7 +134,7 @@ def test_patch_applies_to_the_reference():
     import subprocess
     import tempfile
     ref = "/root/reference"
-    if not os.path.isdir(ref) or shutil.which("patch") is None:
+    if not os.path.isfile(os.path.join(ref, "Cargo.toml")) or shutil.which("patch") is None:
         pytest.skip("reference checkout or patch(1) not available")
     pf = os.path.join(CRATE, "patches", "burn-mamba-backend-rocm.patch")
     files = re.findall(r"^\+\+\+ b/(\S+)", open(pf).read(), re.M)
