@@ -1087,7 +1087,7 @@ def bench_ssd3_bwd(args):
         "dtype": "f32", "data": "synthetic (BASELINE.json configs[4] distributions at the SSD seam, dy ~ N(0,1), "
                                 "seeds 0 / 1)",
         "config": {"workload": "mamba3_ssd_bwd_cfg4", **cfg, "io": "all f32, per-head B / C",
-                   "entry": "mamba_ssd3_bwd (chunk states, reverse chunk loop; 32 fused positions per chunk)"},
+                   "entry": "mamba_ssd3_bwd (chunk states, reverse chunk loop; 64 fused positions per chunk)"},
         "roofline": roof,
     }
 

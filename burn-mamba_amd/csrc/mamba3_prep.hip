@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256) void mamba3_double_inputs_kernel(M3PrepParams 
 // head (16 bytes of bf16) for TL positions, its mimo_z / mimo_o in registers (M
 // <= 4), and issues the loads of a position's ranks together.  Bound by HBM:
 // every rank of y and z read, out written.  Measured at 4 x 8192 positions, 32
-// heads x 64, rank 4, bf16 (805 MB): 1013 -> 160 us against one channel
+// heads x 64, rank 4, bf16 (805 MB): 1013 -> 204 us against one channel
 // per lane and load, whose z and weight loads repeat per rank; TL amortises the
 // weights (64 registers at rank 4) where positions are plenty.
 // out_norm's sum runs over the P / 8 lanes of a head.

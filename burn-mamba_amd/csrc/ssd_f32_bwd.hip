@@ -45,14 +45,14 @@
 // Sums over rows whose weights fall with the row (g, dv, dB) run from the last
 // row: a term rounds at the size of the sum it meets, so the small ones go first.
 // Measured: the backward at 2 x 4096 steps, 32 heads 64 x 128, rank 4, 5.6 ms ->
-// 2.4 ms (reverse loop 4.53 -> 1.70 ms)
+// 2.3 ms (reverse loop 4.53 -> 1.62 ms)
 // against one workgroup per (batch, head, half of dstate) on
 // 32-row chunks, which it replaces; at 2 x 2048, 80 heads, rank 1, 0.98 -> 0.82
 // ms; and at dstate 64 (1 x 1024, 24 heads), where the SIMT kernels ran, 7.6 ms
 // -> 0.08 ms.
 // T: bf16 rows are widened on their way into LDS (the same values as an f32 copy,
 // half the bytes of three passes, and no spills in the reverse loop): a bf16
-// forward and backward at 2 x 2048, 80 heads, rank 1 943 -> 873 us with the four
+// forward and backward at 2 x 2048, 80 heads, rank 1 943 -> 880 us with the four
 // conversion launches gone.
 #include <algorithm>
 #include <type_traits>
