@@ -23,10 +23,10 @@
 //   g <- exp(cs_end) g + sum_i b_i C_i (x) dy_i.
 // Mamba-2: ddt = A dda + dsc + dgm, dA = sum dt dda, dD = sum DV_jj.
 //
-// Three launches (two when a (batch, head) is not split):
+// Three launches (two when a (batch, head) is not split, one for 32 rows or fewer):
 //   1. ssd_f32_bwd_seg: the states of all segments but the last from zero, and
 //      the state gradients of all but the first.
-//   2. ssd_f32_bwd_states: from its entry state, each segment's chunk-entry
+//   2. ssd_f32_bwd_states (more than 32 rows): from its entry state, each segment's chunk-entry
 //      states, written for the next launch.
 //   3. ssd_f32_bwd_chunks: each segment's chunks in reverse, 8 waves with fixed
 //      roles; g stays in registers in both layouts that the products take it in
@@ -346,12 +346,18 @@ struct FBLds {
     float dec;
 };
 
-template <int N, typename T>
+// ONE: the sequence is one chunk of at most 32 rows.  Its second row tile, all
+// zeros, is left out (the sums are the same), and its entry state is the initial one:
+// no states launch.  16 positions, 12 heads, dstate 128, f32: 34.7 -> 22.8 us (25.1
+// before the chunks had 64 rows).  Leaving the tile out of a longer sequence's last
+// chunk too, the chunk's code twice, made the loop itself 3 % slower.
+template <int N, typename T, bool ONE>
 __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) {
     extern __shared__ __align__(16) char fb_smem[];
     FBLds<N>& S = *reinterpret_cast<FBLds<N>*>(fb_smem);
     constexpr int NTN = N / 32, TILES = 2 * NTN, NT = 512, NP = N + 4;
-    constexpr int XT = N == 128 ? 2 : 1;  // row tiles of dB and dC per wave
+    constexpr int RT = ONE ? 1 : 2, KS = 4 * RT;     // row tiles, and their groups of eight rows
+    constexpr int XT = N == 128 && !ONE ? 2 : 1;      // row tiles of dB and dC per wave
     const int tid = threadIdx.x, wv = wave_id(), lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
     const FBJob j = fb_job(p, blockIdx.x / p.S, blockIdx.x % p.S);
     const T* vb = static_cast<const T*>(p.v) + (int64_t)j.b * p.v_sb + (int64_t)j.h * p.v_sh;
@@ -413,7 +419,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             const int lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
             if (c > j.c0) fetch(c - 1, tid);
 #pragma unroll
-            for (int x = 0; x < 2; ++x) {
+            for (int x = 0; x < RT; ++x) {
                 const int row = 32 * x + i32;
                 const float* Bp = S.B + row * NP + 32 * GT * nh + 4 * hf;
                 bwd_f32x16 a = fb_zero();
@@ -436,7 +442,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[x][r] = a[r] * w;
             }
-            {
+            if (RT == 2 || nh) {
                 // the other row tile's share goes to its wave
                 float* out = S.P[2 * pt + nh] + lane;
 #pragma unroll
@@ -522,14 +528,14 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             };
             if (wv == 0)
                 tile(std::true_type{}, 0, 0);
-            else if (wv == 6)
+            else if (RT == 2 && wv == 6)
                 tile(std::false_type{}, 1, 0);
-            else if (wv == 7)
+            else if (RT == 2 && wv == 7)
                 tile(std::true_type{}, 1, 1);
-            else if (c > j.c0)  // wave 1 has no pair tile: the next chunk's decays
+            else if ((RT == 2 || wv == 1) && c > j.c0)  // wave 1 has no pair tile: the next chunk's decays
                 rd = fb_decay(p, rt, A, lane);
             __syncthreads();
-            {
+            if (RT == 2 || !nh) {
                 const float* in = S.P[2 * pt + 1 - nh] + lane;
                 bwd_f32x16 a;
 #pragma unroll
@@ -537,7 +543,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Ap = S.Y + 4 * hf * kBVP + 32 * pt + i32;
                 const float* Bp = S.E1 + 4 * hf * kBVP + 32 * nh + i32;
 #pragma unroll
-                for (int s = 7; s >= 0; --s)
+                for (int s = KS - 1; s >= 0; --s)
                     if (s >= 4 * nh) {
 #pragma unroll
                         for (int k = 3; k >= 0; --k) a = bwd_mfma(Ap[(8 * s + k) * kBVP], Bp[(8 * s + k) * kBVP], a);
@@ -569,7 +575,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * GT * nh + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + 32 * pt + i32;
 #pragma unroll
-                for (int s = 7; s >= 0; --s) {
+                for (int s = KS - 1; s >= 0; --s) {
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
@@ -583,14 +589,15 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             }
             if (wv == 7) {
             // lane = fused row; a step's results on its first rank's lane
-            const float xu = (S.xu[0][lane] + S.xu[1][lane]) + (S.xu[2][lane] + S.xu[3][lane]);
+            float xu = (S.xu[0][lane] + S.xu[1][lane]) + (S.xu[2][lane] + S.xu[3][lane]);
             float uh = 0.f, gh = 0.f;
 #pragma unroll
             for (int k = 0; k < NTN; ++k) {
                 uh += S.uh[k][lane];
                 gh += S.ghc[k];
             }
-            const float xg = lane < 32 ? S.xg[0][lane] + S.xg[1][lane] : S.xg[1][lane];
+            float xg = lane < 32 && RT == 2 ? S.xg[0][lane] + S.xg[1][lane] : S.xg[RT - 1][lane];
+            if (RT == 1 && lane >= 32) xu = uh = xg = 0.f;  // never formed
             const float sc = S.sc[lane];
             const float z = S.w[lane] * xu, pz = wave_incl_scan(z) - z;
             // T's pairs j before t <= i: those of t's own 32-row tile as column
@@ -598,15 +605,19 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             // the tile below the diagonal one-sided, with nothing to cancel, as
             // columns before t or rows from t on.  One scan of 64 rows instead
             // left dA 1.4 times as far from 64 bits.
-            const float d = sc * S.xg[lane >> 5][lane] - S.rowm[lane >> 5][lane];
+            const float d = RT == 2 ? sc * S.xg[lane >> 5][lane] - S.rowm[lane >> 5][lane]
+                            : lane < 32 ? sc * xg - S.rowm[0][lane] : 0.f;
             const float pd = half_incl_scan(d) - d;
             const int rl = lane < 32 ? lane : 95 - lane;  // rows 32 .. 63 from the last
-            const float x = lane < 32 ? sc * S.xg[1][lane] : S.rowm[0][rl];
-            const float sx = __shfl(half_incl_scan(x), rl, 64), px = lane < 32 ? sx - x : sx;
+            float px = 0.f;
+            if constexpr (RT == 2) {
+                const float x = lane < 32 ? sc * S.xg[1][lane] : S.rowm[0][rl], sx = __shfl(half_incl_scan(x), rl, 64);
+                px = lane < 32 ? sx - x : sx;
+            }
             // suffix sums of b_i uh_i: the scan runs from the last lane
             const float su = __shfl(wave_incl_scan(__shfl(S.bv[lane] * uh, 63 - lane, 64)), 63 - lane, 64);
             const float dda = S.dec * gh + pz + su + (px + pd);
-            float ds = xg + S.av[lane] * xu, dg = S.dg[lane];
+            float ds = xg + S.av[lane] * xu, dg = RT == 2 || lane < 32 ? S.dg[lane] : 0.f;
             for (int o = 1; o < p.M; o <<= 1) {
                 ds += __shfl_xor(ds, o, 64);
                 dg += __shfl_xor(dg, o, 64);
@@ -651,7 +662,11 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) G[2 + k][r] = src[k * 1024 + r * 64];
         };
-        fetch_h(j.c1 - 1, lane);
+        if (!ONE)
+            fetch_h(j.c1 - 1, lane);
+        else  // one chunk: its entry state is the initial one
+#pragma unroll
+            for (int k = 0; k < 2; ++k) fb_entry<N, true>(p, j, false, k, nt, i32, hf, G[2 + k]);
 #pragma unroll
         for (int k = 0; k < 2; ++k) fb_entry<N, true>(p, j, true, k, nt, i32, hf, G[k]);
         commit(j.c1 - 1, tid);
@@ -663,6 +678,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             const int lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
 #pragma unroll
             for (int x = 0; x < XT; ++x) {
+                if (ONE && own) break;
                 const int row = 32 * (XT == 2 ? x : own) + i32;
                 const float* Vp = S.V + row * kBVP + 4 * hf;
                 const float* Yp = S.Y + row * kBVP + 4 * hf;
@@ -707,11 +723,12 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             __syncthreads();
 #pragma unroll
             for (int x = 0; x < XT; ++x) {
+                if (ONE && own) break;
                 const int xt = XT == 2 ? x : own, row = 32 * xt + i32;
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Ep = S.E2 + 4 * hf * kBVP + 32 * xt + i32;
 #pragma unroll
-                for (int s = 7; s >= 0; --s)
+                for (int s = KS - 1; s >= 0; --s)
                     if (s >= 4 * xt) {
 #pragma unroll
                         for (int k = 3; k >= 0; --k)
@@ -751,7 +768,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + i32;
 #pragma unroll
-                for (int s = 7; s >= 0; --s) {
+                for (int s = KS - 1; s >= 0; --s) {
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
@@ -821,25 +838,34 @@ bool ssd_f32_bwd_plan(SsdF32BwdParams* q, size_t limit) {
     return best > 0. && units * p.S * 2 < (1ll << 31);
 }
 
-template <int N, typename T>
-static int fb_run(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+static bool fb_one(const SsdF32BwdParams& p) { return (int64_t)p.L << p.mshift <= kFR / 2; }
+
+template <int N, typename T, bool ONE>
+static int fb_run_as(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
     const int units = p.nb * p.H;
     // dynamic LDS above the 64 KB default (up to the CU's 160 KB)
     constexpr size_t lds = sizeof(FBLds<N>);
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N, T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N, T, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)lds));
     if (p.S > 1) {
         hipLaunchKernelGGL((ssd_f32_bwd_seg<N, T>), dim3(units * (p.S - 1) * 2), dim3(256), 0, stream, p);
         MAMBA_CHECK_LAUNCH();
     }
-    hipLaunchKernelGGL((ssd_f32_bwd_states<N, T>), dim3(units * p.S), dim3(256), 0, stream, p);
-    MAMBA_CHECK_LAUNCH();
+    if (!ONE) {
+        hipLaunchKernelGGL((ssd_f32_bwd_states<N, T>), dim3(units * p.S), dim3(256), 0, stream, p);
+        MAMBA_CHECK_LAUNCH();
+    }
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
-    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N, T>), dim3(units * p.S), dim3(512), lds, stream, p);
+    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N, T, ONE>), dim3(units * p.S), dim3(512), lds, stream, p);
     MAMBA_CHECK_LAUNCH();
     if (ev1) MAMBA_CHECK_HIP(hipEventRecord(ev1, stream));
     return MAMBA_OK;
+}
+
+template <int N, typename T>
+static int fb_run(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+    return fb_one(p) ? fb_run_as<N, T, true>(p, stream, ev0, ev1) : fb_run_as<N, T, false>(p, stream, ev0, ev1);
 }
 
 int ssd_f32_bwd_launch(SsdF32BwdParams& p, void* ws, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
