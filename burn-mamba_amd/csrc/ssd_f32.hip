@@ -209,6 +209,7 @@ struct FScanLds {
     float h[N * (PB + 8)];    // the state entering the chunk, [n][p]
     float W[kFR * (kFR + 8)];  // W_ij (C_i . B_j), [j][i]
     FTables T;
+    float zero[32];  // read for v where there is no D: 0 v of an infinite v would be NaN
 };
 
 template <typename T, int PB, int N>
@@ -281,6 +282,7 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
         publish();
     }
     if (wv == 7) rd = f_tab_decay(p, rt, A, j.c0, lane);
+    if (tid < 32) S.zero[tid] = 0.f;
     commit(j.c0);
     __syncthreads();
     // y waves: rows 32 it, columns 32 pt
@@ -353,17 +355,12 @@ __global__ __launch_bounds__(512) void ssd_f32_scan(SsdF32Params p) {
             const int i = 32 * it + i32, t = c * steps + (i >> p.mshift);
             if (t < p.L) {
                 T* yr = yb + (int64_t)t * p.y_sl + (int64_t)(i & (p.M - 1)) * p.y_sm + 32 * pt + 4 * hf;
-                const float* vr = S.V + i * VP + 32 * pt + 4 * hf;
+                const float* vr = p.D ? S.V + i * VP + 32 * pt + 4 * hf : S.zero + 4 * hf;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const float4 x = *reinterpret_cast<const float4*>(vr + 8 * k);
-                    // without D no 0 v: an infinite v stays what its product is (selects, here
-                    // and in the backward: a training step at 2 x 4096, 32 heads, rank 4 takes
-                    // 0.7 % longer than with D = 0, with branches 1.1 %)
-                    const float o0 = p.D ? __builtin_fmaf(D, x.x, ya[4 * k]) : ya[4 * k];
-                    const float o1 = p.D ? __builtin_fmaf(D, x.y, ya[4 * k + 1]) : ya[4 * k + 1];
-                    const float o2 = p.D ? __builtin_fmaf(D, x.z, ya[4 * k + 2]) : ya[4 * k + 2];
-                    const float o3 = p.D ? __builtin_fmaf(D, x.w, ya[4 * k + 3]) : ya[4 * k + 3];
+                    const float o0 = __builtin_fmaf(D, x.x, ya[4 * k]), o1 = __builtin_fmaf(D, x.y, ya[4 * k + 1]);
+                    const float o2 = __builtin_fmaf(D, x.z, ya[4 * k + 2]), o3 = __builtin_fmaf(D, x.w, ya[4 * k + 3]);
                     if constexpr (sizeof(T) == 4)
                         *reinterpret_cast<float4*>(yr + 8 * k) = make_float4(o0, o1, o2, o3);
                     else

@@ -335,6 +335,7 @@ struct FBLds {
     float E1[kFR * kBVP];     // [i][j] W CB
     float E2[kFR * kBVP];     // [i][j] W DV
     float cs[kFR], lo[kFR], gm[kFR], sc[kFR], av[kFR], bv[kFR], w[kFR];
+    float zero[32];           // read for dy where there is no D: 0 dy of an infinite dy would be NaN
     float P[4][16 * 64];      // [pt, nh] its share of g B for the other row tile, accumulator order
     float xu[4][kFR];         // v_j . g B_j over 32 columns of p and half of n
     float uh[4][kFR];         // C_i . h^T dy_i over 32 columns of n
@@ -401,6 +402,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
     // B | commit |), so that no wave holds another role's accumulators.
     fetch(j.c1 - 1, tid);
     if (wv == 1) rd = fb_decay(p, rt, A, lane);
+    if (tid < 32) S.zero[tid] = 0.f;
     if (wv < 2 || wv >= 6) {
         // 32 columns of p (pt) and half of n (nh): its share of g B for both row
         // tiles, a pair tile, then dv of row tile nh
@@ -553,15 +555,14 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 if (t < p.L) {
                     float* out = p.dv + ((((int64_t)j.b * p.L + t) * p.M + (row & (p.M - 1))) * p.H + j.h) * kBP +
                                  32 * pt + 4 * hf;
-                    // without D no 0 dy: an infinite dy stays what its product is
-                    const float* yr = S.Y + row * kBVP + 32 * pt + 4 * hf;
+                    const float* yr = p.D ? S.Y + row * kBVP + 32 * pt + 4 * hf : S.zero + 4 * hf;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const float4 y = fb_ld4(yr + 8 * q);
-                        a[4 * q] = p.D ? __builtin_fmaf(D, y.x, a[4 * q]) : a[4 * q];
-                        a[4 * q + 1] = p.D ? __builtin_fmaf(D, y.y, a[4 * q + 1]) : a[4 * q + 1];
-                        a[4 * q + 2] = p.D ? __builtin_fmaf(D, y.z, a[4 * q + 2]) : a[4 * q + 2];
-                        a[4 * q + 3] = p.D ? __builtin_fmaf(D, y.w, a[4 * q + 3]) : a[4 * q + 3];
+                        a[4 * q] = __builtin_fmaf(D, y.x, a[4 * q]);
+                        a[4 * q + 1] = __builtin_fmaf(D, y.y, a[4 * q + 1]);
+                        a[4 * q + 2] = __builtin_fmaf(D, y.z, a[4 * q + 2]);
+                        a[4 * q + 3] = __builtin_fmaf(D, y.w, a[4 * q + 3]);
                     }
                     fb_put(out, p.vec, a);
                 }
