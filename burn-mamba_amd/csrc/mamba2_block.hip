@@ -175,10 +175,13 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
 #pragma unroll
             for (int u = 0; u < kM2ConvRows; ++u) emit(l + u, xs[u]);
         }
-        for (; l < l1; ++l) {
-            float x[VW];
-            load(l, x);
-            emit(l, x);
+        if (l < l1) {  // the rest, its loads together as well (past the tile: its last row again)
+            float xs[kM2ConvRows - 1][VW];
+#pragma unroll
+            for (int u = 0; u < kM2ConvRows - 1; ++u) load(min(l + u, l1 - 1), xs[u]);
+#pragma unroll
+            for (int u = 0; u < kM2ConvRows - 1; ++u)
+                if (l + u < l1) emit(l + u, xs[u]);
         }
         // the new window: the last K columns of [old window's last K - 1 | inputs],
         // by the only threads that have read the old one
