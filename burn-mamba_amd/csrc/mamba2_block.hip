@@ -90,43 +90,58 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
     const TI* proj = static_cast<const TI*>(p.proj) + (int64_t)b * p.proj_sb;
     if (c0 < p.V) {
         float w[VW][K], bias[VW];
+        // a channel's K weights or window columns
+        auto row = [&](const float* at, float* v) {
+            if (K % 4 == 0 && p.w_vec) {
 #pragma unroll
-        for (int e = 0; e < VW; ++e) {
-            const float* we = p.w + (int64_t)(c0 + e) * K;
-            if (K == 4 && p.w_vec) {
-                const float4 v = *(const float4*)we;
-                const float wk[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int k = 0; k < K; ++k) w[e][k] = wk[k & 3];
+                for (int k = 0; k + 3 < K; k += 4) {
+                    const float4 q = *(const float4*)(at + k);
+                    v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
+                }
             } else {
 #pragma unroll
-                for (int k = 0; k < K; ++k) w[e][k] = we[k];
+                for (int k = 0; k < K; ++k) v[k] = at[k];
             }
+        };
+        float* const st = p.state + ((int64_t)b * p.V + c0) * K;
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+            row(p.w + (int64_t)(c0 + e) * K, w[e]);
             bias[e] = p.bias ? p.bias[c0 + e] : 0.f;
         }
+        auto load = [&](int l, float* x) {
+            const TI* src = proj + (int64_t)l * p.proj_sl + p.xbc_off + c0;
+            if constexpr (VW == 8) {
+                m2_ld8(src, x);
+            } else {
+#pragma unroll
+                for (int e = 0; e < VW; ++e) x[e] = m2_ld1(src + e);
+            }
+        };
         // window: win[j] holds xpad[l0 + j] for j < K - 1 (positions l0 - K + 1 + j)
         float win[K > 1 ? K - 1 : 1][VW];
+        if (tile == 0) {  // the cache's last K - 1 columns
 #pragma unroll
-        for (int j = 0; j < K - 1; ++j) {
-            const int l = l0 - (K - 1) + j;  // uniform over the workgroup
-            bool done = false;
-            if constexpr (VW == 8) {
-                if (l >= 0) {
-                    m2_ld8(proj + (int64_t)l * p.proj_sl + p.xbc_off + c0, win[j]);
-                    done = true;
-                }
-            }
-            if (!done) {
+            for (int e = 0; e < VW; ++e) {
+                float v[K];
+                row(st + e * K, v);
 #pragma unroll
-                for (int e = 0; e < VW; ++e) {
-                    float v;
-                    if (l >= 0)
-                        v = m2_ld1(proj + (int64_t)l * p.proj_sl + p.xbc_off + c0 + e);
-                    else  // cache column (K + l): the window's last K - 1 columns end at column K - 1
-                        v = p.state[((int64_t)b * p.V + c0 + e) * K + K + l];
-                    win[j][e] = v;
-                }
+                for (int j = 0; j < K - 1; ++j) win[j][e] = v[j + 1];
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < K - 1; ++j) load(l0 - (K - 1) + j, win[j]);
+        }
+        // a sequence of one tile: the new window is the last K - 1 rows that slide
+        // through win, after the one that leaves it
+        const bool one = tile == 0 && l1 == p.L;
+        float first[VW] = {};
+        if (one) {
+            if (p.L >= K)
+                load(p.L - K, first);
+            else
+#pragma unroll
+                for (int e = 0; e < VW; ++e) first[e] = st[e * K + p.L];
         }
         TO* out = static_cast<TO*>(p.out) + (int64_t)b * p.out_sb;
         // one position: convolve, slide the window, store
@@ -156,15 +171,6 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
                 for (int e = 0; e < VW; ++e) m2_st1(dst + e, y[e]);
             }
         };
-        auto load = [&](int l, float* x) {
-            const TI* src = proj + (int64_t)l * p.proj_sl + p.xbc_off + c0;
-            if constexpr (VW == 8) {
-                m2_ld8(src, x);
-            } else {
-#pragma unroll
-                for (int e = 0; e < VW; ++e) x[e] = m2_ld1(src + e);
-            }
-        };
         // kM2ConvRows rows are loaded before any is used, so their HBM
         // latencies overlap instead of adding up row by row
         int l = l0;
@@ -186,24 +192,20 @@ __global__ __launch_bounds__(256) void mamba2_conv_kernel(M2ConvParams p) {
         // the new window: the last K columns of [old window's last K - 1 | inputs],
         // by the only threads that have read the old one
         if (tile == 0) {
-            float* st = p.state + ((int64_t)b * p.V + c0) * K;
             float nw[VW][K];
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                const int l = p.L - K + j;  // input position; before 0: old column K + l
                 float x[VW];
-                if (l >= 0)
-                    load(l, x);
-                else
+                if (!one) load(p.L - K + j, x);  // of more than kM2ConvRows >= K rows
 #pragma unroll
-                    for (int e = 0; e < VW; ++e) x[e] = st[e * K + K + l];
-#pragma unroll
-                for (int e = 0; e < VW; ++e) nw[e][j] = x[e];
+                for (int e = 0; e < VW; ++e) nw[e][j] = !one ? x[e] : j > 0 ? win[j > 0 ? j - 1 : 0][e] : first[e];
             }
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
-                if (K == 4 && p.w_vec) {
-                    *(float4*)(st + 4 * e) = make_float4(nw[e][0], nw[e][1 % K], nw[e][2 % K], nw[e][3 % K]);
+                if (K % 4 == 0 && p.w_vec) {
+#pragma unroll
+                    for (int k = 0; k + 3 < K; k += 4)
+                        *(float4*)(st + e * K + k) = make_float4(nw[e][k], nw[e][k + 1], nw[e][k + 2], nw[e][k + 3]);
                 } else {
 #pragma unroll
                     for (int j = 0; j < K; ++j) st[e * K + j] = nw[e][j];
@@ -375,6 +377,9 @@ __global__ __launch_bounds__(256) void mamba2_gated_norm_res_kernel(M2NormParams
 // of its own for the window, 5376 channels, bf16: 1 x 200 tokens 26.6 -> 11.1 us,
 // 2 x 1021 31.4 -> 18.2, 4 x 2000 57.5 -> 50.7, 8 x 4096 173 -> 171 us (with 384
 // or 768 workgroups asked for, 2 x 1021 takes 25.6 or 28.1 us).
+// In f32, with whole rows of weights and window loaded and the window of one tile
+// taken from what slid through it: 1 position 9.3 -> 8.0 (10.9 word by word), 200 24.3
+// -> 9.2 (10.7); a kernel of 8, 8 x 5376 x 1 15.8 -> 11.7 (19.3), 8 x 1021 106 -> 92.
 static int conv_tile(const M2ConvParams& p, int cblocks) {
     int t = 64;
     while (t > kM2ConvRows && (int64_t)((p.L + t - 1) / t) * cblocks * p.nb < 192) t /= 2;

@@ -28,15 +28,25 @@ def test_conv1d_fwd_kernels(case, K):
     _check(*case, K)
 
 
-def _check(b, L, c, K):
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 8])
+@pytest.mark.parametrize("l,c", [(1, 16), (3, 16), (4, 7), (7, 16), (8, 24), (9, 16), (15, 7)])
+def test_conv1d_fwd_of_one_tile(l, c, K, off):
+    """At most 8 positions: the new window is what slid through the old one, on both
+    sides of the kernel's length; whole rows of weights and window where they are
+    16-byte aligned (off 0, kernels of 4 and 8), a word at a time elsewhere."""
+    _check(2, l, c, K, off)
+
+
+def _check(b, L, c, K, off=0):
     import torch
     import mamba_hip
     import oracle
     rng = np.random.default_rng(b + L + c)
     x, st = rng.standard_normal((b, L, c), dtype=np.float32), rng.standard_normal((b, c, K), dtype=np.float32)
     w, bias = rng.standard_normal((c, K), dtype=np.float32), rng.standard_normal(c, dtype=np.float32)
-    s = torch.from_numpy(st).cuda()
     g = lambda a: torch.from_numpy(a).cuda()  # noqa: E731
+    s = torch.empty(st.size + off, device="cuda")[off:].view(st.shape).copy_(g(st))
     out = mamba_hip.conv1d_fwd(g(x), s, g(w), g(bias))
     torch.cuda.synchronize()
     want, _, wst = oracle.mamba2_conv_fwd(x, w, bias, st, np.zeros(0), 0, 0, c, 0)
