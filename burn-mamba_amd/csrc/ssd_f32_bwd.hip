@@ -347,17 +347,22 @@ struct FBLds {
     float dec;
 };
 
-// ONE: the sequence is one chunk of at most 32 rows.  Its second row tile, all
-// zeros, is left out (the sums are the same), and its entry state is the initial one:
-// no states launch.  16 positions, 12 heads, dstate 128, f32: 34.7 -> 22.8 us (25.1
-// before the chunks had 64 rows).  Leaving the tile out of a longer sequence's last
-// chunk too, the chunk's code twice, made the loop itself 3 % slower.
-template <int N, typename T, bool ONE>
+// What the last chunk's rows are.  A second row tile of zeros is left out (the sums
+// are the same): in kernels of their own, as the loop is 1 to 3 % slower with it.
+//   FB_FULL  anything
+//   FB_ONE   a sequence of one chunk of at most 32 rows: no other, and its entry state
+//            is the initial one, no states launch
+//   FB_TAIL  two to four chunks in one segment, the last of at most 32 rows
+// us against 32-row chunks and FB_FULL, dstate 128, f32: 12 heads, 16 positions 25.1 /
+// 34.7 / 22.8; 256 (batch, head), 16 positions 39.3 / 47.0 / 33.5, 90 66.1 / 77.3 / 72.5, 140
+// 93.0 / 105.9 / 101.  In several segments the last one's end is no earlier for it.
+enum FBRows { FB_FULL, FB_ONE, FB_TAIL };
+template <int N, typename T, FBRows R>
 __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) {
     extern __shared__ __align__(16) char fb_smem[];
     FBLds<N>& S = *reinterpret_cast<FBLds<N>*>(fb_smem);
     constexpr int NTN = N / 32, TILES = 2 * NTN, NT = 512, NP = N + 4;
-    constexpr int RT = ONE ? 1 : 2, KS = 4 * RT;     // row tiles, and their groups of eight rows
+    constexpr bool ONE = R == FB_ONE;
     constexpr int XT = N == 128 && !ONE ? 2 : 1;      // row tiles of dB and dC per wave
     const int tid = threadIdx.x, wv = wave_id(), lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
     const FBJob j = fb_job(p, blockIdx.x / p.S, blockIdx.x % p.S);
@@ -416,12 +421,14 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
         __syncthreads();
         for (int c = j.c1 - 1; c >= j.c0; --c) {
             const int t0 = c * steps;
+            const int RT = ONE || (R == FB_TAIL && c == p.nch - 1) ? 1 : 2, KS = 4 * RT;  // row tiles, groups of eight rows
             int tid = threadIdx.x;  // opaque per chunk: addresses and lane masks are formed in the loop
             asm volatile("" : "+v"(tid));
             const int lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
             if (c > j.c0) fetch(c - 1, tid);
 #pragma unroll
-            for (int x = 0; x < RT; ++x) {
+            for (int x = 0; x < 2; ++x) {
+                if (x >= RT) break;
                 const int row = 32 * x + i32;
                 const float* Bp = S.B + row * NP + 32 * GT * nh + 4 * hf;
                 bwd_f32x16 a = fb_zero();
@@ -545,8 +552,8 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Ap = S.Y + 4 * hf * kBVP + 32 * pt + i32;
                 const float* Bp = S.E1 + 4 * hf * kBVP + 32 * nh + i32;
 #pragma unroll
-                for (int s = KS - 1; s >= 0; --s)
-                    if (s >= 4 * nh) {
+                for (int s = 7; s >= 0; --s)
+                    if (s < KS && s >= 4 * nh) {
 #pragma unroll
                         for (int k = 3; k >= 0; --k) a = bwd_mfma(Ap[(8 * s + k) * kBVP], Bp[(8 * s + k) * kBVP], a);
                         if ((s & 1) == 0) fb_fence();
@@ -576,7 +583,8 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * GT * nh + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + 32 * pt + i32;
 #pragma unroll
-                for (int s = KS - 1; s >= 0; --s) {
+                for (int s = 7; s >= 0; --s) {
+                    if (s >= KS) continue;
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
@@ -611,7 +619,7 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             const float pd = half_incl_scan(d) - d;
             const int rl = lane < 32 ? lane : 95 - lane;  // rows 32 .. 63 from the last
             float px = 0.f;
-            if constexpr (RT == 2) {
+            if (RT == 2) {
                 const float x = lane < 32 ? sc * S.xg[1][lane] : S.rowm[0][rl], sx = __shfl(half_incl_scan(x), rl, 64);
                 px = lane < 32 ? sx - x : sx;
             }
@@ -674,12 +682,13 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
         __syncthreads();
         for (int c = j.c1 - 1; c >= j.c0; --c) {
             const int t0 = c * steps;
+            const int RT = ONE || (R == FB_TAIL && c == p.nch - 1) ? 1 : 2, KS = 4 * RT;  // row tiles, groups of eight rows
             int tid = threadIdx.x;  // opaque per chunk: addresses and lane masks are formed in the loop
             asm volatile("" : "+v"(tid));
             const int lane = tid & 63, i32 = lane & 31, hf = lane >> 5;
 #pragma unroll
             for (int x = 0; x < XT; ++x) {
-                if (ONE && own) break;
+                if (RT == 1 && (XT == 2 ? x : own)) break;
                 const int row = 32 * (XT == 2 ? x : own) + i32;
                 const float* Vp = S.V + row * kBVP + 4 * hf;
                 const float* Yp = S.Y + row * kBVP + 4 * hf;
@@ -724,13 +733,13 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
             __syncthreads();
 #pragma unroll
             for (int x = 0; x < XT; ++x) {
-                if (ONE && own) break;
+                if (RT == 1 && (XT == 2 ? x : own)) break;
                 const int xt = XT == 2 ? x : own, row = 32 * xt + i32;
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Ep = S.E2 + 4 * hf * kBVP + 32 * xt + i32;
 #pragma unroll
-                for (int s = KS - 1; s >= 0; --s)
-                    if (s >= 4 * xt) {
+                for (int s = 7; s >= 0; --s)
+                    if (s < KS && s >= 4 * xt) {
 #pragma unroll
                         for (int k = 3; k >= 0; --k)
                             acc[x] = bwd_mfma(Cp[(8 * s + k) * NP], Ep[(8 * s + k) * kBVP], acc[x]);
@@ -769,7 +778,8 @@ __global__ __launch_bounds__(512, 2) void ssd_f32_bwd_chunks(SsdF32BwdParams p) 
                 const float* Cp = S.C + 4 * hf * NP + 32 * nt + i32;
                 const float* Yp = S.Y + 4 * hf * kBVP + i32;
 #pragma unroll
-                for (int s = KS - 1; s >= 0; --s) {
+                for (int s = 7; s >= 0; --s) {
+                    if (s >= KS) continue;
                     const float4 b4 = fb_ld4(&S.bv[8 * s + 4 * hf]);
                     const float bi[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
@@ -839,26 +849,29 @@ bool ssd_f32_bwd_plan(SsdF32BwdParams* q, size_t limit) {
     return best > 0. && units * p.S * 2 < (1ll << 31);
 }
 
-static bool fb_one(const SsdF32BwdParams& p) { return (int64_t)p.L << p.mshift <= kFR / 2; }
+static FBRows fb_rows(const SsdF32BwdParams& p) {
+    const int64_t last = ((int64_t)p.L << p.mshift) - (int64_t)(p.nch - 1) * kFR;  // rows of the last chunk
+    return p.S > 1 || p.nch > 4 || last > kFR / 2 ? FB_FULL : p.nch == 1 ? FB_ONE : FB_TAIL;
+}
 
-template <int N, typename T, bool ONE>
+template <int N, typename T, FBRows R>
 static int fb_run_as(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
     const int units = p.nb * p.H;
     // dynamic LDS above the 64 KB default (up to the CU's 160 KB)
     constexpr size_t lds = sizeof(FBLds<N>);
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N, T, ONE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    MAMBA_CHECK_HIP(hipFuncSetAttribute((const void*)ssd_f32_bwd_chunks<N, T, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)lds));
     if (p.S > 1) {
         hipLaunchKernelGGL((ssd_f32_bwd_seg<N, T>), dim3(units * (p.S - 1) * 2), dim3(256), 0, stream, p);
         MAMBA_CHECK_LAUNCH();
     }
-    if (!ONE) {
+    if (R != FB_ONE) {
         hipLaunchKernelGGL((ssd_f32_bwd_states<N, T>), dim3(units * p.S), dim3(256), 0, stream, p);
         MAMBA_CHECK_LAUNCH();
     }
     if (ev0) MAMBA_CHECK_HIP(hipEventRecord(ev0, stream));
-    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N, T, ONE>), dim3(units * p.S), dim3(512), lds, stream, p);
+    hipLaunchKernelGGL((ssd_f32_bwd_chunks<N, T, R>), dim3(units * p.S), dim3(512), lds, stream, p);
     MAMBA_CHECK_LAUNCH();
     if (ev1) MAMBA_CHECK_HIP(hipEventRecord(ev1, stream));
     return MAMBA_OK;
@@ -866,7 +879,11 @@ static int fb_run_as(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev
 
 template <int N, typename T>
 static int fb_run(const SsdF32BwdParams& p, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-    return fb_one(p) ? fb_run_as<N, T, true>(p, stream, ev0, ev1) : fb_run_as<N, T, false>(p, stream, ev0, ev1);
+    switch (fb_rows(p)) {
+        case FB_ONE: return fb_run_as<N, T, FB_ONE>(p, stream, ev0, ev1);
+        case FB_TAIL: return fb_run_as<N, T, FB_TAIL>(p, stream, ev0, ev1);
+        default: return fb_run_as<N, T, FB_FULL>(p, stream, ev0, ev1);
+    }
 }
 
 int ssd_f32_bwd_launch(SsdF32BwdParams& p, void* ws, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {

@@ -15,9 +15,9 @@ def _same(a, b):
             assert a[k].dtype == w.dtype and float((a[k] - w).abs().max()) <= 3e-5 * float(w.abs().max()) + 1e-30, k
 
 
-# one step, a ragged chunk, several segments; both dstates; grouped; rows that only
+# one step, a ragged chunk, several segments, one that ends in half a chunk; both dstates; grouped; rows that only
 # the f32 route takes (odd offset, every other value, headdim 32)
-@pytest.mark.parametrize("l,h,g,p,n,form", [(1, 4, 1, 64, 64, "plain"), (65, 4, 2, 64, 128, "plain"), (700, 2, 1, 64, 128, "plain"),
+@pytest.mark.parametrize("l,h,g,p,n,form", [(1, 4, 1, 64, 64, "plain"), (65, 4, 2, 64, 128, "plain"), (700, 2, 1, 64, 128, "plain"), (70, 200, 1, 64, 128, "plain"),
                                             (300, 2, 2, 64, 64, "wide"), (70, 4, 1, 64, 64, "odd"),
                                             (70, 4, 1, 64, 128, "every other"), (70, 4, 1, 32, 64, "plain")])
 def test_mamba2(l, h, g, p, n, form):

@@ -22,12 +22,13 @@ def _close(got, want, name):
     np.testing.assert_allclose(got.cpu().numpy(), want, rtol=1e-4, atol=1e-4 * scale, err_msg=name)
 
 
-# (b, l, h, g, n, optional): one row, half a chunk and a chunk +- 1, many segments (one head),
+# (b, l, h, g, n, optional): one row, half a chunk (also as the last one of a whole
+# sequence) and a chunk +- 1, many segments (one head),
 # segments of two chunks, per-head and grouped B / C, with and without D, h0 and
 # d(final state)
 CASES2 = [(1, 1, 2, 1, 64, True), (2, 63, 2, 2, 64, False), (1, 64, 3, 1, 128, True), (1, 65, 2, 1, 64, True),
           (1, 700, 1, 1, 128, True), (2, 333, 4, 2, 64, True), (1, 130, 300, 1, 64, False), (1, 2500, 12, 2, 64, True),
-          (2, 31, 2, 2, 64, True), (1, 32, 4, 2, 128, True), (2, 33, 2, 1, 128, True)]
+          (2, 31, 2, 2, 64, True), (1, 32, 4, 2, 128, True), (2, 33, 2, 1, 128, True), (1, 90, 200, 2, 128, True)]
 
 
 @pytest.mark.parametrize("case", CASES2)
@@ -55,7 +56,7 @@ def test_ssd2(case):
 # two chunks, the double seam's unit weights (optional False)
 CASES3 = [(1, 33, 4, 2, 2, 64, True), (1, 3, 32, 2, 1, 64, True), (2, 100, 2, 2, 1, 128, True),
           (1, 400, 4, 1, 1, 64, True), (1, 129, 1, 3, 3, 64, False), (1, 17, 16, 2, 2, 128, False), (1, 710, 4, 12, 1, 64, True),
-          (2, 8, 4, 2, 1, 128, True), (1, 9, 4, 2, 1, 128, True), (2, 1, 32, 2, 1, 64, True)]
+          (2, 8, 4, 2, 1, 128, True), (1, 9, 4, 2, 1, 128, True), (2, 1, 32, 2, 1, 64, True), (1, 24, 4, 200, 1, 128, True)]
 
 
 @pytest.mark.parametrize("case", CASES3)
