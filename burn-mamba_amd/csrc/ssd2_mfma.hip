@@ -858,10 +858,13 @@ static size_t seg_bytes(const Ssd2Params& p, int S) {
 // chunks; five waves share four SIMDs, which costs a chunk about a fifth.  A
 // chunk takes 1.1 / 2.0 us at dstate 64 (32 / 64 positions) and 1.3 / 2.4 at 128.
 // Splitting adds a launch, 0.24 / 0.31 us of entry state per segment, the state
-// pass (a chunk's time per chunk for every 2048 waves) and the states' bytes: each
-// segment's written and read, and read again by every later one.  These were fitted
-// to 372 calls of 1 to 4 sequences of 65 to 2600 positions, 1 to 80 heads, whole
-// and split (5 to 6 % rms).  Measured at 80 heads x 64 x 128, whole against
+// pass (a chunk's time per chunk for every 2048 waves) and bytes: each segment's state
+// written and read, and read again by every later one, at 10 TB/s (cached), and x and
+// the B fragments once more, for all segments but the last, at 6 TB/s.  Fitted to 372
+// calls of 1 to 4 sequences of 65 to 2600 positions, 1 to 80 heads, whole and split (5
+// to 6 % rms), the last term to 110 of 1 to 8 sequences where the two are close:
+// without it 8 x 1024, 24 heads, dstate 64 was split (44.7 us whole, 47.4), as were
+// many heads with groups of their own (3 x 1847, 64 heads: 108 and 133).  Measured at 80 heads x 64 x 128, whole against
 // split: 1 x 3001 positions 191 / 73 us, 2 x 2048 160 / 87, 1 x 400 25.9 / 31.2 and 2
 // x 200 19.5 / 28.9 (whole); 8 x 4096 fills the chip and stays whole.  Ties go to the
 // larger head set, which stages each fragment for more heads, and to fewer
@@ -893,7 +896,8 @@ static Ssd2Plan choose_plan(const Ssd2Params& p, size_t ws_bytes) {
             double cost = (double)rounds * cps * (hpw == 5 ? 1.2 : 1.) * chunk_us;
             if (S > 1) {
                 const double mb = (double)p.nb * p.H * 64 * p.N * 4e-6 * ((S - 1) * S * 0.5 + 2. * (S - 1));
-                cost += launch_us + entry_us * S + chunk_us * (double)pass * cps + 0.1 * mb;
+                const double again = ((double)p.nb * p.L * p.H * 64 + (double)p.nb * p.nch * p.G * p.N * p.Q) * 2e-6;
+                cost += launch_us + entry_us * S + chunk_us * (double)pass * cps + 0.1 * mb + 0.17 * again * (S - 1) / S;
             }
             if (best_cost == 0. || cost < best_cost) {
                 best_cost = cost;
